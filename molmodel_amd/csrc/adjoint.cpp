@@ -369,7 +369,6 @@ extern "C" int mm_param_gradients(mm_engine *m, int sys, const double *f_ref, in
     }
 
   // forward evaluation: forces, potentials, reciprocal-space fields
-  if (int rc = handle_compute(m)) return rc;
   std::vector<double> f0, phi0;
   if (int rc = evaluate(m, sys, f0, nullptr, &phi0)) return rc;
   std::vector<double> kres(4 * (size_t)N);
@@ -387,10 +386,10 @@ extern "C" int mm_param_gradients(mm_engine *m, int sys, const double *f_ref, in
         Rsoa[(size_t)c * NT + P.site0 + i] = 2 * d;
       }
   if (loss) *loss = L;
-  const int nblk = adj_blocks(e, sys), nslot = adj_part_slots();
+  const int nslot = adj_part_slots();
   TRY_ADJ(ensure(&e.d_adjR, 3 * (size_t)NT));
   TRY_ADJ(ensure(&e.d_chi, (size_t)NT));
-  TRY_ADJ(ensure(&e.d_adjpart, (size_t)std::max(e.ngroup, 1) * nslot));
+  TRY_ADJ(ensure(&e.d_adjpart, (size_t)(e.ngroup + 1) * nslot));
   TRY_ADJ(ensure(&e.d_adjksc, 2 * (size_t)std::max(e.nk_total, 1)));
   TRY_ADJ(ensure(&e.d_adjkres, 4 * (size_t)NT + 16));
   TRY_ADJ(ensure(&e.d_adjacc, (size_t)NACC));
@@ -436,7 +435,7 @@ extern "C" int mm_param_gradients(mm_engine *m, int sys, const double *f_ref, in
   m->pos_dirty = 1;
   if (rc) return rc;
   if (ms) *ms = tms;
-  std::vector<double> chi(N), part((size_t)nblk * nslot), psi(4 * (size_t)N, 0.0);
+  std::vector<double> chi(N), part((size_t)nslot), psi(4 * (size_t)N, 0.0);
   MM_HIP(hipMemcpy(chi.data(), e.d_chi + P.site0, sizeof(double) * N, hipMemcpyDeviceToHost));
   MM_HIP(hipMemcpy(part.data(), e.d_adjpart, sizeof(double) * part.size(), hipMemcpyDeviceToHost));
   if (f_ref && (P.kmode == 0 || (P.kmode == 1 && P.ik)))
@@ -462,11 +461,9 @@ extern "C" int mm_param_gradients(mm_engine *m, int sys, const double *f_ref, in
     const double rdotE = R[3 * i] * E[1] + R[3 * i + 1] * E[2] + R[3 * i + 2] * E[3];
     gL[3 * ty[i]] += chi[i] + (P.kmode <= 1 ? rdotE + psi[4 * (size_t)i] / scale : 0.0);
   }
-  // LJ: per engine type pair, (dL/da, dL/db, dE/da, dE/db) summed over the
-  // blocks in block order, both orientations of an unordered pair together
-  std::vector<double> lj(8 * 8 * 4, 0.0);
-  for (int b = 0; b < nblk; b++)
-    for (int k = 0; k < nslot; k++) lj[k] += part[(size_t)b * nslot + k];
+  // LJ: per engine type pair, (dL/da, dL/db, dE/da, dE/db), both
+  // orientations of an unordered pair together
+  const std::vector<double> &lj = part;
   double ca = 0, cb = 0;
   if (S.include_lj_correction) lj_tail_factors(S, &ca, &cb);
   std::vector<double> nsites(nt, 0.0);

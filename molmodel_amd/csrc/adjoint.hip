@@ -36,160 +36,215 @@
 
 namespace mmamd {
 
-constexpr int ADJ_TB = 128;
 constexpr int ADJ_MAXT = 8;    // LJ types per system (engine limit)
+constexpr int ADJ_W = 64;      // lanes per group: one wavefront
 
-// One thread per sorted group slot of system P; its full neighbour row.
+// One wavefront per sorted group slot of system P, its full neighbour row 64
+// candidates at a time: those inside the cutoff are compacted into an LDS
+// queue, and each lane then evaluates one queued group pair, so erfc and exp
+// (most of the arithmetic) run on full wavefronts.  What bounds it is that
+// arithmetic: about 1 500 instructions per group pair.  One thread per group
+// walking its row alone took 1 045 us for 1 000 groups and 1 048 for 4 096
+// (8 and 32 blocks on 256 CUs, one serial chain); a wavefront per group
+// takes 25 us for 1 000 and 47 us for 4 096.
 // chi: per site (global index), written for the group's sites.
-// part: per block, ADJ_MAXT^2 x 4 (dLa, dLb, dEa, dEb) partial sums, the
-// type pair (t, u) with t the type of this group's site.
-__global__ void __launch_bounds__(ADJ_TB) k_adj_pair(
+// part: [slot][group], the group's share of the nty^2 x 4 sums (dLa, dLb,
+// dEa, dEb) of type pair (t, u), t the type of this group's site; lanes add
+// into private LDS columns, which are then summed in a fixed order.
+__global__ void __launch_bounds__(ADJ_W) k_adj_pair(
     const SysParams *__restrict__ sp, const int4 *__restrict__ gslot,
     const double4 *__restrict__ gpos, const float4 *__restrict__ spk,
     const int2 *__restrict__ gmeta, const int *__restrict__ nbr, const int *__restrict__ nnb,
     int nbcap, const double *__restrict__ R, const double *__restrict__ r, const double *__restrict__ q,
     int N, double *__restrict__ chi, double *__restrict__ part) {
-  __shared__ double lj[ADJ_TB][3][ADJ_MAXT][4];
+  extern __shared__ double lj[];             // [3 sites x nty types x 4][ADJ_W]
+  __shared__ float4 qd[2 * ADJ_W];           // Dx, Dy, Dz, switching value
+  __shared__ float2 qs[2 * ADJ_W];           // switching derivative, neighbour (int bits)
+  __shared__ double sred[3 * ADJ_MAXT * 4];
   const SysParams &P = sp[0];
-  const int nty = P.ntype;
-  const int i = blockIdx.x * ADJ_TB + threadIdx.x;
-  const bool active = i < P.ngroup;
-  for (int k = 0; k < 3; k++)
-    for (int u = 0; u < ADJ_MAXT; u++)
-      for (int c = 0; c < 4; c++) lj[threadIdx.x][k][u][c] = 0.0;
-  if (active) {
-    const int gs = P.group0 + i;
-    const int4 sl = gslot[gs];
-    const int s0 = sl.y, ns = sl.z;
-    const double4 pi = gpos[gs];
-    const int2 mi = gmeta[gs];
-    float4 oi[3];
-    float3 Ri[3];
-    int mki[3], tyi[3];
+  const int nty = P.ntype, nper = 3 * nty * 4;
+  const int lane = threadIdx.x, i = blockIdx.x;
+  for (int e = 0; e < nper; e++) lj[e * ADJ_W + lane] = 0.0;
+  const int gs = P.group0 + i;
+  const int4 sl = gslot[gs];
+  const int s0 = sl.y, ns = sl.z;
+  const double4 pi = gpos[gs];
+  const int2 mi = gmeta[gs];
+  float4 oi[3];
+  float3 Ri[3];
+  int mki[3], tyi[3];
 #pragma unroll
-    for (int k = 0; k < 3; k++) {
-      oi[k] = spk[(long)gs * MAXS + k];
-      const int b = (mi.y >> (8 * k)) & 0xff;
-      mki[k] = k < ns ? (b & 3) : 0;
-      tyi[k] = b >> 2;
-      Ri[k] = k < ns ? make_float3((float)R[s0 + k], (float)R[N + s0 + k], (float)R[2 * N + s0 + k])
-                     : make_float3(0.f, 0.f, 0.f);
+  for (int k = 0; k < 3; k++) {
+    oi[k] = spk[(long)gs * MAXS + k];
+    const int b = (mi.y >> (8 * k)) & 0xff;
+    mki[k] = k < ns ? (b & 3) : 0;
+    tyi[k] = b >> 2;
+    Ri[k] = k < ns ? make_float3((float)R[s0 + k], (float)R[N + s0 + k], (float)R[2 * N + s0 + k])
+                   : make_float3(0.f, 0.f, 0.f);
+  }
+  double ch[3] = {0, 0, 0};
+  const double L = P.L, invL = P.invL;
+  const float eta = (float)P.eta, c2 = (float)(P.eta * 1.1283791670955126);
+
+  // the group pair queued at `at`
+  auto pair = [&](int at) {
+    const float4 ent = qd[at];
+    const float2 e2 = qs[at];
+    const int hs = __float_as_int(e2.y);
+    const float S = ent.w, dsm = e2.x;
+    const float Dx = ent.x, Dy = ent.y, Dz = ent.z;
+    const int4 slj = gslot[hs];
+    const int2 mj = gmeta[hs];
+    const int t0 = slj.y, nsj = slj.z;
+    float3 Rj[3];
+    float4 oj[3];
+#pragma unroll
+    for (int l = 0; l < 3; l++) {
+      oj[l] = spk[(long)hs * MAXS + l];
+      Rj[l] = l < nsj ? make_float3((float)R[t0 + l], (float)R[N + t0 + l], (float)R[2 * N + t0 + l])
+                      : make_float3(0.f, 0.f, 0.f);
     }
-    double ch[3] = {0, 0, 0};
-    const double L = P.L, invL = P.invL;
-    const float eta = (float)P.eta, c2 = (float)(P.eta * 1.1283791670955126);
-    const int cnt = nnb[gs];
-    for (int t = 0; t < cnt; t++) {
-      const int hs = nbr[(long)gs * nbcap + t];
+    // (R_g0 - R_h0) . D dsm
+    const float rdD = ((Ri[0].x - Rj[0].x) * Dx + (Ri[0].y - Rj[0].y) * Dy +
+                       (Ri[0].z - Rj[0].z) * Dz) * dsm;
+#pragma unroll
+    for (int l = 0; l < 3; l++) {
+      if (l >= nsj) break;
+      const int bj = (mj.y >> (8 * l)) & 0xff;
+      const int mkj = bj & 3, tyj = bj >> 2;
+      const float ql = (float)q[t0 + l];
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        const int m = mki[k] & mkj;
+        if (!m) continue;
+        const float rx = Dx - oj[l].x + oi[k].x, ry = Dy - oj[l].y + oi[k].y,
+                    rz = Dz - oj[l].z + oi[k].z;
+        const float rr2 = rx * rx + ry * ry + rz * rz;
+        const float dRr = (Ri[k].x - Rj[l].x) * rx + (Ri[k].y - Rj[l].y) * ry +
+                          (Ri[k].z - Rj[l].z) * rz;
+        if (m & SITE_HAS_Q) {
+          const float rm = sqrtf(rr2), er = eta * rm;
+          const float b0 = erfcf(er) / rm;
+          const float b1 = (b0 + c2 * expf(-er * er)) / rr2;
+          const float w = dRr * b1 * S + rdD * b0;
+          ch[k] += (double)(w * ql);
+        }
+        if (m & SITE_HAS_LJ) {
+          const float ir2 = 1.f / rr2, ir6 = ir2 * ir2 * ir2, ir12 = ir6 * ir6;
+          double *a = lj + (k * nty + tyj) * 4 * ADJ_W + lane;
+          a[0] += 0.5 * (double)(dRr * 12.f * ir12 * ir2 * S + rdD * ir12);
+          a[ADJ_W] -= 0.5 * (double)(dRr * 6.f * ir6 * ir2 * S + rdD * ir6);
+          a[2 * ADJ_W] += 0.5 * (double)(S * ir12);
+          a[3 * ADJ_W] -= 0.5 * (double)(S * ir6);
+        }
+      }
+    }
+  };
+
+  const int cnt = nnb[gs];
+  const int *row = nbr + (long)gs * nbcap;
+  int qn = 0;   // queued pairs, the same in every lane
+  for (int t0 = 0; t0 < cnt; t0 += ADJ_W) {
+    bool take = false;
+    float4 ent = make_float4(0.f, 0.f, 0.f, 1.f);
+    float2 e2 = make_float2(0.f, 0.f);
+    if (t0 + lane < cnt) {
+      const int hs = row[t0 + lane];
       const double4 pj = gpos[hs];
       double dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
       dx -= L * floor(dx * invL + 0.5);
       dy -= L * floor(dy * invL + 0.5);
       dz -= L * floor(dz * invL + 0.5);
       const double r2g = dx * dx + dy * dy + dz * dz;
-      if (r2g > P.rhi2) continue;
+      take = !(r2g > P.rhi2);
       double sm = 1.0, dsm = 0.0;
       if (r2g > P.rlo2) {   // rspace.c:52-58
         const double z = (r2g - P.rlo2) * P.inv_w2;
         sm = ((-6 * z + 15) * z - 10) * z * z * z + 1;
         dsm = ((60 * z - 120) * z + 60) * z * z * P.inv_w2;
       }
-      const float S = (float)sm;
-      const int4 slj = gslot[hs];
-      const int2 mj = gmeta[hs];
-      const int t0 = slj.y, nsj = slj.z;
-      float3 Rj[3];
-      float4 oj[3];
-#pragma unroll
-      for (int l = 0; l < 3; l++) {
-        oj[l] = spk[(long)hs * MAXS + l];
-        Rj[l] = l < nsj ? make_float3((float)R[t0 + l], (float)R[N + t0 + l], (float)R[2 * N + t0 + l])
-                        : make_float3(0.f, 0.f, 0.f);
-      }
-      const float Dx = (float)dx, Dy = (float)dy, Dz = (float)dz;
-      // (R_g0 - R_h0) . D dsm
-      const float rdD = ((Ri[0].x - Rj[0].x) * Dx + (Ri[0].y - Rj[0].y) * Dy +
-                         (Ri[0].z - Rj[0].z) * Dz) * (float)dsm;
-#pragma unroll
-      for (int l = 0; l < 3; l++) {
-        if (l >= nsj) break;
-        const int bj = (mj.y >> (8 * l)) & 0xff;
-        const int mkj = bj & 3, tyj = bj >> 2;
-        const float ql = (float)q[t0 + l];
-#pragma unroll
-        for (int k = 0; k < 3; k++) {
-          const int m = mki[k] & mkj;
-          if (!m) continue;
-          const float rx = Dx - oj[l].x + oi[k].x, ry = Dy - oj[l].y + oi[k].y,
-                      rz = Dz - oj[l].z + oi[k].z;
-          const float rr2 = rx * rx + ry * ry + rz * rz;
-          const float dRr = (Ri[k].x - Rj[l].x) * rx + (Ri[k].y - Rj[l].y) * ry +
-                            (Ri[k].z - Rj[l].z) * rz;
-          if (m & SITE_HAS_Q) {
-            const float rm = sqrtf(rr2), er = eta * rm;
-            const float b0 = erfcf(er) / rm;
-            const float b1 = (b0 + c2 * expf(-er * er)) / rr2;
-            const float w = dRr * b1 * S + rdD * b0;
-            ch[k] += (double)(w * ql);
-          }
-          if (m & SITE_HAS_LJ) {
-            const float ir2 = 1.f / rr2, ir6 = ir2 * ir2 * ir2, ir12 = ir6 * ir6;
-            double *a = lj[threadIdx.x][k][tyj];
-            a[0] += 0.5 * (double)(dRr * 12.f * ir12 * ir2 * S + rdD * ir12);
-            a[1] -= 0.5 * (double)(dRr * 6.f * ir6 * ir2 * S + rdD * ir6);
-            a[2] += 0.5 * (double)(S * ir12);
-            a[3] -= 0.5 * (double)(S * ir6);
-          }
-        }
-      }
+      ent = make_float4((float)dx, (float)dy, (float)dz, (float)sm);
+      e2 = make_float2((float)dsm, __int_as_float(hs));
     }
-    // excluded pairs inside the group (rspace.c:492-521), FP64 as the forward
-    const int ex = sl.w;
-    if (ex) {
-      double x[3][3];
-#pragma unroll
-      for (int k = 0; k < 3; k++) {
-        const int sk = s0 + (k < ns ? k : 0);
-        x[k][0] = r[sk]; x[k][1] = r[N + sk]; x[k][2] = r[2 * N + sk];
-      }
-#pragma unroll
-      for (int k = 0; k < 3; k++)
-#pragma unroll
-        for (int l = k + 1; l < 3; l++) {
-          if (l >= ns || !((ex >> (k * MAXS + l)) & 1)) continue;
-          double d0 = x[k][0] - x[l][0], d1 = x[k][1] - x[l][1], d2 = x[k][2] - x[l][2];
-          d0 -= L * floor(d0 * invL + 0.5);
-          d1 -= L * floor(d1 * invL + 0.5);
-          d2 -= L * floor(d2 * invL + 0.5);
-          const double rr2 = d0 * d0 + d1 * d1 + d2 * d2, rm = sqrt(rr2), er = P.eta * rm;
-          const double b0 = -erf(er) / rm;
-          const double b1 = (b0 + P.eta * 1.1283791670955126 * exp(-er * er)) / rr2;
-          const double w = ((R[s0 + k] - R[s0 + l]) * d0 + (R[N + s0 + k] - R[N + s0 + l]) * d1 +
-                            (R[2 * N + s0 + k] - R[2 * N + s0 + l]) * d2) * b1;
-          ch[k] += w * q[s0 + l];
-          ch[l] += w * q[s0 + k];
-        }
+    const unsigned long long bal = __ballot(take);
+    if (take) {
+      const int at = qn + __popcll(bal & ((1ull << lane) - 1ull));
+      qd[at] = ent;
+      qs[at] = e2;
     }
+    qn += __popcll(bal);
+    __syncthreads();
+    if (qn >= ADJ_W) {
+      qn -= ADJ_W;
+      pair(qn + lane);
+    }
+    __syncthreads();   // the queue's tail is written again next
+  }
+  if (lane < qn) pair(lane);
+
+  // excluded pairs inside the group (rspace.c:492-521), FP64 as the forward:
+  // lane 0 takes sites (0, 1), lane 1 (0, 2), lane 2 (1, 2)
+  if (lane < 3) {
+    const int k = lane == 2 ? 1 : 0, l = lane == 0 ? 1 : 2;
+    if (l < ns && ((sl.w >> (k * MAXS + l)) & 1)) {
+      const int sk = s0 + k, sq = s0 + l;
+      double d0 = r[sk] - r[sq], d1 = r[N + sk] - r[N + sq], d2 = r[2 * N + sk] - r[2 * N + sq];
+      d0 -= L * floor(d0 * invL + 0.5);
+      d1 -= L * floor(d1 * invL + 0.5);
+      d2 -= L * floor(d2 * invL + 0.5);
+      const double rr2 = d0 * d0 + d1 * d1 + d2 * d2, rm = sqrt(rr2), er = P.eta * rm;
+      const double b0 = -erf(er) / rm;
+      const double b1 = (b0 + P.eta * 1.1283791670955126 * exp(-er * er)) / rr2;
+      const double w = ((R[sk] - R[sq]) * d0 + (R[N + sk] - R[N + sq]) * d1 +
+                        (R[2 * N + sk] - R[2 * N + sq]) * d2) * b1;
+      const double wl = w * q[sq], wk = w * q[sk];
+      if (k == 0) ch[0] += wl; else ch[1] += wl;
+      if (l == 1) ch[1] += wk; else ch[2] += wk;
+    }
+  }
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1)
+#pragma unroll
+    for (int k = 0; k < 3; k++) ch[k] += __shfl_xor(ch[k], o);
+  if (lane == 0) {
 #pragma unroll
     for (int k = 0; k < 3; k++)
       if (k < ns) chi[s0 + k] = ch[k];
   }
+  // the lanes' columns, each slot summed by one lane (starting at a lane of
+  // its own, so that the reads spread over the banks)
   __syncthreads();
-  // per block: sum the threads' LJ slots in thread order into (t, u) slots
-  const int nslot = nty * nty * 4;
-  for (int e = threadIdx.x; e < nslot; e += ADJ_TB) {
+  for (int e = lane; e < nper; e += ADJ_W) {
+    double s = 0;
+    for (int j = 0; j < ADJ_W; j++) s += lj[e * ADJ_W + ((j + e) & (ADJ_W - 1))];
+    sred[e] = s;
+  }
+  __syncthreads();
+  for (int e = lane; e < nty * nty * 4; e += ADJ_W) {
     const int t = e / (nty * 4), u = (e / 4) % nty, c = e % 4;
     double s = 0;
-    for (int th = 0; th < ADJ_TB; th++) {
-      const int ii = blockIdx.x * ADJ_TB + th;
-      if (ii >= P.ngroup) break;
-      const int2 mi = gmeta[P.group0 + ii];
-      for (int k = 0; k < 3; k++)
-        if (k < mi.x && ((mi.y >> (8 * k)) & SITE_HAS_LJ) && (((mi.y >> (8 * k)) & 0xff) >> 2) == t)
-          s += lj[th][k][u][c];
-    }
-    part[(long)blockIdx.x * ADJ_MAXT * ADJ_MAXT * 4 + (t * ADJ_MAXT + u) * 4 + c] = s;
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+      if ((mki[k] & SITE_HAS_LJ) && tyi[k] == t) s += sred[(k * nty + u) * 4 + c];
+    part[(long)e * P.ngroup + i] = s;
   }
+}
+
+// the groups' shares of each slot, one block per slot, into
+// out[(t ADJ_MAXT + u) 4 + c]
+__global__ void __launch_bounds__(256) k_adj_sum(const SysParams *__restrict__ sp,
+                                                 const double *__restrict__ part,
+                                                 double *__restrict__ out) {
+  const SysParams &P = sp[0];
+  const int nty = P.ntype, e = blockIdx.x;
+  __shared__ double red[4];
+  double s = 0;
+  for (int i = threadIdx.x; i < P.ngroup; i += 256) s += part[(long)e * P.ngroup + i];
+  for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+  __syncthreads();
+  if (threadIdx.x == 0)
+    out[(e / (nty * 4) * ADJ_MAXT + (e / 4) % nty) * 4 + e % 4] = red[0] + red[1] + red[2] + red[3];
 }
 
 // Ewald adjoint structure factors of system P: (S', C') = (-B_k, A_k) with
@@ -267,16 +322,21 @@ __global__ void k_adj_ik_acc(const SysParams *__restrict__ sp, const double *__r
 }
 
 int adj_part_slots() { return ADJ_MAXT * ADJ_MAXT * 4; }
-int adj_blocks(const Engine &e, int sys) { return (e.hsp[sys].ngroup + ADJ_TB - 1) / ADJ_TB; }
 
+// part: adj_part_slots() sums, then as many per group
 int launch_adj_pair(Engine &e, int sys, const double *R, double *chi, double *part) {
-  if (e.hsp[sys].ntype > ADJ_MAXT) {
+  const SysParams &P = e.hsp[sys];
+  if (P.ntype > ADJ_MAXT) {
     set_last_error("more LJ types than the adjoint kernel holds");
     return -1;
   }
-  hipLaunchKernelGGL(k_adj_pair, dim3(adj_blocks(e, sys)), dim3(ADJ_TB), 0, e.stream,
-                     e.d_sp + sys, e.d_gslot, e.d_gpos, e.d_spk, e.d_gmeta, e.d_nbr, e.d_nnb,
-                     e.nbcap, R, e.d_r, e.d_q, e.nsite, chi, part);
+  double *share = part + adj_part_slots();
+  hipLaunchKernelGGL(k_adj_pair, dim3(P.ngroup), dim3(ADJ_W),
+                     sizeof(double) * 3 * P.ntype * 4 * ADJ_W, e.stream, e.d_sp + sys, e.d_gslot,
+                     e.d_gpos, e.d_spk, e.d_gmeta, e.d_nbr, e.d_nnb, e.nbcap, R, e.d_r, e.d_q,
+                     e.nsite, chi, share);
+  hipLaunchKernelGGL(k_adj_sum, dim3(P.ntype * P.ntype * 4), dim3(256), 0, e.stream, e.d_sp + sys,
+                     share, part);
   MM_HIP(hipGetLastError());
   return 0;
 }

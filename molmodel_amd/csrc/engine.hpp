@@ -263,7 +263,6 @@ int launch_p3m_adjoint(Engine &e, int sys, const float4 *src, hipStream_t st);
 // site index): bin, spread, the ik convolution, gather into kres
 int launch_p3m_ik_pass(Engine &e, int sys, const double *q, hipStream_t st);
 int adj_part_slots();
-int adj_blocks(const Engine &e, int sys);
 int launch_adj_pair(Engine &e, int sys, const double *R, double *chi, double *part);
 int launch_adj_ewald(Engine &e, int sys, const double *R, double *ksc_adj, double *kres_adj,
                      double *acc_scratch);
