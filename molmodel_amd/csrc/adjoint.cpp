@@ -392,7 +392,6 @@ extern "C" int mm_param_gradients(mm_engine *m, int sys, const double *f_ref, in
   TRY_ADJ(ensure(&e.d_adjpart, (size_t)(e.ngroup + 1) * nslot));
   TRY_ADJ(ensure(&e.d_adjksc, 2 * (size_t)std::max(e.nk_total, 1)));
   TRY_ADJ(ensure(&e.d_adjkres, 4 * (size_t)NT + 16));
-  TRY_ADJ(ensure(&e.d_adjacc, (size_t)NACC));
   TRY_ADJ(ensure(&e.d_adjsrc, (size_t)NT));
   TRY_ADJ(ensure(&e.d_adjq, (size_t)NT));
   MM_HIP(hipMemcpy(e.d_adjR, Rsoa.data(), sizeof(double) * Rsoa.size(), hipMemcpyHostToDevice));
@@ -417,7 +416,7 @@ extern "C" int mm_param_gradients(mm_engine *m, int sys, const double *f_ref, in
   MM_HIP(hipEventRecord(t0, e.stream));
   int rc = launch_adj_pair(e, sys, e.d_adjR, e.d_chi, e.d_adjpart);
   if (!rc && f_ref && P.kmode == 0)
-    rc = launch_adj_ewald(e, sys, e.d_adjR, e.d_adjksc, e.d_adjkres, e.d_adjacc);
+    rc = launch_adj_ewald(e, sys, e.d_adjR, e.d_adjksc, e.d_adjkres);
   if (!rc && f_ref && P.kmode == 1 && P.ik)
     rc = launch_adj_p3m_ik(e, sys, e.d_adjR, scale, e.d_adjq, e.d_adjkres);
   if (!rc && f_ref && P.kmode == 1 && !P.ik) {

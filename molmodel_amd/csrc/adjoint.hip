@@ -342,14 +342,13 @@ int launch_adj_pair(Engine &e, int sys, const double *R, double *chi, double *pa
 }
 
 // psi of an Ewald system into kres_adj[4 i] (k_ks_field with the adjoint
-// structure factors; its energy and virial slots go to scratch)
-int launch_adj_ewald(Engine &e, int sys, const double *R, double *ksc_adj, double *kres_adj,
-                     double *acc_scratch) {
+// structure factors)
+int launch_adj_ewald(Engine &e, int sys, const double *R, double *ksc_adj, double *kres_adj) {
   const SysParams &P = e.hsp[sys];
   if (P.kmode != 0) return 0;
   hipLaunchKernelGGL(k_adj_ks_sf, dim3(P.nk), dim3(256), 0, e.stream, e.d_sp + sys,
                      (const double4 *)e.d_kvec, e.d_r, e.d_q, R, e.nsite, ksc_adj);
-  return launch_kspace_field_only(e, sys, ksc_adj, kres_adj, acc_scratch);
+  return launch_kspace_field_only(e, sys, ksc_adj, kres_adj);
 }
 
 // psi of an ik P3M system into psi[4 i]: F_i = q_i E_i with E_a = W^T M_a W q

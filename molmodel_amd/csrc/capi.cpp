@@ -421,7 +421,7 @@ static int enqueue_forces(mm_engine *m, int field_mode, int want_virial,
     MM_HIP(hipStreamWaitEvent(e.stream2, e.ev_fork, 0));
     kst = e.stream2;
   }
-  TRY(launch_kspace(e, want_virial, kst));
+  TRY(launch_kspace(e, want_virial, kst, energy || want_virial));
   TRY(launch_p3m(e, want_virial, kst, energy || want_virial));
   if (e.external_nl) {
     e.first_eval = 0;

@@ -525,6 +525,10 @@ int engine_layout(Engine &e, const std::vector<SystemInput> &in, HostLayout &h) 
             }
       P.nk = nk;
       k0 += nk;
+      P.krow0 = (int)h.krow.size();
+      P.nkmax = nm;
+      MM_REQ(kspace_rows(S.kc, h.krow) == nk, "wave vector rows");
+      P.nkrow = (int)h.krow.size() - P.krow0;
     } else if (S.kmode == 1) {
       MM_REQ(S.ik == 0 || S.ik == 1, "ik must be 0 (real-space differentiation) or 1 (-i k on the mesh)");
       MM_REQ(S.order >= 1 && S.order <= 7, "assignment order must be 1..7");
@@ -630,7 +634,7 @@ int engine_check_layout(const Engine &e, const HostLayout &h) {
     }
     return 0;
   };
-  std::vector<Slice> site, group, cell, st, tb, lj, kv, mesh, cmesh, gr, tw, bin, halo;
+  std::vector<Slice> site, group, cell, st, tb, lj, kv, kr, mesh, cmesh, gr, tw, bin, halo;
   for (int s = 0; s < e.nsys; s++) {
     const SysParams &P = e.hsp[s];
     site.push_back({P.site0, P.nsite, s});
@@ -640,6 +644,7 @@ int engine_check_layout(const Engine &e, const HostLayout &h) {
     tb.push_back({P.tab0, P.ntabA + P.ntabB, s});
     lj.push_back({P.lj0, (long)P.ntype * P.ntype, s});
     if (P.kmode == 0) kv.push_back({4L * P.k0, 4L * P.nk, s});
+    if (P.kmode == 0) kr.push_back({P.krow0, P.nkrow, s});
     if (P.kmode == 1) {
       const long nzh = P.nz / 2 + 1, ncomp = P.ik ? 4 : 1;
       mesh.push_back({P.mesh0, ncomp * P.nx * P.ny * P.nz, s});
@@ -664,6 +669,7 @@ int engine_check_layout(const Engine &e, const HostLayout &h) {
   MM_TRY(check("erfc table", tb, (long)h.tab.size()));
   MM_TRY(check("LJ table", lj, (long)h.ljt.size()));
   MM_TRY(check("wave vectors", kv, (long)h.kvec.size()));
+  MM_TRY(check("wave vector rows", kr, (long)h.krow.size()));
   MM_TRY(check("mesh", mesh, e.mesh_total));
   MM_TRY(check("half spectrum", cmesh, e.cmesh_total));
   MM_TRY(check("influence function", gr, (long)h.green.size()));
@@ -753,6 +759,7 @@ int engine_create(Engine &e, const std::vector<SystemInput> &in) {
   MM_TRY(dalloc(&e.d_kres, 4 * (size_t)N + 9 * e.nsys));
   MM_TRY(dalloc(&e.d_kvec, kvec.size())); MM_TRY(dput(e.d_kvec, kvec));
   MM_TRY(dalloc(&e.d_ksc, 2 * (size_t)e.nk_total));
+  MM_TRY(dalloc(&e.d_krow, h.krow.size())); MM_TRY(dput(e.d_krow, h.krow));
   MM_TRY(dalloc(&e.d_mesh, e.mesh_total));
   MM_TRY(dalloc(&e.d_cmesh, e.cmesh_total));
   MM_TRY(dalloc(&e.d_green, green.size())); MM_TRY(dput(e.d_green, green));
@@ -975,7 +982,7 @@ void engine_destroy(Engine &e) {
                   e.d_bgrid, e.d_bfrac, e.d_acc, e.d_part, e.d_fpart, e.d_done, e.d_phi, e.d_scratch,
                   e.d_nlb, e.d_ladder, e.d_kT, e.d_tail, e.d_rtmp, e.d_mom, e.d_perm,
                   e.d_remd_stats, e.d_tile_start, e.d_snap, e.d_snap_perm, e.d_snap_stats,
-                  e.d_adjR, e.d_chi, e.d_adjpart, e.d_adjksc, e.d_adjkres, e.d_adjacc,
+                  e.d_adjR, e.d_chi, e.d_adjpart, e.d_adjksc, e.d_adjkres, e.d_krow,
                   e.d_adjsrc, e.d_adjq};
   for (void *p : ptrs)
     if (p) hipFree(p);

@@ -105,6 +105,7 @@ struct Engine {
   // Ewald
   double *d_kvec = nullptr;   // 4 per k: kx ky kz a_k
   double *d_ksc = nullptr;    // 2 per k: S, C
+  int4 *d_krow = nullptr;     // rows of wave vectors: first, nx, ny, largest |nz|
   int nk_total = 0;
   // P3M
   long mesh_total = 0, cmesh_total = 0, green_total = 0;
@@ -170,7 +171,7 @@ struct Engine {
   std::vector<std::vector<double>> pert;
   // adjoint buffers (allocated by the first gradient call)
   double *d_adjR = nullptr, *d_chi = nullptr, *d_adjpart = nullptr, *d_adjksc = nullptr;
-  double *d_adjkres = nullptr, *d_adjacc = nullptr;
+  double *d_adjkres = nullptr;
   float4 *d_adjsrc = nullptr;
   double *d_adjq = nullptr;
   // state saved at the start of an MD block or exchange interval, restored
@@ -197,6 +198,7 @@ struct HostLayout {
   std::vector<float2> ljt;
   std::vector<int4> sten;
   std::vector<double> kvec;
+  std::vector<int4> krow;
   std::vector<float> green;
   std::vector<float2> twid;
 };
@@ -237,8 +239,9 @@ int pair_tiles(int ngroup);
 // partial-sum slot per workgroup
 constexpr int P3M_FFT_LINES = 16;
 
-int launch_kspace(Engine &e, int want_virial, hipStream_t st);
-// energies 0: the mesh energy (a diagnostic total) is not formed
+// energies 0: the reciprocal-space energy (a diagnostic total) is not formed
+int launch_kspace(Engine &e, int want_virial, hipStream_t st, int energies = 1);
+int kspace_rows(double kc, std::vector<int4> &rows);
 int launch_p3m(Engine &e, int want_virial, hipStream_t st, int energies = 1);
 inline int launch_kspace(Engine &e, int want_virial) { return launch_kspace(e, want_virial, e.stream); }
 inline int launch_p3m(Engine &e, int want_virial) { return launch_p3m(e, want_virial, e.stream); }
@@ -252,20 +255,18 @@ int launch_nonperiodic_points(const double4 *site, const double *rscreen, int n,
                               const double *pts, int npts, double *phi, hipStream_t st);
 // k-space structure factors and field of one system in buffers the caller
 // provides (kspace.hip)
-int launch_kspace_raw(const SysParams *sp, const double4 *kvec, int nk, int nsite,
-                      const double *r, const double *q, double *ksc, double *kres, double *acc,
-                      hipStream_t st);
+int launch_kspace_raw(const SysParams *sp, const double4 *kvec, const int4 *krow, int nkrow,
+                      int nm, int nsite, const double *r, const double *q, double *ksc,
+                      double *kres, hipStream_t st);
 // adjoint passes of one system (adjoint.hip, kspace.hip, pppm.hip)
-int launch_kspace_field_only(Engine &e, int sys, const double *ksc, double *kres_out,
-                             double *acc_out);
+int launch_kspace_field_only(Engine &e, int sys, const double *ksc, double *kres_out);
 int launch_p3m_adjoint(Engine &e, int sys, const float4 *src, hipStream_t st);
 // one forward ik P3M pass of system sys with per-site charges q (global
 // site index): bin, spread, the ik convolution, gather into kres
 int launch_p3m_ik_pass(Engine &e, int sys, const double *q, hipStream_t st);
 int adj_part_slots();
 int launch_adj_pair(Engine &e, int sys, const double *R, double *chi, double *part);
-int launch_adj_ewald(Engine &e, int sys, const double *R, double *ksc_adj, double *kres_adj,
-                     double *acc_scratch);
+int launch_adj_ewald(Engine &e, int sys, const double *R, double *ksc_adj, double *kres_adj);
 int launch_adj_p3m_src(Engine &e, int sys, const double *R, double scale, float4 *src);
 int launch_adj_p3m_ik(Engine &e, int sys, const double *R, double scale, double *qsrc,
                       double *psi);

@@ -4,64 +4,140 @@
 // (4 pi / V) exp(-k^2 / 4 eta^2) / k^2 (kspace.c:96-103), structure factors
 // S_k = sum q sin(k.r), C_k = sum q cos(k.r) (kspace.c:147-155), then
 // phi_i += sum 2 a_k (S s_i + C c_i) and E_i += sum 2 a_k (C s_i - S c_i) k
-// (kspace.c:156-173).  Trigonometric values come from FP64 sincos of k.r
-// directly rather than the reference's angle-addition recurrences; both
-// are FP64-accurate.  One block per k-vector forms S_k, C_k; one thread per
-// site then sums over k.  The k-sum energy and virial
+// (kspace.c:156-173).  Wave vectors come in rows: all nz of one (nx, ny), and
+// k.r = (nx b1 + ny b2).r + nz b3.r, so a row's sines and cosines follow from
+// those of its (nx, ny) part and of nz b3.r by the addition theorems.
+// Everything is FP64.  What bounds both kernels is latency at the sizes plain
+// Ewald is used for (hundreds to a few thousand sites): a sincos is about 100
+// FP64 instructions, so each kernel keeps the number of them per thread small
+// and spreads rows and sites over the chip.
+//   k_ks_sf     one block per row (and per eight |nz| of it), one thread per
+//               site: two sincos per site and row, then a rotation per |nz|;
+//               648 sites, 709 wave vectors: 6.4 us (5.3 with a sincos per site
+//               and wave vector), 3 120 sites: 10.2 (12.2)
+//   k_ks_field  a block serves 16 sites and its 64 16-lane teams take a row
+//               each; the sites' e^{i n b.r} for every n are formed once, in
+//               LDS; 7.9 us for 648 and for 3 120 sites (38 with 16 waves
+//               that walk the wave vectors with a sincos each, 64 sites a block)
+// The k-sum energy and virial
 // (W_ab = sum a_k |rho_k|^2 (delta_ab - 2 k_a k_b (1/k^2 + 1/(4 eta^2))))
-// are formed by the first block of the field kernel.
+// are formed by a block of its own beside the field kernel's.
 #include "engine.hpp"
 
 namespace mmamd {
 
-__global__ void __launch_bounds__(256) k_ks_sf(const SysParams *__restrict__ sp,
-                                               const double4 *__restrict__ kvec,
+// A row of the half space: (first wave vector, nx, ny, m): nz = -m .. m, or
+// 1 .. m for nx = ny = 0.
+struct KRow {
+  int k0, nx, ny, m;
+  bool half;
+  __device__ __forceinline__ explicit KRow(int4 v)
+      : k0(v.x), nx(v.y), ny(v.z), m(v.w), half(v.y == 0 && v.z == 0) {}
+  __device__ __forceinline__ int at(int nz) const { return k0 + nz + (half ? -1 : m); }
+};
+
+constexpr int KS_NZ = 8;       // |nz| values a structure-factor block serves
+constexpr int SF_TB = 512;
+
+__global__ void __launch_bounds__(SF_TB) k_ks_sf(const SysParams *__restrict__ sp,
+                                               const int4 *__restrict__ krow,
                                                const double *__restrict__ r, const double *__restrict__ q,
                                                int N, double *__restrict__ ksc) {
   const int s = blockIdx.y;
   const SysParams &P = sp[s];
-  const int k = blockIdx.x;
-  if (P.kmode != 0 || k >= P.nk) return;
-  const double4 kv = kvec[P.k0 + k];
-  double ss = 0, cc = 0;
-  for (int i = threadIdx.x; i < P.nsite; i += blockDim.x) {
+  if (P.kmode != 0 || (int)blockIdx.x >= P.nkrow) return;
+  const KRow row(krow[P.krow0 + blockIdx.x]);
+  const int z0 = blockIdx.z * KS_NZ;
+  if (z0 > row.m) return;
+  const double *B = P.RL;
+  const double b0 = row.nx * B[0] + row.ny * B[3], b1 = row.nx * B[1] + row.ny * B[4],
+               b2 = row.nx * B[2] + row.ny * B[5];
+  // per |nz|: sums of q times cos cos, sin sin, sin cos, cos sin of the
+  // (nx, ny) and nz parts
+  double a[4 * KS_NZ];
+#pragma unroll
+  for (int c = 0; c < 4 * KS_NZ; c++) a[c] = 0;
+  for (int i = threadIdx.x; i < P.nsite; i += SF_TB) {
     const int si = P.site0 + i;
-    const double kr = kv.x * r[si] + kv.y * r[N + si] + kv.z * r[2 * N + si];
-    double sn, cs;
-    sincos(kr, &sn, &cs);
-    ss += q[si] * sn;
-    cc += q[si] * cs;
+    const double x = r[si], y = r[N + si], z = r[2 * N + si], qi = q[si];
+    double xs, xc, s1, c1, sz = 0, cz = 1;
+    sincos(b0 * x + b1 * y + b2 * z, &xs, &xc);
+    const double tz = B[6] * x + B[7] * y + B[8] * z;
+    sincos(tz, &s1, &c1);
+    if (z0) sincos(z0 * tz, &sz, &cz);
+    xs *= qi;
+    xc *= qi;
+#pragma unroll
+    for (int j = 0; j < KS_NZ; j++) {
+      if (z0 + j > row.m) break;
+      a[4 * j] += xc * cz;
+      a[4 * j + 1] += xs * sz;
+      a[4 * j + 2] += xs * cz;
+      a[4 * j + 3] += xc * sz;
+      const double t = cz * c1 - sz * s1;
+      sz = sz * c1 + cz * s1;
+      cz = t;
+    }
   }
-  __shared__ double rs[4], rc[4];
-  for (int o = 32; o >= 1; o >>= 1) { ss += __shfl_xor(ss, o); cc += __shfl_xor(cc, o); }
-  const int wid = threadIdx.x >> 6;
-  if ((threadIdx.x & 63) == 0) { rs[wid] = ss; rc[wid] = cc; }
+  // the wave's 32 sums over 64 lanes: at each step a lane hands half of its
+  // values to its partner and keeps the other half (31 exchanges instead of
+  // the 192 of a reduction value by value, which took longer than the sums)
+  __shared__ double red[SF_TB / 64][4 * KS_NZ];
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+#pragma unroll
+  for (int h = 2 * KS_NZ; h >= 1; h >>= 1) {
+    const bool up = lane & (2 * h);
+#pragma unroll
+    for (int c = 0; c < h; c++) {
+      const double mine = up ? a[c + h] : a[c], other = up ? a[c] : a[c + h];
+      a[c] = mine + __shfl_xor(other, 2 * h);
+    }
+  }
+  a[0] += __shfl_xor(a[0], 1);
+  if (!(lane & 1)) red[w][lane >> 1] = a[0];
   __syncthreads();
-  if (threadIdx.x == 0) {
-    double a = 0, b = 0;
-    for (int w = 0; w < (int)(blockDim.x >> 6); w++) { a += rs[w]; b += rc[w]; }
-    ksc[2 * (P.k0 + k)] = a;
-    ksc[2 * (P.k0 + k) + 1] = b;
+  const int j = threadIdx.x, nz = z0 + j;
+  if (j >= KS_NZ || nz > row.m) return;
+  double t[4];
+  for (int c = 0; c < 4; c++) {
+    t[c] = 0;
+    for (int k = 0; k < SF_TB / 64; k++) t[c] += red[k][4 * j + c];
+  }
+  if (!(row.half && nz == 0)) {
+    double *o = ksc + 2L * (P.k0 + row.at(nz));
+    o[0] = t[2] + t[3];
+    o[1] = t[0] - t[1];
+  }
+  if (!row.half && nz > 0) {
+    double *o = ksc + 2L * (P.k0 + row.at(-nz));
+    o[0] = t[2] - t[3];
+    o[1] = t[0] + t[1];
   }
 }
 
-// Field kernel: a block serves KS_SITES sites; its KS_SPLIT waves split the
-// k-vectors (wave w takes k = w, w + KS_SPLIT, ...), and the per-wave sums
-// are added in wave order (deterministic).
-constexpr int KS_SITES = 64, KS_SPLIT = 16, KS_TB = KS_SITES * KS_SPLIT;
+constexpr int KS_SITES = 16, KS_SPLIT = 64, KS_TB = KS_SITES * KS_SPLIT;
+constexpr int KS_MAXTAB = 31;   // largest |n| whose table fits beside the partial sums
 
+// Each team of 16 lanes (one per site) takes rows team, team + KS_SPLIT, ...;
+// the teams' sums are added in team order (deterministic).  TABLE false: wave
+// vectors beyond KS_MAXTAB, whose factors are formed where they are used.
+template <bool TABLE>
 __global__ void __launch_bounds__(KS_TB) k_ks_field(const SysParams *__restrict__ sp,
                                                     const double4 *__restrict__ kvec,
+                                                    const int4 *__restrict__ krow,
                                                     const double *__restrict__ ksc,
                                                     const double *__restrict__ r, int N,
                                                     double *__restrict__ kres,
                                                     double *__restrict__ acc, int want_virial) {
-  __shared__ double part[KS_SPLIT][4][KS_SITES];
+  extern __shared__ double2 tab[];   // [axis][n][site]: (cos, sin)
+  __shared__ double part[KS_SPLIT][4 * KS_SITES];
   const int s = blockIdx.y;
   const SysParams &P = sp[s];
   if (P.kmode != 0) return;
-  if ((int)(blockIdx.x * KS_SITES) >= P.nsite) return;
-  if (blockIdx.x == 0) {
+  const int nblk = (P.nsite + KS_SITES - 1) / KS_SITES;
+  if ((int)blockIdx.x > nblk) return;
+  if ((int)blockIdx.x == nblk) {
+    if (!acc) return;
     // k-sum energy and virial of this system
     double e = 0, w[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     const double c4 = 0.25 / (P.eta * P.eta);
@@ -78,90 +154,180 @@ __global__ void __launch_bounds__(KS_TB) k_ks_field(const SysParams *__restrict_
           for (int b = 0; b < 3; b++) w[3 * a + b] += ek * ((a == b ? 1.0 : 0.0) - f * kk[a] * kk[b]);
       }
     }
-    __shared__ double red[KS_TB / 64][10];
     for (int o = 32; o >= 1; o >>= 1) {
       e += __shfl_xor(e, o);
-      for (int c = 0; c < 9; c++) w[c] += __shfl_xor(w[c], o);
+      if (want_virial)
+        for (int c = 0; c < 9; c++) w[c] += __shfl_xor(w[c], o);
     }
     const int wid = threadIdx.x >> 6;
     if ((threadIdx.x & 63) == 0) {
-      red[wid][0] = e;
-      for (int c = 0; c < 9; c++) red[wid][1 + c] = w[c];
+      part[wid][0] = e;
+      for (int c = 0; c < 9; c++) part[wid][1 + c] = w[c];
     }
     __syncthreads();
     if (threadIdx.x == 0) {
       double t[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
       for (int ww = 0; ww < KS_TB / 64; ww++)
-        for (int c = 0; c < 10; c++) t[c] += red[ww][c];
+        for (int c = 0; c < 10; c++) t[c] += part[ww][c];
       acc[s * NACC + ACC_KSPACE_E] = t[0];
       // reciprocal virial kept beside the per-site results; finish adds it
       for (int c = 0; c < 9; c++) kres[(long)4 * N + 9 * s + c] = want_virial ? t[1 + c] : 0.0;
     }
+    return;
   }
-  const int lane = threadIdx.x & (KS_SITES - 1), split = threadIdx.x / KS_SITES;
-  const int i = blockIdx.x * KS_SITES + lane;
-  const bool on = i < P.nsite;
-  const int si = P.site0 + (on ? i : 0);
-  const double x = r[si], y = r[N + si], z = r[2 * N + si];
-  double p = 0, gx = 0, gy = 0, gz = 0;
-  for (int k = split; k < P.nk; k += KS_SPLIT) {
-    const double4 kv = kvec[P.k0 + k];
-    const double S = ksc[2 * (P.k0 + k)], C = ksc[2 * (P.k0 + k) + 1];
-    double sn, cs;
-    sincos(kv.x * x + kv.y * y + kv.z * z, &sn, &cs);
-    const double two_a = 2 * kv.w;
-    const double t = two_a * (C * sn - S * cs);
-    gx += t * kv.x; gy += t * kv.y; gz += t * kv.z;
-    p += two_a * (S * sn + C * cs);
+  const int site = threadIdx.x & (KS_SITES - 1), team = threadIdx.x / KS_SITES;
+  const int i = blockIdx.x * KS_SITES + site;
+  const int si = P.site0 + (i < P.nsite ? i : 0);
+  const double *B = P.RL;
+  double th[3];
+  {
+    const double x = r[si], y = r[N + si], z = r[2 * N + si];
+#pragma unroll
+    for (int a = 0; a < 3; a++) th[a] = B[3 * a] * x + B[3 * a + 1] * y + B[3 * a + 2] * z;
   }
-  part[split][0][lane] = p;
-  part[split][1][lane] = gx;
-  part[split][2][lane] = gy;
-  part[split][3][lane] = gz;
+  const int nm = P.nkmax;
+  if (TABLE) {
+    for (int t = team; t < 3 * (nm + 1); t += KS_SPLIT) {
+      const int a = t / (nm + 1), n = t - a * (nm + 1);
+      double sn, cs;
+      sincos(n * (a == 0 ? th[0] : a == 1 ? th[1] : th[2]), &sn, &cs);
+      tab[t * KS_SITES + site] = make_double2(cs, sn);
+    }
+    __syncthreads();
+  }
+  auto factor = [&](int a, int n) {
+    if (TABLE) return tab[(a * (nm + 1) + n) * KS_SITES + site];
+    double2 f;
+    sincos(n * th[a], &f.y, &f.x);
+    return f;
+  };
+  double p = 0, g1 = 0, g2 = 0, g3 = 0;   // phi; field components along b1, b2, b3
+  for (int rw = team; rw < P.nkrow; rw += KS_SPLIT) {
+    const KRow row(krow[P.krow0 + rw]);
+    const double2 ex = factor(0, row.nx);
+    double2 ey = factor(1, row.ny < 0 ? -row.ny : row.ny);
+    if (row.ny < 0) ey.y = -ey.y;
+    const double xc = ex.x * ey.x - ex.y * ey.y, xs = ex.x * ey.y + ex.y * ey.x;
+    double t0 = 0;
+    const int first = row.half ? 1 : 0;
+    for (int nz = first; nz <= row.m; nz++) {
+      const double2 ez = factor(2, nz);
+      const double cc = xc * ez.x, ss = xs * ez.y, sc = xs * ez.x, cs = xc * ez.y;
+      const int kp = P.k0 + row.at(nz);
+      const double ap = 2 * kvec[kp].w, Sp = ksc[2 * kp], Cp = ksc[2 * kp + 1];
+      const double snp = sc + cs, csp = cc - ss;
+      double t = ap * (Cp * snp - Sp * csp);
+      p += ap * (Sp * snp + Cp * csp);
+      t0 += t;
+      g3 += nz * t;
+      if (!row.half && nz > 0) {
+        const int km = P.k0 + row.at(-nz);
+        const double am = 2 * kvec[km].w, Sm = ksc[2 * km], Cm = ksc[2 * km + 1];
+        const double snm = sc - cs, csm = cc + ss;
+        t = am * (Cm * snm - Sm * csm);
+        p += am * (Sm * snm + Cm * csm);
+        t0 += t;
+        g3 -= nz * t;
+      }
+    }
+    g1 += row.nx * t0;
+    g2 += row.ny * t0;
+  }
+  double *o = &part[team][site];
+  o[0] = p;
+  o[KS_SITES] = g1 * B[0] + g2 * B[3] + g3 * B[6];
+  o[2 * KS_SITES] = g1 * B[1] + g2 * B[4] + g3 * B[7];
+  o[3 * KS_SITES] = g1 * B[2] + g2 * B[5] + g3 * B[8];
   __syncthreads();
-  if (split < 4 && on) {   // four waves finish one component each
-    double t = 0;
-    for (int w = 0; w < KS_SPLIT; w++) t += part[w][split][lane];
-    kres[4 * si + split] = t;
+  // sixteen waves add four teams each, then one wave the sixteen sums
+  const int at = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const double t = part[4 * w][at] + part[4 * w + 1][at] + part[4 * w + 2][at] + part[4 * w + 3][at];
+  __syncthreads();
+  part[w][at] = t;
+  __syncthreads();
+  if (w == 0) {
+    double u = 0;
+#pragma unroll
+    for (int k = 0; k < KS_TB / 64; k++) u += part[k][at];
+    const int c = at / KS_SITES, j = blockIdx.x * KS_SITES + (at & (KS_SITES - 1));
+    if (j < P.nsite) kres[4L * (P.site0 + j) + c] = u;
   }
 }
 
-int launch_kspace(Engine &e, int want_virial, hipStream_t st) {
-  int maxk = 0, maxn = 0;
+// the rows of |n| <= kc (kspace.c:35-58), in the lexicographic order of the
+// wave vectors; returns the number of wave vectors
+int kspace_rows(double kc, std::vector<int4> &rows) {
+  const double nsqmax = kc * kc + 1e-8;
+  const int nm = (int)floor(kc);
+  int nk = 0;
+  for (int nx = 0; nx <= nm; nx++)
+    for (int ny = (nx == 0) ? 0 : -nm; ny <= nm; ny++) {
+      int m = -1;
+      while (m < nm && nx * nx + ny * ny + (m + 1) * (m + 1) <= nsqmax) m++;
+      const bool half = nx == 0 && ny == 0;
+      if (m < (half ? 1 : 0)) continue;
+      rows.push_back(make_int4(nk, nx, ny, m));
+      nk += half ? m : 2 * m + 1;
+    }
+  return nk;
+}
+
+static void launch_sf(dim3 rows_sys, int nm, hipStream_t st, const SysParams *sp,
+                      const int4 *krow, const double *r, const double *q, int N, double *ksc) {
+  rows_sys.z = nm / KS_NZ + 1;
+  hipLaunchKernelGGL(k_ks_sf, rows_sys, dim3(SF_TB), 0, st, sp, krow, r, q, N, ksc);
+}
+
+// acc null: energy and virial are not formed
+static void launch_field(int nsite, int nsys, int nm, hipStream_t st, const SysParams *sp,
+                         const double4 *kvec, const int4 *krow, const double *ksc,
+                         const double *r, int N, double *kres, double *acc, int want_virial) {
+  const dim3 grid((nsite + KS_SITES - 1) / KS_SITES + (acc ? 1 : 0), nsys);
+  if (nm <= KS_MAXTAB)
+    hipLaunchKernelGGL(k_ks_field<true>, grid, dim3(KS_TB),
+                       sizeof(double2) * 3 * (nm + 1) * KS_SITES, st, sp, kvec, krow, ksc, r, N,
+                       kres, acc, want_virial);
+  else
+    hipLaunchKernelGGL(k_ks_field<false>, grid, dim3(KS_TB), 0, st, sp, kvec, krow, ksc, r, N,
+                       kres, acc, want_virial);
+}
+
+int launch_kspace(Engine &e, int want_virial, hipStream_t st, int energies) {
+  int maxrow = 0, maxn = 0, nm = 0;
   for (auto &p : e.hsp)
-    if (p.kmode == 0) { maxk = std::max(maxk, p.nk); maxn = std::max(maxn, p.nsite); }
-  if (maxk == 0) return 0;
-  hipLaunchKernelGGL(k_ks_sf, dim3(maxk, e.nsys), dim3(256), 0, st, e.d_sp,
-                     (const double4 *)e.d_kvec, e.d_r, e.d_q, e.nsite, e.d_ksc);
-  hipLaunchKernelGGL(k_ks_field, dim3((maxn + KS_SITES - 1) / KS_SITES, e.nsys), dim3(KS_TB), 0, st,
-                     e.d_sp, (const double4 *)e.d_kvec, e.d_ksc, e.d_r, e.nsite, e.d_kres,
-                     e.d_acc, want_virial);
+    if (p.kmode == 0) {
+      maxrow = std::max(maxrow, p.nkrow);
+      maxn = std::max(maxn, p.nsite);
+      nm = std::max(nm, p.nkmax);
+    }
+  if (maxrow == 0) return 0;
+  launch_sf(dim3(maxrow, e.nsys), nm, st, e.d_sp, e.d_krow, e.d_r, e.d_q, e.nsite, e.d_ksc);
+  launch_field(maxn, e.nsys, nm, st, e.d_sp, (const double4 *)e.d_kvec, e.d_krow, e.d_ksc, e.d_r,
+               e.nsite, e.d_kres, energies ? e.d_acc : nullptr, want_virial);
   MM_HIP(hipGetLastError());
   return 0;
 }
 
 // Structure factors and field of one system whose parameters, wave vectors,
-// SoA positions and result buffers the caller provides (kspace_field_noalloc
-// keeps them in its own device array): ksc 2 nk, kres 4 nsite + 9, acc NACC.
-int launch_kspace_raw(const SysParams *sp, const double4 *kvec, int nk, int nsite,
-                      const double *r, const double *q, double *ksc, double *kres, double *acc,
-                      hipStream_t st) {
-  hipLaunchKernelGGL(k_ks_sf, dim3(nk, 1), dim3(256), 0, st, sp, kvec, r, q, nsite, ksc);
-  hipLaunchKernelGGL(k_ks_field, dim3((nsite + KS_SITES - 1) / KS_SITES, 1), dim3(KS_TB), 0, st,
-                     sp, kvec, ksc, r, nsite, kres, acc, 0);
+// rows (nkrow of them, |n| up to nm), SoA positions and result buffers the
+// caller provides (kspace_field_noalloc keeps them in its own device array):
+// ksc 2 nk, kres 4 nsite.
+int launch_kspace_raw(const SysParams *sp, const double4 *kvec, const int4 *krow, int nkrow,
+                      int nm, int nsite, const double *r, const double *q, double *ksc,
+                      double *kres, hipStream_t st) {
+  launch_sf(dim3(nkrow, 1), nm, st, sp, krow, r, q, nsite, ksc);
+  launch_field(nsite, 1, nm, st, sp, kvec, krow, ksc, r, nsite, kres, nullptr, 0);
   MM_HIP(hipGetLastError());
   return 0;
 }
 
 // the field kernel of one system with other structure factors and outputs
-// (the adjoint pass): kres_out needs 4 N + 9 entries, acc_out NACC
-int launch_kspace_field_only(Engine &e, int sys, const double *ksc, double *kres_out,
-                             double *acc_out) {
+// (the adjoint pass): kres_out needs 4 N entries
+int launch_kspace_field_only(Engine &e, int sys, const double *ksc, double *kres_out) {
   const SysParams &P = e.hsp[sys];
   if (P.kmode != 0) return 0;
-  hipLaunchKernelGGL(k_ks_field, dim3((P.nsite + KS_SITES - 1) / KS_SITES, 1), dim3(KS_TB), 0,
-                     e.stream, e.d_sp + sys, (const double4 *)e.d_kvec, ksc, e.d_r, e.nsite,
-                     kres_out, acc_out, 0);
+  launch_field(P.nsite, 1, P.nkmax, e.stream, e.d_sp + sys, (const double4 *)e.d_kvec, e.d_krow,
+               ksc, e.d_r, e.nsite, kres_out, nullptr, 0);
   MM_HIP(hipGetLastError());
   return 0;
 }

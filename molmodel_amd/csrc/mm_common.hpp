@@ -53,6 +53,8 @@ struct SysParams {
   int ntype, lj0;              // LJ type-pair table offset (float2 entries)
   int kmode;                   // 0 Ewald, 1 P3M
   int nk, k0;                  // Ewald k-vectors
+  int nkrow, krow0;            // their rows (kspace_rows)
+  int nkmax;                   // largest |n| of a component
   // P3M
   int nx, ny, nz, order;
   long mesh0, cmesh0;          // real mesh / complex half-spectrum offsets

@@ -27,12 +27,12 @@ constexpr int NA_MAX_K = 4096;           // wave vectors (|n| <= kc, half space)
 constexpr long NA_SP = 0;                                 // SysParams (<= 1 KB)
 constexpr long NA_KVEC = NA_SP + 128;                     // double4 per wave vector
 constexpr long NA_KSC = NA_KVEC + 4L * NA_MAX_K;          // S_k, C_k
-constexpr long NA_ACC = NA_KSC + 2L * NA_MAX_K;           // NACC energy slots
-constexpr long NA_R = NA_ACC + 32;                        // x[N] y[N] z[N]
-constexpr long NA_KRES = NA_R + 3L * NA_MAX_SITES;        // phi, E per site (+ 9 virial)
+constexpr int NA_MAX_ROW = 512;                           // rows of wave vectors (326 at kc = 12)
+constexpr long NA_ROW = NA_KSC + 2L * NA_MAX_K;           // int4 per row
+constexpr long NA_R = NA_ROW + 2L * NA_MAX_ROW;             // x[N] y[N] z[N]
+constexpr long NA_KRES = NA_R + 3L * NA_MAX_SITES;        // phi, E per site
 constexpr long NA_TOTAL = NA_KRES + 4L * NA_MAX_SITES + 32;   // 3.9 MB
 static_assert(sizeof(SysParams) <= 128 * sizeof(double), "SysParams slot too small");
-static_assert(NACC <= 32, "energy slot too small");
 
 static __device__ __align__(256) double scratch[NA_TOTAL];
 
@@ -42,10 +42,12 @@ struct Lat9 { double v[9]; };
 // System parameters, then the half-space wave vectors with |n|^2 <= kc^2
 // (kspace.c:41-57) in lexicographic (nx, ny, nz) order, compacted in one
 // block chunk by chunk (so the order is fixed), with
-// a_k = (4 pi / V) exp(-k^2 / 4 eta^2) / k^2 (kspace.c:96-103).
+// a_k = (4 pi / V) exp(-k^2 / 4 eta^2) / k^2 (kspace.c:96-103), and their
+// rows (nx, ny), as kspace_rows lists them: one thread per (nx, ny).
 __global__ void __launch_bounds__(1024) k_na_setup(SysParams P, Lat9 L, double kc, double *sc) {
   __shared__ int wsum[16];
   __shared__ int base;
+  __shared__ int rn[NA_MAX_ROW], rk[NA_MAX_ROW], ri[NA_MAX_ROW];
   if (threadIdx.x == 0) {
     *reinterpret_cast<SysParams *>(sc + NA_SP) = P;
     base = 0;
@@ -57,7 +59,25 @@ __global__ void __launch_bounds__(1024) k_na_setup(SysParams P, Lat9 L, double k
   const double c = 0.25 / (P.eta * P.eta), fourpi_V = 4 * M_PI / P.volume;
   double4 *kv = reinterpret_cast<double4 *>(sc + NA_KVEC);
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int npair = min((nm + 1) * w, NA_MAX_ROW), t = threadIdx.x;
+  const int px = t / w, py = t % w - nm;
+  int m = -1;
+  if (t < npair) {
+    if (px > 0 || py >= 0)
+      while (m < nm && (double)(px * px + py * py + (m + 1) * (m + 1)) <= nsqmax) m++;
+    rn[t] = m < 0 ? 0 : (px == 0 && py == 0) ? m : 2 * m + 1;
+  }
   __syncthreads();
+  if (threadIdx.x == 0)
+    for (int p = 0, k = 0, i = 0; p < npair; p++) {
+      rk[p] = k;
+      ri[p] = i;
+      k += rn[p];
+      i += rn[p] > 0;
+    }
+  __syncthreads();
+  if (t < npair && rn[t] > 0 && ri[t] < P.nkrow)
+    reinterpret_cast<int4 *>(sc + NA_ROW)[ri[t]] = make_int4(rk[t], px, py, m);
   for (long c0 = 0; c0 < ncand; c0 += 1024) {
     const long cand = c0 + threadIdx.x;
     int nx = 0, ny = 0, nz = 0;
@@ -137,16 +157,6 @@ int na_scratch(double **out) {
   return 0;
 }
 
-int na_count_k(double kc) {   // kspace.c:41-57
-  const double nsqmax = kc * kc + 1e-8;
-  const int nm = (int)floor(kc);
-  int nk = 0;
-  for (int nx = 0; nx <= nm; nx++)
-    for (int ny = (nx == 0) ? 0 : -nm; ny <= nm; ny++)
-      for (int nz = (nx == 0 && ny == 0) ? 1 : -nm; nz <= nm; nz++)
-        if (nx * nx + ny * ny + nz * nz <= nsqmax) nk++;
-  return nk;
-}
 }  // namespace
 
 }  // namespace mmamd
@@ -163,7 +173,8 @@ extern "C" int kspace_field_noalloc(double cutoff, int nsite, const cart_t *r, c
     set_last_error("kspace_field_noalloc: bad cutoff, eta, volume or lattice");
     return -1;
   }
-  const int nk = na_count_k(cutoff);
+  std::vector<int4> rows;
+  const int nk = kspace_rows(cutoff, rows);
   if (nk > NA_MAX_K) {
     set_last_error("kspace_field_noalloc: more than " + std::to_string(NA_MAX_K) +
                    " wave vectors (cutoff above 12)");
@@ -182,6 +193,9 @@ extern "C" int kspace_field_noalloc(double cutoff, int nsite, const cart_t *r, c
   P.kmode = 0;
   P.nk = nk;
   P.k0 = 0;
+  P.nkrow = (int)rows.size();
+  P.nkmax = (int)floor(cutoff);
+  memcpy(P.RL, latv, sizeof P.RL);
   P.nsite = nsite;
   P.site0 = 0;
   P.eta = eta;
@@ -193,8 +207,9 @@ extern "C" int kspace_field_noalloc(double cutoff, int nsite, const cart_t *r, c
                      nsite, sc);
   const SysParams *dsp = reinterpret_cast<const SysParams *>(sc + NA_SP);
   const double4 *kv = reinterpret_cast<const double4 *>(sc + NA_KVEC);
-  if (int rc = launch_kspace_raw(dsp, kv, nk, nsite, sc + NA_R, q, sc + NA_KSC, sc + NA_KRES,
-                                 sc + NA_ACC, st))
+  const int4 *krow = reinterpret_cast<const int4 *>(sc + NA_ROW);
+  if (int rc = launch_kspace_raw(dsp, kv, krow, P.nkrow, P.nkmax, nsite, sc + NA_R, q,
+                                 sc + NA_KSC, sc + NA_KRES, st))
     return rc;
   hipLaunchKernelGGL(k_na_out, dim3((nsite + 255) / 256), dim3(256), 0, st, sc, nsite, phi,
                      (double *)evec);

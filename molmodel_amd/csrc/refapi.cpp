@@ -537,6 +537,7 @@ struct kspace {
   double kc;
   int nsite, nk, nmax;
   std::vector<int> ik;   // 3 per vector, reference order (kspace.c:35-58)
+  std::vector<int4> row; // the device's order: rows of one (nx, ny), lexicographic
   Engine e;
   int ready = 0;
 };
@@ -556,7 +557,7 @@ extern "C" struct kspace *kspace_new(double cutoff, int nsite) {
         if (nx * nx + ny * ny + nz * nz <= nsqmax) {
           k->ik.push_back(nx); k->ik.push_back(ny); k->ik.push_back(nz);
         }
-  k->nk = (int)k->ik.size() / 3;
+  k->nk = kspace_rows(cutoff, k->row);
   // sorted by |n|^2, largest first (kspace.c:23-33, 58)
   std::vector<int> idx(k->nk);
   for (int i = 0; i < k->nk; i++) idx[i] = i;
@@ -598,6 +599,8 @@ static void kspace_run(struct kspace *k, const cart_t *r, const double *q, const
     HIPCHK(hipMalloc((void **)&e.d_q, sizeof(double) * N));
     HIPCHK(hipMalloc((void **)&e.d_kvec, sizeof(double) * 4 * k->nk));
     HIPCHK(hipMalloc((void **)&e.d_ksc, sizeof(double) * 2 * k->nk));
+    HIPCHK(hipMalloc((void **)&e.d_krow, sizeof(int4) * k->row.size()));
+    HIPCHK(hipMemcpy(e.d_krow, k->row.data(), sizeof(int4) * k->row.size(), hipMemcpyHostToDevice));
     HIPCHK(hipMalloc((void **)&e.d_kres, sizeof(double) * (4 * (size_t)N + 9)));
     HIPCHK(hipMalloc((void **)&e.d_acc, sizeof(double) * NACC));
     k->ready = 1;
@@ -609,18 +612,23 @@ static void kspace_run(struct kspace *k, const cart_t *r, const double *q, const
   P.nsite = N;
   P.eta = eta;
   P.volume = volume;
+  P.nkrow = (int)k->row.size();
+  P.nkmax = k->nmax;
+  const double rl[9] = {L->xx, L->yx, L->zx, L->xy, L->yy, L->zy, L->xz, L->yz, L->zz};
+  memcpy(P.RL, rl, sizeof rl);
   // kspace.c:96-103 with the caller's reciprocal lattice
   std::vector<double> kv(4 * (size_t)k->nk);
   const double c = 0.25 / (eta * eta), fourpi_V = 4 * M_PI / volume;
-  for (int i = 0; i < k->nk; i++) {
-    const int nx = k->ik[3 * i], ny = k->ik[3 * i + 1], nz = k->ik[3 * i + 2];
-    const double kx = L->xx * nx + L->xy * ny + L->xz * nz;
-    const double ky = L->yx * nx + L->yy * ny + L->yz * nz;
-    const double kz = L->zx * nx + L->zy * ny + L->zz * nz;
-    const double t = kx * kx + ky * ky + kz * kz;
-    kv[4 * i] = kx; kv[4 * i + 1] = ky; kv[4 * i + 2] = kz;
-    kv[4 * i + 3] = fourpi_V * exp(-t * c) / t;
-  }
+  double *kp = kv.data();
+  for (const int4 &w : k->row)
+    for (int nx = w.y, ny = w.z, nz = (nx == 0 && ny == 0) ? 1 : -w.w; nz <= w.w; nz++, kp += 4) {
+      const double kx = L->xx * nx + L->xy * ny + L->xz * nz;
+      const double ky = L->yx * nx + L->yy * ny + L->yz * nz;
+      const double kz = L->zx * nx + L->zy * ny + L->zz * nz;
+      const double t = kx * kx + ky * ky + kz * kz;
+      kp[0] = kx; kp[1] = ky; kp[2] = kz;
+      kp[3] = fourpi_V * exp(-t * c) / t;
+    }
   std::vector<double> soa;
   to_soa((const double *)r, N, soa);
   HIPCHK(hipMemcpy(e.d_sp, &P, sizeof(SysParams), hipMemcpyHostToDevice));
