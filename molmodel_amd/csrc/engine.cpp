@@ -543,10 +543,7 @@ int engine_layout(Engine &e, const std::vector<SystemInput> &in, HostLayout &h) 
       P.T[1] *= S.ny; P.T[4] *= S.ny; P.T[7] *= S.ny;
       P.T[2] *= S.nz; P.T[5] *= S.nz; P.T[8] *= S.nz;
       const int nzh = S.nz / 2 + 1;
-      const int ncomp = S.ik ? 4 : 1;   // phi [, Ex, Ey, Ez]
-      mesh0 = (mesh0 + 3) & ~3L;   // 16-byte aligned: an ik system's points are float4
-      P.mesh0 = mesh0; mesh0 += ncomp * (long)S.nx * S.ny * S.nz;
-      P.cmesh0 = cmesh0; cmesh0 += ncomp * (long)S.nx * S.ny * nzh;
+      MM_REQ(p3m_mesh_layout(P, mesh0, cmesh0) == 0, "mesh dimensions have no transform plan");
       P.green0 = green0;
       green0 += (long)S.nx * S.ny * nzh;
       const double inv_4eta2 = 1 / sq(2 * S.eta), inv_v = 1.0 / P.volume;
@@ -556,19 +553,14 @@ int engine_layout(Engine &e, const std::vector<SystemInput> &in, HostLayout &h) 
         for (int iy = 0; iy < S.ny; iy++) {
           const int jy = iy > S.ny / 2 ? iy - S.ny : iy;
           for (int iz = 0; iz < nzh; iz++)
-            gh[((size_t)iy * nzh + iz) * S.nx + ix] =
+            gh[p3m_green_at(P, ix, iy, iz)] =
                 (float)green_at(jx, jy, iz, S.nx, S.ny, S.nz, P.RL, inv_4eta2, inv_v, S.nalias, S.order,
                                 S.ik, nullptr);
         }
       }
       green.insert(green.end(), gh.begin(), gh.end());
-      const int nn[3] = {S.nx, S.ny, S.nz};
       P.twid0 = (int)twid.size();
-      for (int d = 0; d < 3; d++)
-        for (int t = 0; t < 128; t++) {
-          const double a = -2 * M_PI * (t % nn[d]) / nn[d];
-          twid.push_back(make_float2((float)cos(a), (float)sin(a)));
-        }
+      p3m_twiddles(P, twid);
       MM_REQ(choose_spread_blocks(S.nx, S.ny, S.nz, 4096, 4096, P.bx, P.by, e.spread_block,
                                   e.spread_halo ? S.order : 0),
              "mesh dimensions give no valid spreading column blocks");
@@ -604,7 +596,7 @@ int engine_layout(Engine &e, const std::vector<SystemInput> &in, HostLayout &h) 
   int nb = (e.maxg + 63) / 64;
   for (auto &P : e.hsp)
     if (P.kmode == 1)
-      nb = std::max(nb, (P.ny * (P.nz / 2 + 1) + P3M_FFT_LINES - 1) / P3M_FFT_LINES);
+      nb = std::max(nb, p3m_energy_blocks(P));
   e.nblk_part = nb;
   for (auto &P : e.hsp) {
     P.water = P.ngroup > 0;
@@ -646,11 +638,12 @@ int engine_check_layout(const Engine &e, const HostLayout &h) {
     if (P.kmode == 0) kv.push_back({4L * P.k0, 4L * P.nk, s});
     if (P.kmode == 0) kr.push_back({P.krow0, P.nkrow, s});
     if (P.kmode == 1) {
-      const long nzh = P.nz / 2 + 1, ncomp = P.ik ? 4 : 1;
-      mesh.push_back({P.mesh0, ncomp * P.nx * P.ny * P.nz, s});
-      cmesh.push_back({P.cmesh0, ncomp * P.nx * P.ny * nzh, s});
+      const long nzh = P.nz / 2 + 1, xy = (long)P.nx * P.ny;
+      mesh.push_back({P.mesh0, xy * P.nz, s});
+      mesh.push_back({P.omesh0, P.ik ? 4 * xy * P.nz : xy * P.mzs, s});
+      cmesh.push_back({P.cmesh0, (P.ik ? 5 : 1) * xy * nzh, s});
       gr.push_back({P.green0, (long)P.nx * P.ny * nzh, s});
-      tw.push_back({P.twid0, 3L * 128, s});
+      tw.push_back({P.twid0, P3M_TWIDDLES, s});
       bin.push_back({P.bin0, (long)P.nbx * P.nby, s});
       const long hpts = (long)(P.bx + P.order - 1) * (P.by + P.order - 1) * P.nz;
       if (e.spread_halo) halo.push_back({P.halo0, (long)P.nbx * P.nby * hpts, s});

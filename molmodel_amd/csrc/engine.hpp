@@ -112,7 +112,7 @@ struct Engine {
   float *d_mesh = nullptr;
   float2 *d_cmesh = nullptr;
   float *d_green = nullptr;
-  float2 *d_twid = nullptr;   // per P3M system (at SysParams::twid0): twiddles for nx, ny, nz (3*128)
+  float2 *d_twid = nullptr;   // per P3M system (at SysParams::twid0): tables of p3m_twiddles
   int4 *d_sgrid = nullptr;    // per site: jx jy jz bin
   float4 *d_sfrac = nullptr;  // per site: sx sy sz q
   int nbin_total = 0;
@@ -235,9 +235,12 @@ int launch_nl_build(Engine &e, int force, int from_partials = 0);
 int launch_pack(Engine &e);
 int launch_pair(Engine &e, int field_mode, int want_virial, int energy = 1);
 int pair_tiles(int ngroup);
-// mesh lines per FFT workgroup (16 threads per line); the x pass writes one
-// partial-sum slot per workgroup
-constexpr int P3M_FFT_LINES = 16;
+// P3M mesh buffers of one system (pppm.hip)
+int p3m_mesh_layout(SysParams &P, long &mesh, long &cmesh);
+long p3m_green_at(const SysParams &P, int ix, int iy, int kz);
+int p3m_energy_blocks(const SysParams &P);
+constexpr int P3M_TWIDDLES = 6 * 128;
+void p3m_twiddles(const SysParams &P, std::vector<float2> &tw);
 
 // energies 0: the reciprocal-space energy (a diagnostic total) is not formed
 int launch_kspace(Engine &e, int want_virial, hipStream_t st, int energies = 1);

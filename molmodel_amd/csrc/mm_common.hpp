@@ -57,20 +57,22 @@ struct SysParams {
   int nkmax;                   // largest |n| of a component
   // P3M
   int nx, ny, nz, order;
-  long mesh0, cmesh0;          // real mesh / complex half-spectrum offsets
-  long green0;                 // influence function offset (layout [ky][kz][kx])
+  long mesh0, omesh0, cmesh0;  // charge mesh, gathered mesh, half-spectrum offsets
+  int mzs;                     // z stride of the gathered mesh (nz + order - 1)
+  int rad[3][3];               // radices of the transforms along x, y, z (0: none)
+  int plane;                   // a kz plane is transformed in one block
+  long green0;                 // influence function offset (p3m_green_at)
   double T[9];                 // diag(n) L^-1, tensor_t layout (pppm.c:523-525)
   double RL[9];                // reciprocal lattice 2 pi (L^-1)^T, tensor_t layout
   int bx, by, nbx, nby, bin0;  // spread column blocks (bx x by mesh columns each)
   long halo0;                  // the blocks' fixed-point halo partials: block k at
                                // halo0 + k (bx+order-1)(by+order-1) nz
-  int twid0;                   // first of this system's 3 x 128 FFT twiddles
+  int twid0;                   // first of this system's FFT tables (p3m_twiddles)
   int water;                   // every group is a three-site water (mask bytes WATER_MASKS)
-  int ik;                      // P3M field by -i k on the mesh: four half spectra at
-                               // cmesh0 + c nx ny (nz/2+1), c = 0..3 (phi, Ex, Ey, Ez), and
-                               // 4 nx ny nz floats of real mesh from mesh0 (the density in
-                               // the first nx ny nz, the transformed field interleaved as
-                               // (phi, Ex, Ey, Ez) per point); mesh0 is a multiple of 4
+  int ik;                      // P3M field by -i k on the mesh: the half spectra of phi, Ex, Ey
+                               // and Ez follow the density's at cmesh0, each nx ny (nz/2+1),
+                               // and the gathered mesh holds (phi, Ex, Ey, Ez) per point
+                               // (nx ny nz float4; omesh0 is a multiple of 4)
   // dynamics
   double dt;
   double bg_phi;               // neutralising background potential (or 0)
@@ -113,6 +115,10 @@ inline bool choose_spread_blocks(int nx, int ny, int nz, int maxpts, int maxbins
   if (!fits()) by = 1;
   return fits() && (nx / bx) * (ny / by) <= maxbins;
 }
+
+// points of the largest kz plane that is transformed in one block (46 KB of
+// LDS with an odd line stride)
+constexpr int FFT_PLANE_MAX = 5632;
 
 // slots per P3M column bin: four times the mean occupancy plus a margin,
 // rounded to 32 (an overfull bin raises ERR_BIN_OVERFLOW)

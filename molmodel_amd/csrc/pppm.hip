@@ -18,10 +18,10 @@
 //            pulling re-reads every site for each block its stencil
 //            reaches, the halos cost their traffic, so columns holding many
 //            sites favour pulling and few sites the halos;
-//   fft      Stockham mixed-radix (4,2,3,5,7) line FFTs in LDS: z (real to
-//            half spectrum), y, then x forward, multiply by the influence
-//            function (and form the mesh energy/virial), x inverse, y
-//            inverse, z (half spectrum to real), unnormalised like FFTW;
+//   fft      in-place mixed-radix line FFTs in LDS (fft.hpp): z (real to half
+//            spectrum), then per kz plane y and x forward, the influence
+//            function (and the mesh energy/virial), x and y inverse, then z
+//            (half spectrum to real), unnormalised like FFTW;
 //   gather   phi_i = sum w phi_m and, with real-space differentiation (the
 //            reference default), E_i = (diag(n) L^-1)^T (sum -dw phi_m)
 //            (pppm.c:603-640); with the field formed on the mesh (ik), the
@@ -32,6 +32,9 @@
 #include "engine.hpp"
 #include "scan.hpp"
 #include "reduce.hpp"
+#include "fft.hpp"
+#include <cmath>
+#include <cstring>
 
 namespace mmamd {
 
@@ -321,95 +324,29 @@ __global__ void __launch_bounds__(256) k_p3m_spread_halo(const SysParams *__rest
   for (int t = threadIdx.x; t < npts; t += blockDim.x) dst[t] = hacc[t];
 }
 
-// ---------------- line FFTs in LDS ----------------
-constexpr int FFT_T = 16;                 // threads per line
-constexpr int FFT_LINES = P3M_FFT_LINES;  // lines per block
-constexpr int FFT_TB = FFT_T * FFT_LINES; // one wave
+// ---------------- transforms ----------------
+// Half spectra are stored plane by plane, [kz][x][y], the influence function
+// likewise but with x and y in the digit-reversed order the forward
+// transforms leave (fft.hpp), so that its factors line up with the spectrum.
 constexpr int FFT_MAXN = 128;
+constexpr int FZ_LINES = 16;                 // complex lines per z block: 32 mesh lines
+constexpr int FZ_TB = 256;
+constexpr int FP_TB = 512;                   // plane block
 
-__device__ __forceinline__ float2 cmul(float2 a, float2 b) {
-  return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
-}
-__device__ __forceinline__ float2 cadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
-__device__ __forceinline__ float2 csub(float2 a, float2 b) { return make_float2(a.x - b.x, a.y - b.y); }
-
-// twiddle exp(sign*2*pi*i*t/n) from tw[t] = exp(-2 pi i t/n)
-__device__ __forceinline__ float2 twid(const float2 *tw, int t, int n, int sign) {
-  const float2 w = tw[t % n];
-  return sign < 0 ? w : make_float2(w.x, -w.y);
-}
-
-// one Stockham stage of radix R over a line of length n (stride p)
-template <int R>
-__device__ __forceinline__ void fft_stage(const float2 *xl, float2 *yl, int n, int p,
-                                          const float2 *tw, int sign, int tid) {
-  const int nb = n / R;
-  const int tstep = n / (p * R);
-  for (int i = tid; i < nb; i += FFT_T) {
-    const int k = i % p;
-    float2 u[R], v[R];
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-      u[r] = xl[i + r * nb];
-      if (r > 0 && k > 0) u[r] = cmul(u[r], twid(tw, r * k * tstep, n, sign));
-    }
-    if (R == 2) {
-      v[0] = cadd(u[0], u[1]); v[1] = csub(u[0], u[1]);
-    } else if (R == 4) {
-      const float2 a = cadd(u[0], u[2]), b = csub(u[0], u[2]);
-      const float2 c = cadd(u[1], u[3]), d = csub(u[1], u[3]);
-      const float2 di = sign < 0 ? make_float2(d.y, -d.x) : make_float2(-d.y, d.x);
-      v[0] = cadd(a, c); v[2] = csub(a, c);
-      v[1] = cadd(b, di); v[3] = csub(b, di);
-    } else {
-      const int ws = n / R;
-#pragma unroll
-      for (int r = 0; r < R; r++) {
-        float2 acc = u[0];
-#pragma unroll
-        for (int t = 1; t < R; t++) acc = cadd(acc, cmul(u[t], twid(tw, ((r * t) % R) * ws, n, sign)));
-        v[r] = acc;
-      }
-    }
-    const int j = (i - k) * R + k;
-#pragma unroll
-    for (int r = 0; r < R; r++) yl[j + r * p] = v[r];
-  }
-}
-
-// Stockham autosort FFT of FFT_LINES lines of length n held in x (line l at
-// x + l*FFT_MAXN); every thread of the block must call it.  Radices are
-// taken greedily (4, 2, 3, 5, 7).  Returns the buffer holding the result.
-// Always inlined: as a called function (the compiler's choice for the
-// mixed-radix build) it took a call and 192-416 bytes of scratch per lane in
-// every kernel that uses it, and the x pass with virial and the field on
-// the mesh gave wrong results in that form; inlined, the mixed-radix
-// kernels fit in registers (at most 32 bytes of spill).
-template <bool POW2>
-__device__ __forceinline__ float2 *lds_fft_lines(float2 *x, float2 *y, int n, const float2 *tw,
-                                                 int sign) {
-  const int l = threadIdx.x / FFT_T, tid = threadIdx.x % FFT_T;
-  int p = 1, rem = n;
-  while (rem > 1) {
-    float2 *xl = x + l * FFT_MAXN, *yl = y + l * FFT_MAXN;
-    int R;
-    if (rem % 4 == 0) { R = 4; fft_stage<4>(xl, yl, n, p, tw, sign, tid); }
-    else if (rem % 2 == 0) { R = 2; fft_stage<2>(xl, yl, n, p, tw, sign, tid); }
-    else if (POW2) { R = rem; }   // not reached: the host launches POW2 only for 2^k lines
-    else if (rem % 3 == 0) { R = 3; fft_stage<3>(xl, yl, n, p, tw, sign, tid); }
-    else if (rem % 5 == 0) { R = 5; fft_stage<5>(xl, yl, n, p, tw, sign, tid); }
-    else { R = 7; fft_stage<7>(xl, yl, n, p, tw, sign, tid); }
-    __syncthreads();
-    float2 *t = x; x = y; y = t;
-    p *= R;
-    rem /= R;
-  }
-  return x;
-}
-
+// an axis' factors exp(-2 pi i t / n), and (pos) each frequency's place and
+// each place's signed frequency, from the system's tables (p3m_twiddles)
 __device__ __forceinline__ void load_tw(float2 *stw, const float2 *tw, int n) {
   for (int t = threadIdx.x; t < n; t += blockDim.x) stw[t] = tw[t];
 }
+__device__ __forceinline__ void load_pos(int *pos, const float2 *tw, int n) {
+  for (int t = threadIdx.x; t < n; t += blockDim.x) pos[t] = __float_as_int(tw[3 * FFT_MAXN + t].x);
+}
+__device__ __forceinline__ void load_freq(short *f, const float2 *tw, int n) {
+  for (int t = threadIdx.x; t < n; t += blockDim.x)
+    f[t] = (short)__float_as_int(tw[3 * FFT_MAXN + t].y);
+}
+
+constexpr int HALO_T = 16;   // threads per halo line
 
 // The z line `line` (mesh column xi = line / ny, yi = line % ny) of a P3M
 // system as the sum of the spreading blocks' halo columns that cover it:
@@ -417,17 +354,18 @@ __device__ __forceinline__ void load_tw(float2 *stw, const float2 *tw, int n) {
 // (bi bx + istart + dx, bj by + istart + dy) mod n, so the covering blocks
 // have dx = xi - istart (mod bx), dy likewise; up to 4 x 4 of them are
 // read at once (all loads in flight), more in further rounds.  Integer
-// sums, then the conversion a single accumulator would make.
+// sums, then the conversion a single accumulator would make, into every
+// other float of xl (one component of a packed line).
 __device__ __forceinline__ void halo_line(const SysParams &P,
                                           const unsigned long long *__restrict__ halo, int line,
-                                          int tid, float2 *xl) {
+                                          int tid, float *xl) {
   const int nx = P.nx, ny = P.ny, nz = P.nz;
   const int xi = line / ny, yi = line % ny;
   const int istart = -((P.order + 1) / 2 - 1);
   const int bxs = P.bx, bys = P.by, HX = bxs + P.order - 1, HY = bys + P.order - 1;
   const int hpts = HX * HY * nz;
   const unsigned long long *h = halo + P.halo0;
-  constexpr int NK = FFT_MAXN / FFT_T;
+  constexpr int NK = FFT_MAXN / HALO_T;
   unsigned long long acc[NK];
 #pragma unroll
   for (int k = 0; k < NK; k++) acc[k] = 0ull;
@@ -449,7 +387,7 @@ __device__ __forceinline__ void halo_line(const SysParams &P,
       }
 #pragma unroll
       for (int k = 0; k < NK; k++) {
-        const int t = tid + k * FFT_T;
+        const int t = tid + k * HALO_T;
         if (t < nz) {
           unsigned long long v = 0ull;
 #pragma unroll
@@ -461,212 +399,352 @@ __device__ __forceinline__ void halo_line(const SysParams &P,
     }
 #pragma unroll
   for (int k = 0; k < NK; k++) {
-    const int t = tid + k * FFT_T;
-    if (t < nz) xl[t] = make_float2((float)((double)(long long)acc[k] * FIX_INV), 0.f);
+    const int t = tid + k * HALO_T;
+    if (t < nz) xl[2 * t] = (float)((double)(long long)acc[k] * FIX_INV);
   }
 }
 
-// pass 0: z lines, real -> half spectrum; HALO: the line is the sum of the
-// spreading blocks' halo columns that cover it (halo_line), else the real
-// mesh.  pass 1/3: y lines fwd/inv.  pass 4: z lines, half
-// spectrum -> real.  blockIdx.z: the mesh component (phi, then Ex, Ey, Ez
-// of a system whose field is formed as -i k phi on the mesh; the forward
-// passes run over component 0 only).
-template <bool POW2, bool HALO = false>
-__global__ void __launch_bounds__(FFT_TB, 4) k_fft_pass(const SysParams *__restrict__ sp,
-                                                     const float2 *__restrict__ twid_all,
-                                                     float *__restrict__ mesh,
-                                                     float2 *__restrict__ cmesh, int pass,
-                                                     const unsigned long long *__restrict__ halo) {
-  __shared__ float2 bx_[FFT_LINES * FFT_MAXN], by_[FFT_LINES * FFT_MAXN];
-  __shared__ float2 stw[FFT_MAXN];
-  const int s = blockIdx.y;
-  const SysParams &P = sp[s];
+// z lines, real to half spectrum.  Two neighbouring mesh lines are one complex
+// line (a in the real, b in the imaginary part) whose transform Z separates
+// as a_k = (Z_k + conj Z_-k) / 2, b_k = (Z_k - conj Z_-k) / 2i, so a block of
+// two waves takes 32 lines with one butterfly per thread and stage.
+// HALO: a line is the sum of the spreading blocks' halo columns that cover it
+// (halo_line) instead of the real mesh.  What bounds it is the launch and one
+// trip to memory: 5.7 us at 48^3, 6.7 at 64^3, and the inverse 5.9 and 7
+// (5.65 and 6 with one line per transform, 16 lines a block).
+template <bool HALO>
+__global__ void __launch_bounds__(FZ_TB) k_fft_z(
+    const SysParams *__restrict__ sp, const float2 *__restrict__ twid_all,
+    const float *__restrict__ mesh, float2 *__restrict__ cmesh,
+    const unsigned long long *__restrict__ halo) {
+  __shared__ float2 buf[FZ_LINES * (FFT_MAXN + 1)], stw[FFT_MAXN];
+  __shared__ int pos[FFT_MAXN];
+  const SysParams &P = sp[blockIdx.y];
+  if (P.kmode != 1) return;
+  const int nz = P.nz, nzh = nz / 2 + 1, ls = nz | 1;
+  const int nlines = P.nx * P.ny, l0 = blockIdx.x * 2 * FZ_LINES, nl = min(2 * FZ_LINES, nlines - l0);
+  if (nl <= 0) return;
+  load_tw(stw, twid_all + P.twid0 + 2 * FFT_MAXN, nz);
+  load_pos(pos, twid_all + P.twid0 + 2 * FFT_MAXN, nz);
+  float *fb = reinterpret_cast<float *>(buf);
+  if constexpr (HALO) {
+    for (int l = threadIdx.x / HALO_T; l < 2 * FZ_LINES; l += FZ_TB / HALO_T) {
+      float *xl = fb + 2 * (l >> 1) * ls + (l & 1);
+      if (l < nl) halo_line(P, halo, l0 + l, threadIdx.x % HALO_T, xl);
+      else
+        for (int z = threadIdx.x % HALO_T; z < nz; z += HALO_T) xl[2 * z] = 0.f;
+    }
+  } else {
+    const float *src = mesh + P.mesh0 + (long)l0 * nz;
+    const float inv = 1.f / (float)nz;
+    batched<8>(2 * FZ_LINES * nz, [&](int t) { return t < nl * nz ? src[t] : 0.f; },
+               [&](int t, float v) {
+                 const int l = div_small(t, inv), z = t - l * nz;
+                 fb[2 * ((l >> 1) * ls + z) + (l & 1)] = v;
+               });
+  }
+  __syncthreads();
+  fft_forward(buf, FZ_LINES, ls, 1, nz, P.rad[2], stw);
+  float2 *dst = cmesh + P.cmesh0 + l0;
+  for (int t = threadIdx.x; t < nzh * FZ_LINES; t += blockDim.x) {
+    const int k = t / FZ_LINES, l = t % FZ_LINES;
+    const float2 zp = buf[l * ls + pos[k]], zm = buf[l * ls + pos[k ? nz - k : 0]];
+    float2 *o = dst + (long)k * nlines + 2 * l;
+    if (2 * l < nl) o[0] = make_float2(0.5f * (zp.x + zm.x), 0.5f * (zp.y - zm.y));
+    if (2 * l + 1 < nl) o[1] = make_float2(0.5f * (zp.y + zm.y), 0.5f * (zm.x - zp.x));
+  }
+}
+
+// z lines, half spectrum to real, two lines in one complex line as above.
+// The potential's lines are followed by their first order - 1 points again,
+// so that a site's run along z is contiguous for the gather; with the field
+// on the mesh (blockIdx.z: phi, Ex, Ey, Ez) the components are interleaved
+// per point instead.
+__global__ void __launch_bounds__(FZ_TB) k_fft_zinv(const SysParams *__restrict__ sp,
+                                                    const float2 *__restrict__ twid_all,
+                                                    const float2 *__restrict__ cmesh,
+                                                    float *__restrict__ mesh) {
+  __shared__ float2 buf[FZ_LINES * (FFT_MAXN + 1)], stw[FFT_MAXN];
+  __shared__ int pos[FFT_MAXN];
+  const SysParams &P = sp[blockIdx.y];
   if (P.kmode != 1) return;
   const int comp = blockIdx.z;
   if (comp > 0 && !P.ik) return;
-  const int nx = P.nx, ny = P.ny, nz = P.nz, nzh = nz / 2 + 1;
-  const long mesh0 = P.mesh0 + comp * (long)nx * ny * nz;
-  const long cmesh0 = P.cmesh0 + comp * (long)nx * ny * nzh;
-  int nlines, n, twoff;
-  if (pass == 0 || pass == 4) { nlines = nx * ny; n = nz; twoff = 2 * FFT_MAXN; }
-  else { nlines = nx * nzh; n = ny; twoff = FFT_MAXN; }
-  if ((int)(blockIdx.x * FFT_LINES) >= nlines) return;
-  load_tw(stw, twid_all + P.twid0 + twoff, n);
-  const int l = threadIdx.x / FFT_T, tid = threadIdx.x % FFT_T;
-  const int line = blockIdx.x * FFT_LINES + l;
-  const bool on = line < nlines;
-  float2 *xl = bx_ + l * FFT_MAXN;
-  const int sign = (pass == 3 || pass == 4) ? 1 : -1;
-  // load
-  if (pass == 0) {
-    if constexpr (HALO) {
-      if (on) halo_line(P, halo, line, tid, xl);
-    } else if (on) {
-      const float *src = mesh + mesh0 + (long)line * nz;
-      for (int t = tid; t < n; t += FFT_T) xl[t] = make_float2(src[t], 0.f);
-    }
-  } else if (pass == 4) {
-    if (on) {
-      const float2 *src = cmesh + cmesh0 + (long)line * nzh;
-      for (int t = tid; t < nzh; t += FFT_T) xl[t] = src[t];
-    }
-    __syncthreads();
-    if (on)
-      for (int t = nzh + tid; t < n; t += FFT_T) {
-        const float2 c = xl[n - t];
-        xl[t] = make_float2(c.x, -c.y);
-      }
-  } else {
-    if (on) {
-      const int xi = line / nzh, kz = line % nzh;
-      const float2 *src = cmesh + cmesh0 + (long)xi * ny * nzh + kz;
-      for (int t = tid; t < n; t += FFT_T) xl[t] = src[(long)t * nzh];
-    }
-  }
+  const int nz = P.nz, nzh = nz / 2 + 1, ls = nz | 1;
+  const int nlines = P.nx * P.ny, l0 = blockIdx.x * 2 * FZ_LINES, nl = min(2 * FZ_LINES, nlines - l0);
+  if (nl <= 0) return;
+  load_tw(stw, twid_all + P.twid0 + 2 * FFT_MAXN, nz);
+  load_pos(pos, twid_all + P.twid0 + 2 * FFT_MAXN, nz);
   __syncthreads();
-  float2 *res = lds_fft_lines<POW2>(bx_, by_, n, stw, sign);
-  float2 *rl = res + l * FFT_MAXN;
-  if (!on) return;
-  if (pass == 0) {
-    float2 *dst = cmesh + cmesh0 + (long)line * nzh;
-    for (int t = tid; t < nzh; t += FFT_T) dst[t] = rl[t];
-  } else if (pass == 4) {
-    if (P.ik) {   // (phi, Ex, Ey, Ez) interleaved per point: the gather reads one float4
-      float *dst = mesh + P.mesh0 + 4 * ((long)line * nz) + comp;
-      for (int t = tid; t < n; t += FFT_T) dst[4 * t] = rl[t].x;
-    } else {
-      float *dst = mesh + mesh0 + (long)line * nz;
-      for (int t = tid; t < n; t += FFT_T) dst[t] = rl[t].x;
-    }
-  } else {
-    const int xi = line / nzh, kz = line % nzh;
-    float2 *dst = cmesh + cmesh0 + (long)xi * ny * nzh + kz;
-    for (int t = tid; t < n; t += FFT_T) dst[(long)t * nzh] = rl[t];
+  const float2 *src = cmesh + P.cmesh0 + (P.ik ? comp + 1 : 0) * (long)nlines * nzh + l0;
+  batched<4>(nzh * FZ_LINES,
+             [&](int t) {
+               const int k = t / FZ_LINES, l = t % FZ_LINES;
+               const float2 *o = src + (long)k * nlines + 2 * l;
+               float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+               if (2 * l < nl) { const float2 a = o[0]; v.x = a.x; v.y = a.y; }
+               if (2 * l + 1 < nl) { const float2 b = o[1]; v.z = b.x; v.w = b.y; }
+               return v;
+             },
+             [&](int t, float4 v) {
+               const int k = t / FZ_LINES;
+               float2 *x = buf + (t % FZ_LINES) * ls;
+               if (k == 0 || 2 * k == nz) {
+                 x[pos[k]] = make_float2(v.x, v.z);   // real lines: no imaginary part here
+               } else {
+                 x[pos[k]] = make_float2(v.x - v.w, v.y + v.z);
+                 x[pos[nz - k]] = make_float2(v.x + v.w, v.z - v.y);
+               }
+             });
+  __syncthreads();
+  fft_inverse(buf, FZ_LINES, ls, 1, nz, P.rad[2], stw);
+  const float *fb = reinterpret_cast<const float *>(buf);
+  const int out = P.ik ? nz : P.mzs;
+  const float inv = 1.f / (float)out;
+  for (int t = threadIdx.x; t < nl * out; t += blockDim.x) {
+    const int l = div_small(t, inv), z = t - l * out;
+    const float v = fb[2 * ((l >> 1) * ls + (z < nz ? z : z - nz)) + (l & 1)];
+    if (P.ik) mesh[P.omesh0 + 4 * ((long)l0 * nz + t) + comp] = v;
+    else mesh[P.omesh0 + (long)l0 * out + t] = v;
   }
 }
 
-// x lines: forward FFT, multiply by the influence function, inverse FFT.
-// Also the mesh energy 1/2 sum G |rho_k|^2 and its virial
-// W_ab = sum e_k (delta_ab - 2 k_a k_b (1/k^2 + 1/(4 eta^2))); ENER false:
-// the convolution alone (inner MD steps, whose energies are not formed).
-// IK: systems whose field is formed on the mesh also get E_a = -i k_a phi_k
-// (k from the signed x, y index and the half-spectrum z index,
-// pppm.c:577-594), each inverse-transformed along x into its own component.
-template <bool VIR, bool POW2, bool ENER = true, bool IK = false>
-__global__ void __launch_bounds__(FFT_TB, 4) k_fft_xgreen(const SysParams *__restrict__ sp,
-                                                       const float2 *__restrict__ twid_all,
-                                                       const float *__restrict__ green,
-                                                       float2 *__restrict__ cmesh,
-                                                       double *__restrict__ part,
-                                                       int *__restrict__ done,
-                                                       double *__restrict__ acc,
-                                                       double *__restrict__ kvir, int want_virial,
-                                                       int maxblk) {
-  __shared__ float2 bx_[FFT_LINES * FFT_MAXN], by_[FFT_LINES * FFT_MAXN];
-  __shared__ float2 stw[FFT_MAXN];
-  constexpr int NV = VIR ? 10 : 1;   // energy [, virial]
-  __shared__ double red[FFT_TB / 64][NV];
-  __shared__ int last;
-  (void)acc;
-  const int s = blockIdx.y;
-  const SysParams &P = sp[s];
-  if (P.kmode != 1) return;
-  const int nx = P.nx, ny = P.ny, nz = P.nz, nzh = nz / 2 + 1;
-  const int nlines = ny * nzh;
-  const int nblk = (nlines + FFT_LINES - 1) / FFT_LINES;
-  if ((int)blockIdx.x >= nblk) return;
-  load_tw(stw, twid_all + P.twid0, nx);
-  const int l = threadIdx.x / FFT_T, tid = threadIdx.x % FFT_T;
-  const int line = blockIdx.x * FFT_LINES + l;
-  const bool on = line < nlines;
-  const int ky = on ? line / nzh : 0, kz = on ? line % nzh : 0;
-  float2 *xl = bx_ + l * FFT_MAXN;
-  float2 *src = cmesh + P.cmesh0 + (long)ky * nzh + kz;
-  const long xstride = (long)ny * nzh;
-  if (on)
-    for (int t = tid; t < nx; t += FFT_T) xl[t] = src[t * xstride];
-  __syncthreads();
-  float2 *res = lds_fft_lines<POW2>(bx_, by_, nx, stw, -1);
-  float2 *oth = (res == bx_) ? by_ : bx_;
-  double e = 0, w[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-  if (on) {
-    float2 *rl = res + l * FFT_MAXN;
-    const float *g = green + P.green0 + ((long)ky * nzh + kz) * nx;
-    const double mult = (kz == 0 || (nz % 2 == 0 && kz == nz / 2)) ? 1.0 : 2.0;
-    const int jy = ky > ny / 2 ? ky - ny : ky;
-    const double c4 = 0.25 / (P.eta * P.eta);
-    for (int t = tid; t < nx; t += FFT_T) {
-      const float2 v = rl[t];
-      const float gg = g[t];
-      const double ek = ENER ? 0.5 * mult * (double)gg * ((double)v.x * v.x + (double)v.y * v.y) : 0.0;
-      e += ek;
-      if (VIR && gg != 0.f) {
-        const int jx = t > nx / 2 ? t - nx : t;
-        double k[3];
-        for (int a = 0; a < 3; a++) k[a] = P.RL[a] * jx + P.RL[3 + a] * jy + P.RL[6 + a] * kz;
-        const double k2 = k[0] * k[0] + k[1] * k[1] + k[2] * k[2];
-        const double f = 2 * (1 / k2 + c4);
-        for (int a = 0; a < 3; a++)
-          for (int b = 0; b < 3; b++) w[3 * a + b] += ek * ((a == b ? 1.0 : 0.0) - f * k[a] * k[b]);
-      }
-      rl[t] = make_float2(v.x * gg, v.y * gg);
-    }
-  }
-  if constexpr (IK) {
-    // each thread keeps its own points of phi_k in registers and rebuilds
-    // the line in LDS for every component
-    constexpr int NK = FFT_MAXN / FFT_T;
-    float2 keep[NK];
-    float2 *rl = res + l * FFT_MAXN;
-#pragma unroll
-    for (int j = 0; j < NK; j++) {
-      const int t = tid + j * FFT_T;
-      keep[j] = (on && t < nx) ? rl[t] : make_float2(0.f, 0.f);
-    }
-    const int jy = ky > ny / 2 ? ky - ny : ky;
-    const int ncomp = P.ik ? 4 : 1;
-    const long cstride = (long)nx * ny * nzh;
-    for (int c = 0; c < ncomp; c++) {
-      if (c > 0) {
-        const int a = c - 1;
-#pragma unroll
-        for (int j = 0; j < NK; j++) {
-          const int t = tid + j * FFT_T;
-          if (on && t < nx) {
-            const int jx = t > nx / 2 ? t - nx : t;
-            const float k = (float)(P.RL[a] * jx + P.RL[3 + a] * jy + P.RL[6 + a] * kz);
-            rl[t] = make_float2(k * keep[j].y, -k * keep[j].x);
+// The x transforms of a tile of one kz plane in LDS (its ncol columns y0 ..
+// of the plane's ny, x points ls apart): forward, the influence function,
+// inverse, and what the points add to the mesh energy 1/2 sum G |rho_k|^2
+// and its virial W_ab = sum e_k (delta_ab - 2 k_a k_b (1/k^2 + 1/(4 eta^2)))
+// (ENER, VIR).  comp > 0: E_a = -i k_a phi_k, a = comp - 1, k from the signed
+// x, y index and the half-spectrum z index (pppm.c:577-594).
+// fx, fy: signed frequencies of the places along x and y.
+template <bool VIR, bool ENER, bool IK>
+__device__ __forceinline__ void convolve_x(const SysParams &P, float2 *buf, int ls, int ncol, int y0,
+                                           int kz, int comp, const float2 *twx, const short *fx,
+                                           const short *fy, const float *__restrict__ green,
+                                           double &e, double *w) {
+  const float *g = green + P.green0 + (long)kz * P.nx * P.ny + y0;
+  const int ny = P.ny;
+  const double mult = (kz == 0 || 2 * kz == P.nz) ? 1.0 : 2.0;
+  const double c4 = 0.25 / (P.eta * P.eta);
+  fft_forward<false>(buf, ncol, 1, ls, P.nx, P.rad[0], twx);
+  fft_middle(
+      buf, ncol, 1, ls, P.nx, P.rad[0], [&](int c, int px) { return g[px * ny + c]; },
+      [&](int c, int px, float gg, float2 &v) {
+        if (ENER && comp == 0) {
+          const double ek = 0.5 * mult * (double)gg * ((double)v.x * v.x + (double)v.y * v.y);
+          e += ek;
+          if (VIR && gg != 0.f) {
+            double k[3];
+            for (int a = 0; a < 3; a++)
+              k[a] = P.RL[a] * fx[px] + P.RL[3 + a] * fy[y0 + c] + P.RL[6 + a] * kz;
+            const double k2 = k[0] * k[0] + k[1] * k[1] + k[2] * k[2];
+            const double f = 2 * (1 / k2 + c4);
+            for (int a = 0; a < 3; a++)
+              for (int b = 0; b < 3; b++)
+                w[3 * a + b] += ek * ((a == b ? 1.0 : 0.0) - f * k[a] * k[b]);
           }
         }
-      }
-      __syncthreads();
-      float2 *out = lds_fft_lines<POW2>(res, oth, nx, stw, +1);
-      if (on) {
-        const float2 *ol = out + l * FFT_MAXN;
-        for (int t = tid; t < nx; t += FFT_T) src[c * cstride + t * xstride] = ol[t];
-      }
-      __syncthreads();   // the next component rebuilds its line in these buffers
-    }
-  } else {
-    __syncthreads();
-    res = lds_fft_lines<POW2>(res, oth, nx, stw, +1);
-    if (on) {
-      float2 *rl = res + l * FFT_MAXN;
-      for (int t = tid; t < nx; t += FFT_T) src[t * xstride] = rl[t];
-    }
-  }
-  if constexpr (!ENER) return;
-  // deterministic block partials, reduced by the last block
+        {   // rounded here in every variant of the kernel, not fused into the butterfly
+#pragma clang fp contract(off)
+          v = make_float2(v.x * gg, v.y * gg);
+          if (IK && comp > 0) {
+            const int a = comp - 1;
+            const float k = (float)(P.RL[a] * fx[px] + P.RL[3 + a] * fy[y0 + c] + P.RL[6 + a] * kz);
+            v = make_float2(k * v.y, -k * v.x);
+          }
+        }
+      });
+  fft_inverse<false>(buf, ncol, 1, ls, P.nx, P.rad[0], twx);
+}
+
+template <int NV, int TB>
+__device__ __forceinline__ void mesh_energy(double e, const double *w, int s, int nblk, int blk,
+                                            double *part, int *done, double *acc, double *kvir,
+                                            int maxblk) {
+  __shared__ double red[TB / 64][NV];
+  __shared__ int last;
   double vals[NV];
   vals[0] = e;
-  if constexpr (VIR)
-    for (int c = 0; c < 9; c++) vals[1 + c] = w[c];
-  if (finish_partials<NV, NV, FFT_TB>(vals, part + (long)s * maxblk * NV, nblk, blockIdx.x,
-                                      &done[s], red, &last)) {
+  for (int c = 1; c < NV; c++) vals[c] = w[c - 1];
+  if (finish_partials<NV, NV, TB>(vals, part + (long)s * maxblk * NV, nblk, blk, &done[s], red, &last)) {
     acc[s * NACC + ACC_KSPACE_E] = vals[0];
-    for (int c = 0; c < 9; c++) kvir[9 * s + c] = VIR ? vals[1 + c] : 0.0;
+    for (int c = 0; c < 9; c++) kvir[9 * s + c] = NV > 1 ? vals[c + 1] : 0.0;
   }
+}
+
+// One kz plane of a system: forward y and x, the influence function, inverse
+// x and y, all in LDS, where the four line passes of a mesh used to go to
+// memory and back and cost a launch each.  One block per plane (and per
+// component with the field on the mesh, which repeats the forward transforms
+// rather than wait for them); 512 threads of at most 64 registers and up to
+// 46 KB of LDS, so that a block fits beside three blocks of the pair kernel
+// on a CU.  What bounds it is the chain of nine LDS round trips, about 1 us
+// each: 12 us at 48^3 and 16 at 64^3, against 21 and 22 us and two launches
+// more for a pass per axis (39 against 14 at 45 x 42 x 48 with the field on
+// the mesh).  Pairing the z and y lines of an x slab in one block instead and
+// leaving x alone takes as long (9 + 7 + 9 us at 48^3 against 6 + 12 + 6).
+template <bool VIR, bool ENER, bool IK>
+__global__ void __launch_bounds__(FP_TB, (VIR || ENER) ? 4 : 8) k_fft_plane(const SysParams *__restrict__ sp,
+                                                        const float2 *__restrict__ twid_all,
+                                                        const float *__restrict__ green,
+                                                        float2 *__restrict__ cmesh,
+                                                        double *__restrict__ part,
+                                                        int *__restrict__ done,
+                                                        double *__restrict__ acc,
+                                                        double *__restrict__ kvir, int maxblk) {
+  extern __shared__ float2 plane[];
+  __shared__ float2 twx[FFT_MAXN], twy[FFT_MAXN];
+  __shared__ short fx[FFT_MAXN], fy[FFT_MAXN];
+  const int s = blockIdx.y, kz = blockIdx.x, comp = IK ? blockIdx.z : 0;
+  const SysParams &P = sp[s];
+  if (P.kmode != 1 || !P.plane) return;
+  const int nx = P.nx, ny = P.ny, nzh = P.nz / 2 + 1, ls = ny | 1;
+  if (kz >= nzh || (IK && comp > 0 && !P.ik)) return;
+  load_tw(twx, twid_all + P.twid0, nx);
+  load_tw(twy, twid_all + P.twid0 + FFT_MAXN, ny);
+  if (VIR || IK) {
+    load_freq(fx, twid_all + P.twid0, nx);
+    load_freq(fy, twid_all + P.twid0 + FFT_MAXN, ny);
+  }
+  float2 *src = cmesh + P.cmesh0 + (long)kz * nx * ny;
+  const float inv = 1.f / (float)ny;
+  batched<8>(nx * ny, [&](int t) { return src[t]; },
+             [&](int t, float2 v) { plane[t + div_small(t, inv) * (ls - ny)] = v; });
+  __syncthreads();
+  fft_forward(plane, nx, ls, 1, ny, P.rad[1], twy);
+  double e = 0, w[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+  convolve_x<VIR, ENER, IK>(P, plane, ls, ny, 0, kz, comp, twx, fx, fy, green, e, w);
+  fft_inverse(plane, nx, ls, 1, ny, P.rad[1], twy);
+  // the field's components go beside the density's spectrum, which the
+  // blocks of the other components read
+  float2 *dst = src + (IK && P.ik ? (comp + 1) * (long)nx * ny * nzh : 0);
+  for (int t = threadIdx.x; t < nx * ny; t += FP_TB) {
+    const int x = div_small(t, inv);
+    dst[t] = plane[t + x * (ls - ny)];
+  }
+  if (ENER && comp == 0)
+    mesh_energy<VIR ? 10 : 1, FP_TB>(e, w, s, nzh, kz, part, done, acc, kvir, maxblk);
+}
+
+// Planes too large for that: y lines forward and inverse in passes of their
+// own, and x lines with the influence function between them, 16 lines a block.
+constexpr int FL_LINES = 16, FL_TB = 256;
+
+template <bool INV>
+__global__ void __launch_bounds__(FL_TB, 4) k_fft_y(const SysParams *__restrict__ sp,
+                                                    const float2 *__restrict__ twid_all,
+                                                    float2 *__restrict__ cmesh) {
+  __shared__ float2 buf[FL_LINES * (FFT_MAXN + 1)], twy[FFT_MAXN];
+  const SysParams &P = sp[blockIdx.y];
+  if (P.kmode != 1 || P.plane) return;
+  const int comp = blockIdx.z;
+  if (comp > 0 && !P.ik) return;
+  const int ny = P.ny, ls = ny | 1, nlines = P.nx * (P.nz / 2 + 1);
+  const int l0 = blockIdx.x * FL_LINES, nl = min(FL_LINES, nlines - l0);
+  if (nl <= 0) return;
+  load_tw(twy, twid_all + P.twid0 + FFT_MAXN, ny);
+  float2 *src = cmesh + P.cmesh0 + (INV && P.ik ? comp + 1 : 0) * (long)nlines * ny + (long)l0 * ny;
+  const float inv = 1.f / (float)ny;
+  batched<8>(nl * ny, [&](int t) { return src[t]; },
+             [&](int t, float2 v) { buf[t + div_small(t, inv) * (ls - ny)] = v; });
+  __syncthreads();
+  if (INV) fft_inverse(buf, nl, ls, 1, ny, P.rad[1], twy);
+  else fft_forward(buf, nl, ls, 1, ny, P.rad[1], twy);
+  for (int t = threadIdx.x; t < nl * ny; t += FL_TB) src[t] = buf[t + div_small(t, inv) * (ls - ny)];
+}
+
+template <bool VIR, bool ENER, bool IK>
+__global__ void __launch_bounds__(FL_TB, 4) k_fft_x(const SysParams *__restrict__ sp,
+                                                    const float2 *__restrict__ twid_all,
+                                                    const float *__restrict__ green,
+                                                    float2 *__restrict__ cmesh,
+                                                    double *__restrict__ part,
+                                                    int *__restrict__ done,
+                                                    double *__restrict__ acc,
+                                                    double *__restrict__ kvir, int maxblk) {
+  constexpr int LS = FL_LINES + 1;
+  __shared__ float2 buf[LS * FFT_MAXN], twx[FFT_MAXN];
+  __shared__ short fx[FFT_MAXN], fy[FFT_MAXN];
+  const int s = blockIdx.y, comp = IK ? blockIdx.z : 0;
+  const SysParams &P = sp[s];
+  if (P.kmode != 1 || P.plane || (IK && comp > 0 && !P.ik)) return;
+  const int nx = P.nx, ny = P.ny, nzh = P.nz / 2 + 1, nt = (ny + FL_LINES - 1) / FL_LINES;
+  if ((int)blockIdx.x >= nzh * nt) return;
+  const int kz = blockIdx.x / nt, y0 = blockIdx.x % nt * FL_LINES, nl = min(FL_LINES, ny - y0);
+  load_tw(twx, twid_all + P.twid0, nx);
+  if (VIR || IK) {
+    load_freq(fx, twid_all + P.twid0, nx);
+    load_freq(fy, twid_all + P.twid0 + FFT_MAXN, ny);
+  }
+  float2 *src = cmesh + P.cmesh0 + (long)kz * nx * ny + y0;
+  batched<8>(nx * FL_LINES,
+             [&](int t) {
+               const int c = t % FL_LINES;
+               return c < nl ? src[t / FL_LINES * ny + c] : make_float2(0.f, 0.f);
+             },
+             [&](int t, float2 v) { buf[t / FL_LINES * LS + t % FL_LINES] = v; });
+  __syncthreads();
+  double e = 0, w[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+  convolve_x<VIR, ENER, IK>(P, buf, LS, nl, y0, kz, comp, twx, fx, fy, green, e, w);
+  float2 *dst = src + (IK && P.ik ? (comp + 1) * (long)nx * ny * nzh : 0);
+  for (int t = threadIdx.x; t < nx * FL_LINES; t += FL_TB) {
+    const int x = t / FL_LINES, c = t % FL_LINES;
+    if (c < nl) dst[(long)x * ny + c] = buf[x * LS + c];
+  }
+  if (ENER && comp == 0)
+    mesh_energy<VIR ? 10 : 1, FL_TB>(e, w, s, nzh * nt, blockIdx.x, part, done, acc, kvir, maxblk);
+}
+
+// Mesh buffers of one system, whose sizes, order and ik are set: the charge
+// mesh at mesh0, the mesh the gather reads at omesh0, the half spectra at
+// cmesh0; mesh and cmesh (floats and complex numbers so far) advance.
+// A plane goes through k_fft_plane if it leaves three pair blocks of a CU
+// their LDS (48 KB of 160 free beside them).
+int p3m_mesh_layout(SysParams &P, long &mesh, long &cmesh) {
+  const int n[3] = {P.nx, P.ny, P.nz};
+  for (int d = 0; d < 3; d++)
+    if (n[d] > FFT_MAXN || !fft_plan(n[d], P.rad[d])) return -1;
+  const long M = (long)P.nx * P.ny * P.nz, Mc = (long)P.nx * P.ny * (P.nz / 2 + 1);
+  P.plane = P.nx * (P.ny | 1) <= FFT_PLANE_MAX;
+  P.mzs = P.nz + P.order - 1;
+  P.mesh0 = mesh;
+  mesh = (mesh + M + 3) & ~3L;   // 16-byte aligned: an ik system's points are float4
+  P.omesh0 = mesh;
+  mesh = (mesh + (P.ik ? 4 * M : (long)P.nx * P.ny * P.mzs) + 3) & ~3L;
+  P.cmesh0 = cmesh;
+  cmesh += (P.ik ? 5 : 1) * Mc;   // the density's, then phi, Ex, Ey, Ez of an ik system
+  return 0;
+}
+
+// The system's tables: exp(-2 pi i t / n) for each axis (128 entries), then
+// for each axis (place of frequency t, signed frequency of place t) as ints
+// (128 entries).
+void p3m_twiddles(const SysParams &P, std::vector<float2> &tw) {
+  const int n[3] = {P.nx, P.ny, P.nz};
+  const size_t at = tw.size();
+  tw.resize(at + P3M_TWIDDLES);
+  for (int d = 0; d < 3; d++)
+    for (int t = 0; t < FFT_MAXN; t++) {
+      const double a = -2 * M_PI * (t % n[d]) / n[d];
+      tw[at + d * FFT_MAXN + t] = make_float2((float)cos(a), (float)sin(a));
+    }
+  for (int d = 0; d < 3; d++) {
+    float2 *f = &tw[at + (3 + d) * FFT_MAXN];
+    for (int k = 0; k < n[d]; k++) {
+      const int p = fft_pos(k, n[d], P.rad[d]), sg = k > n[d] / 2 ? k - n[d] : k;
+      memcpy(&f[k].x, &p, sizeof p);
+      memcpy(&f[p].y, &sg, sizeof sg);
+    }
+  }
+}
+
+// where the influence function's value at (ix, iy, kz) is stored, relative to green0
+long p3m_green_at(const SysParams &P, int ix, int iy, int kz) {
+  return ((long)kz * P.nx + fft_pos(ix, P.nx, P.rad[0])) * P.ny + fft_pos(iy, P.ny, P.rad[1]);
+}
+
+// partial sums of the mesh energy: one per block of the x transforms
+int p3m_energy_blocks(const SysParams &P) {
+  return (P.nz / 2 + 1) * (P.plane ? 1 : (P.ny + FL_LINES - 1) / FL_LINES);
 }
 
 // IK: systems whose field was formed on the mesh; phi and E_a are
@@ -702,7 +780,7 @@ __global__ void __launch_bounds__(256) k_p3m_gather(const SysParams *__restrict_
     iy[a] = wrap(g.y + istart + a, ny);
     iz[a] = wrap(g.z + istart + a, nz);
   }
-  const float *m0 = mesh + Q.mesh0;
+  const float *m0 = mesh + Q.omesh0;
   float ph = 0.f, e0 = 0.f, e1 = 0.f, e2 = 0.f;
   if constexpr (IK) {
     // the last inverse pass leaves (phi, Ex, Ey, Ez) interleaved per point
@@ -734,13 +812,15 @@ __global__ void __launch_bounds__(256) k_p3m_gather(const SysParams *__restrict_
   for (int a = 0; a < P; a++) {
 #pragma unroll
     for (int b = 0; b < P; b++) {
-      const float *col = m0 + ((long)ix[a] * ny + iy[b]) * nz;
+      // the run of P points along z, contiguous in the padded line (the
+      // compiler makes it wide loads: two instead of five at order 5)
+      float run[P];
+      __builtin_memcpy(run, m0 + (ix[a] * ny + iy[b]) * Q.mzs + iz[0], sizeof run);
       float cp = 0.f, cz = 0.f;
 #pragma unroll
       for (int c = 0; c < P; c++) {
-        const float pm = col[iz[c]];
-        cp += wz[c] * pm;
-        cz += dz[c] * pm;
+        cp += wz[c] * run[c];
+        cz += dz[c] * run[c];
       }
       const float wxy = wx[a] * wy[b];
       ph += wxy * cp;
@@ -756,60 +836,71 @@ __global__ void __launch_bounds__(256) k_p3m_gather(const SysParams *__restrict_
   kres[4 * si + 3] = (double)e0 * T[6] + (double)e1 * T[7] + (double)e2 * T[8];
 }
 
-// forward z, y passes; x pass with the influence function; inverse y, z.
-// sp / nsg: the systems the grid's y extent covers (all of them, or one
-// system's parameters with nsg = 1); ik: some system forms its field on the
-// mesh (four components through the inverse passes)
-template <bool POW2, bool IK>
-static void launch_xgreen(Engine &e, int want_virial, int energies, hipStream_t st, dim3 g,
-                          const SysParams *sp) {
-  if (want_virial)
-    hipLaunchKernelGGL((k_fft_xgreen<true, POW2, true, IK>), g, dim3(FFT_TB), 0, st, sp,
-                       e.d_twid, e.d_green, e.d_cmesh, e.d_part, e.d_done + e.nsys, e.d_acc,
-                       e.d_kres + 4L * e.nsite, want_virial, e.nblk_part);
-  else if (energies)
-    hipLaunchKernelGGL((k_fft_xgreen<false, POW2, true, IK>), g, dim3(FFT_TB), 0, st, sp,
-                       e.d_twid, e.d_green, e.d_cmesh, e.d_part, e.d_done + e.nsys, e.d_acc,
-                       e.d_kres + 4L * e.nsite, want_virial, e.nblk_part);
-  else
-    hipLaunchKernelGGL((k_fft_xgreen<false, POW2, false, IK>), g, dim3(FFT_TB), 0, st, sp,
-                       e.d_twid, e.d_green, e.d_cmesh, e.d_part, e.d_done + e.nsys, e.d_acc,
-                       e.d_kres + 4L * e.nsite, want_virial, e.nblk_part);
+// The convolution: forward z, the kz planes, inverse z.  sp / nsg: the systems
+// the grid's y extent covers (all of them, or one system's parameters with
+// nsg = 1), hp their host copies; halo: the spreading blocks' partials the z
+// pass sums (null: the real mesh holds the charges).
+template <bool VIR, bool ENER, bool IK>
+static void launch_planes(Engine &e, hipStream_t st, const SysParams *sp, const SysParams *hp, int nsg) {
+  int np = 0, lds = 0, ny = 0, nx = 0;
+  for (int s = 0; s < nsg; s++) {
+    const SysParams &P = hp[s];
+    if (P.kmode != 1) continue;
+    const int nzh = P.nz / 2 + 1;
+    if (P.plane) {
+      np = std::max(np, nzh);
+      lds = std::max(lds, P.nx * (P.ny | 1));
+    } else {
+      ny = std::max(ny, (P.nx * nzh + FL_LINES - 1) / FL_LINES);
+      nx = std::max(nx, p3m_energy_blocks(P));
+    }
+  }
+  const int nc = IK ? 4 : 1;
+  if (np)
+    hipLaunchKernelGGL((k_fft_plane<VIR, ENER, IK>), dim3(np, nsg, nc), dim3(FP_TB),
+                       lds * sizeof(float2), st, sp, e.d_twid, e.d_green, e.d_cmesh, e.d_part,
+                       e.d_done + e.nsys, e.d_acc, e.d_kres + 4L * e.nsite, e.nblk_part);
+  if (nx) {
+    hipLaunchKernelGGL(k_fft_y<false>, dim3(ny, nsg), dim3(FL_TB), 0, st, sp, e.d_twid, e.d_cmesh);
+    hipLaunchKernelGGL((k_fft_x<VIR, ENER, IK>), dim3(nx, nsg, nc), dim3(FL_TB), 0, st, sp, e.d_twid,
+                       e.d_green, e.d_cmesh, e.d_part, e.d_done + e.nsys, e.d_acc,
+                       e.d_kres + 4L * e.nsite, e.nblk_part);
+    hipLaunchKernelGGL(k_fft_y<true>, dim3(ny, nsg, nc), dim3(FL_TB), 0, st, sp, e.d_twid, e.d_cmesh);
+  }
 }
 
-// halo: the spreading blocks' partials the z pass sums (null: the real
-// mesh holds the charges)
-template <bool POW2>
-static void launch_fft(Engine &e, int want_virial, int energies, hipStream_t st, int maxx,
-                       int maxy, int maxz, const SysParams *sp, int nsg, bool ik,
-                       const unsigned long long *halo) {
+static void launch_fft(Engine &e, int want_virial, int energies, hipStream_t st, const SysParams *sp,
+                       const SysParams *hp, int nsg, const unsigned long long *halo) {
+  int nz = 0;
+  bool ik = false;
+  for (int s = 0; s < nsg; s++)
+    if (hp[s].kmode == 1) {
+      nz = std::max(nz, (hp[s].nx * hp[s].ny + 2 * FZ_LINES - 1) / (2 * FZ_LINES));
+      ik |= hp[s].ik != 0;
+    }
   if (halo)
-    hipLaunchKernelGGL((k_fft_pass<POW2, true>), dim3(maxz, nsg), dim3(FFT_TB), 0, st, sp,
-                       e.d_twid, e.d_mesh, e.d_cmesh, 0, halo);
+    hipLaunchKernelGGL(k_fft_z<true>, dim3(nz, nsg), dim3(FZ_TB), 0, st, sp, e.d_twid, e.d_mesh,
+                       e.d_cmesh, halo);
   else
-    hipLaunchKernelGGL((k_fft_pass<POW2>), dim3(maxz, nsg), dim3(FFT_TB), 0, st, sp,
-                       e.d_twid, e.d_mesh, e.d_cmesh, 0, nullptr);
-  hipLaunchKernelGGL((k_fft_pass<POW2>), dim3(maxy, nsg), dim3(FFT_TB), 0, st, sp,
-                     e.d_twid, e.d_mesh, e.d_cmesh, 1, nullptr);
-  if (ik) launch_xgreen<POW2, true>(e, want_virial, energies, st, dim3(maxx, nsg), sp);
-  else launch_xgreen<POW2, false>(e, want_virial, energies, st, dim3(maxx, nsg), sp);
-  const int ncomp = ik ? 4 : 1;
-  hipLaunchKernelGGL((k_fft_pass<POW2>), dim3(maxy, nsg, ncomp), dim3(FFT_TB), 0, st, sp,
-                     e.d_twid, e.d_mesh, e.d_cmesh, 3, nullptr);
-  hipLaunchKernelGGL((k_fft_pass<POW2>), dim3(maxz, nsg, ncomp), dim3(FFT_TB), 0, st, sp,
-                     e.d_twid, e.d_mesh, e.d_cmesh, 4, nullptr);
+    hipLaunchKernelGGL(k_fft_z<false>, dim3(nz, nsg), dim3(FZ_TB), 0, st, sp, e.d_twid, e.d_mesh,
+                       e.d_cmesh, halo);
+#define PLANES(V, E)                                             \
+  if (ik) launch_planes<V, E, true>(e, st, sp, hp, nsg);         \
+  else launch_planes<V, E, false>(e, st, sp, hp, nsg);
+  if (want_virial) { PLANES(true, true) }
+  else if (energies) { PLANES(false, true) }
+  else { PLANES(false, false) }
+#undef PLANES
+  hipLaunchKernelGGL(k_fft_zinv, dim3(nz, nsg, ik ? 4 : 1), dim3(FZ_TB), 0, st, sp, e.d_twid,
+                     e.d_cmesh, e.d_mesh);
 }
 
 int launch_p3m(Engine &e, int want_virial, hipStream_t st, int energies) {
-  int maxn = 0, maxbins = 0, maxz = 0, maxy = 0, maxx = 0;
+  int maxn = 0, maxbins = 0;
   for (auto &p : e.hsp)
     if (p.kmode == 1) {
       maxn = std::max(maxn, p.nsite);
       maxbins = std::max(maxbins, p.nbx * p.nby);
-      const int nzh = p.nz / 2 + 1;
-      maxz = std::max(maxz, (p.nx * p.ny + FFT_LINES - 1) / FFT_LINES);
-      maxy = std::max(maxy, (p.nx * nzh + FFT_LINES - 1) / FFT_LINES);
-      maxx = std::max(maxx, (p.ny * nzh + FFT_LINES - 1) / FFT_LINES);
     }
   if (maxn == 0) return 0;
   const int tb = 256;
@@ -819,12 +910,10 @@ int launch_p3m(Engine &e, int want_virial, hipStream_t st, int energies) {
                      e.d_bin_fill + e.nbin_total);
   bool used[MAXORDER + 1] = {false}, used_ad[MAXORDER + 1] = {false},
        used_ik[MAXORDER + 1] = {false};
-  bool ik = false;
   for (auto &p : e.hsp)
     if (p.kmode == 1) {
       used[p.order] = true;
       (p.ik ? used_ik : used_ad)[p.order] = true;
-      ik |= p.ik != 0;
     }
   // LDS of the spreading: the largest halo of the systems of each order
   size_t hbytes[MAXORDER + 1] = {0};
@@ -841,17 +930,8 @@ int launch_p3m(Engine &e, int want_virial, hipStream_t st, int energies) {
                        e.d_bin_fill, e.bcap, e.d_bgrid, e.d_bfrac, e.d_mesh);
   SPREAD(1) SPREAD(2) SPREAD(3) SPREAD(4) SPREAD(5) SPREAD(6) SPREAD(7)
 #undef SPREAD
-  const unsigned long long *halo = e.spread_halo ? e.d_halo : nullptr;
-  // meshes whose sides are all powers of two take FFT kernels built with
-  // the radix-4/2 stages only (fewer registers)
-  bool pow2 = true;
-  for (auto &p : e.hsp)
-    if (p.kmode == 1)
-      for (int n : {p.nx, p.ny, p.nz}) pow2 &= (n & (n - 1)) == 0;
-  if (pow2)
-    launch_fft<true>(e, want_virial, energies, st, maxx, maxy, maxz, e.d_sp, e.nsys, ik, halo);
-  else
-    launch_fft<false>(e, want_virial, energies, st, maxx, maxy, maxz, e.d_sp, e.nsys, ik, halo);
+  launch_fft(e, want_virial, energies, st, e.d_sp, e.hsp.data(), e.nsys,
+             e.spread_halo ? e.d_halo : nullptr);
 #define GATHER(PO)                                                                        \
   if (used_ad[PO])                                                                        \
     hipLaunchKernelGGL(k_p3m_gather<PO>, gs, dim3(tb), 0, st, e.d_sp, e.d_sgrid,     \
@@ -891,18 +971,7 @@ int launch_p3m_adjoint(Engine &e, int sys, const float4 *src, hipStream_t st) {
     default: set_last_error("assignment order out of range"); return -1;
   }
 #undef ADJ_ORDER
-  const int nzh = P.nz / 2 + 1;
-  const int maxz = (P.nx * P.ny + FFT_LINES - 1) / FFT_LINES;
-  const int maxy = (P.nx * nzh + FFT_LINES - 1) / FFT_LINES;
-  const int maxx = (P.ny * nzh + FFT_LINES - 1) / FFT_LINES;
-  bool pow2 = true;
-  for (int n : {P.nx, P.ny, P.nz}) pow2 &= (n & (n - 1)) == 0;
-  // the engine chose one FFT build for all its meshes; keep to it
-  for (auto &p : e.hsp)
-    if (p.kmode == 1)
-      for (int n : {p.nx, p.ny, p.nz}) pow2 &= (n & (n - 1)) == 0;
-  if (pow2) launch_fft<true>(e, 0, 0, st, maxx, maxy, maxz, sp, 1, false, nullptr);
-  else launch_fft<false>(e, 0, 0, st, maxx, maxy, maxz, sp, 1, false, nullptr);
+  launch_fft(e, 0, 0, st, sp, &P, 1, nullptr);
 #define ADJ_GATHER(PO)                                                                      \
   case PO:                                                                                  \
     hipLaunchKernelGGL(k_p3m_gather<PO>, gs, dim3(tb), 0, st, sp, e.d_sgrid, e.d_sfrac,     \
@@ -944,16 +1013,7 @@ int launch_p3m_ik_pass(Engine &e, int sys, const double *q, hipStream_t st) {
     default: set_last_error("assignment order out of range"); return -1;
   }
 #undef IK_SPREAD
-  const int nzh = P.nz / 2 + 1;
-  const int maxz = (P.nx * P.ny + FFT_LINES - 1) / FFT_LINES;
-  const int maxy = (P.nx * nzh + FFT_LINES - 1) / FFT_LINES;
-  const int maxx = (P.ny * nzh + FFT_LINES - 1) / FFT_LINES;
-  bool pow2 = true;
-  for (auto &p : e.hsp)   // the engine's one FFT build, as in the forward
-    if (p.kmode == 1)
-      for (int n : {p.nx, p.ny, p.nz}) pow2 &= (n & (n - 1)) == 0;
-  if (pow2) launch_fft<true>(e, 0, 0, st, maxx, maxy, maxz, sp, 1, true, nullptr);
-  else launch_fft<false>(e, 0, 0, st, maxx, maxy, maxz, sp, 1, true, nullptr);
+  launch_fft(e, 0, 0, st, sp, &P, 1, nullptr);
 #define IK_GATHER(PO)                                                                       \
   case PO:                                                                                  \
     hipLaunchKernelGGL((k_p3m_gather<PO, true>), gs, dim3(tb), 0, st, sp, e.d_sgrid,        \

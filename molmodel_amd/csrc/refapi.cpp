@@ -702,7 +702,7 @@ static void p3m_upload_params(p3m *p) {
     for (int ix = 0; ix < nx; ix++)
       for (int iy = 0; iy < ny; iy++)
         for (int iz = 0; iz < nzh; iz++)
-          g[((size_t)iy * nzh + iz) * nx + ix] = (float)p->green[((size_t)ix * ny + iy) * nzh + iz];
+          g[p3m_green_at(P, ix, iy, iz)] = (float)p->green[((size_t)ix * ny + iy) * nzh + iz];
     HIPCHK(hipMemcpy(p->e.d_green, g.data(), sizeof(float) * g.size(), hipMemcpyHostToDevice));
   }
 }
@@ -747,17 +747,18 @@ extern "C" p3m_t p3m_new(int nsite, const double ptv[9], double grid_spacing, in
   P.nbx = P.nx / P.bx;
   P.nby = P.ny / P.by;
   e.nbin_total = P.nbx * P.nby;   // d_bin_fill[nbin_total] records an overfull bin's need
-  e.nblk_part = std::max(1, (P.ny * nzh + P3M_FFT_LINES - 1) / P3M_FFT_LINES);
-  const size_t M = (size_t)P.nx * P.ny * P.nz, Mc = (size_t)P.nx * P.ny * nzh;
-  const size_t ncomp = P.ik ? 4 : 1;
+  long mesh = 0, cmesh = 0;
+  if (p3m_mesh_layout(P, mesh, cmesh)) die_msg("p3m_new", "mesh dimensions have no transform plan");
+  e.nblk_part = p3m_energy_blocks(P);
+  const size_t Mc = (size_t)P.nx * P.ny * nzh;
   HIPCHK(hipStreamCreateWithFlags(&e.stream, hipStreamNonBlocking));
   HIPCHK(hipMalloc((void **)&e.d_sp, sizeof(SysParams)));
   HIPCHK(hipMalloc((void **)&e.d_r, sizeof(double) * 3 * N));
   HIPCHK(hipMalloc((void **)&e.d_q, sizeof(double) * N));
   HIPCHK(hipMalloc((void **)&e.d_kres, sizeof(double) * (4 * (size_t)N + 9)));
   HIPCHK(hipMalloc((void **)&e.d_acc, sizeof(double) * NACC));
-  HIPCHK(hipMalloc((void **)&e.d_mesh, sizeof(float) * M * ncomp));
-  HIPCHK(hipMalloc((void **)&e.d_cmesh, sizeof(float2) * Mc * ncomp));
+  HIPCHK(hipMalloc((void **)&e.d_mesh, sizeof(float) * mesh));
+  HIPCHK(hipMalloc((void **)&e.d_cmesh, sizeof(float2) * cmesh));
   HIPCHK(hipMalloc((void **)&e.d_green, sizeof(float) * Mc));
   HIPCHK(hipMemset(e.d_green, 0, sizeof(float) * Mc));
   HIPCHK(hipMalloc((void **)&e.d_sgrid, sizeof(int4) * N));
@@ -774,12 +775,7 @@ extern "C" p3m_t p3m_new(int nsite, const double ptv[9], double grid_spacing, in
   HIPCHK(hipMalloc((void **)&e.d_done, sizeof(int) * 4));
   HIPCHK(hipMemset(e.d_done, 0, sizeof(int) * 4));
   std::vector<float2> tw;
-  for (int d = 0; d < 3; d++)
-    for (int t = 0; t < 128; t++) {
-      const int n = p->ngrid[d];
-      const double a = -2 * M_PI * (t % n) / n;
-      tw.push_back(make_float2((float)cos(a), (float)sin(a)));
-    }
+  p3m_twiddles(P, tw);
   HIPCHK(hipMalloc((void **)&e.d_twid, sizeof(float2) * tw.size()));
   HIPCHK(hipMemcpy(e.d_twid, tw.data(), sizeof(float2) * tw.size(), hipMemcpyHostToDevice));
   p3m_upload_params(p);
