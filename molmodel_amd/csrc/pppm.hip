@@ -40,6 +40,18 @@ namespace mmamd {
 
 constexpr float FIX_SCALE = 4294967296.0f;   // 2^32
 constexpr double FIX_INV = 1.0 / 4294967296.0;
+// A contribution in fixed point, to the nearest even: adding 1.5 2^20 to the
+// FP64 value leaves it in units of 2^-32 in the low bits (three instructions;
+// the conversion of a scaled float to 64 bits takes about ten).  Exact for
+// contributions below 2^19: sites with larger charges take the conversion.
+constexpr double FIX_MAGIC = 1572864.0;
+constexpr float FIX_MAXQ = 262144.f;
+template <bool WIDE = false>
+__device__ __forceinline__ unsigned long long to_fix(float x) {
+  if (WIDE) return (unsigned long long)__float2ll_rn(x * FIX_SCALE);
+  return (unsigned long long)(__double_as_longlong((double)x + FIX_MAGIC) -
+                              __double_as_longlong(FIX_MAGIC));
+}
 
 template <int P>
 __device__ __forceinline__ void bspline_w(float s, float *w, float *ndw) {
@@ -149,118 +161,220 @@ __global__ void __launch_bounds__(256) k_p3m_bin(const SysParams *__restrict__ s
 
 __device__ __forceinline__ int floor_div(int a, int b) { return a >= 0 ? a / b : -((-a + b - 1) / b); }
 
-// LDS accumulator: bx * by columns of nz points (the host keeps the product
-// within SPREAD_MAXPTS, see choose_spread_blocks)
-constexpr int SPREAD_MAXPTS = 4096;
+// The sites whose stencils reach a spreading block's columns: the bins of the
+// neighbouring column blocks (at most 8 per axis for P <= 7), flattened into
+// one list so that all threads work whatever the bins' sizes: thread t < nbin
+// takes bin t, wave 0 scans the counts.
+struct ReachedSites {
+  int start[64], off[65], nbin;
 
-// ADJ: the transpose of the gather's field instead of the charge: site i
-// contributes src_i . (dw_x w_y w_z, w_x dw_y w_z, w_x w_y dw_z) with dw the
-// negated weight derivatives the gather uses and src_i = q_i (R_i T) (the
-// adjoint of E_i = T^T sum_m dw phi_m for a given R_i), so that the
-// convolution and an ordinary gather of the result give
-// sum_i q_i R_i . dE_i/dq_j at every site j.
-template <int P, bool ADJ = false>
+  template <int P>
+  __device__ __forceinline__ void collect(const SysParams &Q, int X0, int Y0,
+                                          const int *__restrict__ fill, int bcap) {
+    constexpr int istart = -((P + 1) / 2 - 1);
+    const int bx = Q.bx, by = Q.by;
+    int xlo = floor_div(X0 - istart - P + 1, bx), xhi = floor_div(X0 + bx - 1 - istart, bx);
+    int ylo = floor_div(Y0 - istart - P + 1, by), yhi = floor_div(Y0 + by - 1 - istart, by);
+    if (xhi - xlo + 1 >= Q.nbx) { xlo = 0; xhi = Q.nbx - 1; }
+    if (yhi - ylo + 1 >= Q.nby) { ylo = 0; yhi = Q.nby - 1; }
+    const int ncy = yhi - ylo + 1, n = (xhi - xlo + 1) * ncy;   // <= 64
+    if (threadIdx.x < 64) {
+      int cnt = 0;
+      const int t = threadIdx.x;
+      if (t < n) {
+        const int ccx = mod_nonneg(xlo + t / ncy, Q.nbx), ccy = mod_nonneg(ylo + t % ncy, Q.nby);
+        const int b = Q.bin0 + ccx * Q.nby + ccy;
+        start[t] = b * bcap;
+        cnt = min(fill[b], bcap);
+      }
+      int incl = cnt;   // inclusive scan over the wave
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(incl, o);
+        if (t >= o) incl += y;
+      }
+      off[t + 1] = incl;
+      if (t == 0) { off[0] = 0; nbin = n; }
+    }
+    __syncthreads();
+  }
+  __device__ __forceinline__ int total() const { return off[nbin]; }
+  // where site u of the list is kept
+  __device__ __forceinline__ int slot(int u) const {
+    int lo = 0, hi = nbin - 1;   // last bin with off[bin] <= u
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (off[mid] <= u) lo = mid; else hi = mid - 1;
+    }
+    return start[lo] + (u - off[lo]);
+  }
+};
+
+// the block's points out to the mesh
+__device__ __forceinline__ void store_columns(const SysParams &Q, const unsigned long long *acc,
+                                              int X0, int Y0, float *__restrict__ mesh) {
+  const int nz = Q.nz, by = Q.by;
+  for (int t = threadIdx.x; t < Q.bx * by * nz; t += blockDim.x) {
+    const int gz = t % nz, gy = (t / nz) % by, gx = t / (nz * by);
+    mesh[Q.mesh0 + ((long)(X0 + gx) * Q.ny + (Y0 + gy)) * nz + gz] =
+        (float)((double)(long long)acc[t] * FIX_INV);
+  }
+}
+
+// Spreading by pulling.  One site per thread, which runs over the block's own
+// columns and takes the weights that its stencil has there, if any (with 2 x
+// 2 columns a reached site has on average 2.8 of the four; running over the
+// 25 columns of its stencil and testing each took 1 250 instructions a site).
+// What bounds it is instruction issue (72% of the cycles at 98 304 sites on
+// 64^3): every site is weighted again for each block that it reaches.  17.2
+// us there (24.2 before), 7.0 for 12 288 on 48^3 (11.1).
+//
+// stencil offset of the column k past the one at offset a (n columns round)
+__device__ __forceinline__ unsigned column_offset(unsigned a, unsigned k, unsigned n) {
+  const unsigned v = a + k, w = v - n;   // w is huge unless v >= n
+  return v < w ? v : w;
+}
+
+// swx, swy: this thread's columns of the block's staged weights, 256 apart
+template <int P, bool WIDE>
+__device__ __forceinline__ void spread_site(const SysParams &Q, int X0, int Y0, const int4 &g,
+                                            const float4 &f, float *swx, float *swy,
+                                            unsigned long long *acc) {
+  constexpr int istart = -((P + 1) / 2 - 1);
+  const int nz = Q.nz, bx = Q.bx, by = Q.by;
+  float wx[P], wy[P], wz[P];
+  bspline_w<P>(f.x, wx, nullptr);
+  bspline_w<P>(f.y, wy, nullptr);
+  bspline_w<P>(f.z, wz, nullptr);
+#pragma unroll
+  for (int k = 0; k < P; k++) {
+    swx[256 * k] = f.w * wx[k];
+    swy[256 * k] = wy[k];
+  }
+  int iz[P];
+#pragma unroll
+  for (int c = 0; c < P; c++) iz[c] = wrap(g.z + istart + c, nz);
+  const unsigned a0 = wrap(X0 - g.x - istart, Q.nx), b0 = wrap(Y0 - g.y - istart, Q.ny);
+  for (int ox = 0; ox < bx; ox++) {
+    const unsigned a = column_offset(a0, ox, Q.nx);
+    if (a >= P) continue;
+    const float wa = swx[256 * a];
+    unsigned long long *col = acc + ox * by * nz;
+    for (int oy = 0; oy < by; oy++, col += nz) {
+      const unsigned b = column_offset(b0, oy, Q.ny);
+      if (b >= P) continue;
+      const float w = wa * swy[256 * b];
+#pragma unroll
+      for (int c = 0; c < P; c++) atomicAdd(col + iz[c], to_fix<WIDE>(w * wz[c]));
+    }
+  }
+}
+
+template <int P>
 __global__ void __launch_bounds__(256) k_p3m_spread(const SysParams *__restrict__ sp,
                                                     const int *__restrict__ fill, int bcap,
                                                     const int4 *__restrict__ bgrid,
                                                     const float4 *__restrict__ bfrac,
-                                                    float *__restrict__ mesh,
-                                                    const float4 *__restrict__ src = nullptr) {
-  __shared__ unsigned long long acc[SPREAD_MAXPTS];
+                                                    float *__restrict__ mesh) {
+  extern __shared__ unsigned long long acc[];
+  __shared__ ReachedSites reached;
+  __shared__ float swx[P * 256], swy[P * 256];   // staged so that an offset can index them
   const int s = blockIdx.y;
   const SysParams &Q = sp[s];
   if (Q.kmode != 1 || Q.order != P) return;
   const int blk = blockIdx.x;
   if (blk >= Q.nbx * Q.nby) return;
-  const int bx = Q.bx, by = Q.by, nx = Q.nx, ny = Q.ny, nz = Q.nz;
-  const int bi = blk / Q.nby, bj = blk % Q.nby;
-  const int X0 = bi * bx, Y0 = bj * by;
-  const int npts = bx * by * nz;
-  for (int t = threadIdx.x; t < npts; t += blockDim.x) acc[t] = 0ull;
-  __syncthreads();
-  constexpr int istart = -((P + 1) / 2 - 1);
-  // neighbouring column blocks whose sites reach the owned columns (at most
-  // 8 per axis for P <= 7), flattened into one list of sites so that all
-  // threads work whatever the bins' sizes: thread t < nbins takes bin t,
-  // wave 0 scans the counts
-  __shared__ int sb_start[64], sb_off[65];
-  int xlo = floor_div(X0 - istart - P + 1, bx), xhi = floor_div(X0 + bx - 1 - istart, bx);
-  int ylo = floor_div(Y0 - istart - P + 1, by), yhi = floor_div(Y0 + by - 1 - istart, by);
-  if (xhi - xlo + 1 >= Q.nbx) { xlo = 0; xhi = Q.nbx - 1; }
-  if (yhi - ylo + 1 >= Q.nby) { ylo = 0; yhi = Q.nby - 1; }
-  const int ncy = yhi - ylo + 1, nbin = (xhi - xlo + 1) * ncy;   // <= 64
-  if (threadIdx.x < 64) {
-    int cnt = 0;
-    const int t = threadIdx.x;
-    if (t < nbin) {
-      const int ccx = mod_nonneg(xlo + t / ncy, Q.nbx), ccy = mod_nonneg(ylo + t % ncy, Q.nby);
-      const int b = Q.bin0 + ccx * Q.nby + ccy;
-      sb_start[t] = b * bcap;
-      cnt = min(fill[b], bcap);
-    }
-    int incl = cnt;   // inclusive scan over the wave
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int y = __shfl_up(incl, o);
-      if (t >= o) incl += y;
-    }
-    sb_off[t + 1] = incl;
-    if (t == 0) sb_off[0] = 0;
+  const int X0 = blk / Q.nby * Q.bx, Y0 = blk % Q.nby * Q.by;
+  for (int t = threadIdx.x; t < Q.bx * Q.by * Q.nz; t += blockDim.x) acc[t] = 0ull;
+  reached.collect<P>(Q, X0, Y0, fill, bcap);
+  const int total = reached.total();
+  // a site is loaded while the one before it is spread
+  float *wx = swx + threadIdx.x, *wy = swy + threadIdx.x;
+  int4 gn = make_int4(0, 0, 0, 0);
+  float4 fn = make_float4(0.f, 0.f, 0.f, 0.f);
+  auto load = [&](int u) {
+    if (u >= total) return;
+    const int t = reached.slot(u);
+    gn = bgrid[t];
+    fn = bfrac[t];
+  };
+  load(threadIdx.x);
+  for (int u = threadIdx.x; u < total; u += blockDim.x) {
+    const int4 g = gn;
+    const float4 f = fn;
+    load(u + blockDim.x);
+    if (fabsf(f.w) < FIX_MAXQ) spread_site<P, false>(Q, X0, Y0, g, f, wx, wy, acc);
+    else spread_site<P, true>(Q, X0, Y0, g, f, wx, wy, acc);
   }
   __syncthreads();
-  const int total = sb_off[nbin];
+  store_columns(Q, acc, X0, Y0, mesh);
+}
+
+// The transpose of the gather's field instead of the charge: site i
+// contributes src_i . (dw_x w_y w_z, w_x dw_y w_z, w_x w_y dw_z) with dw the
+// negated weight derivatives the gather uses and src_i = q_i (R_i T) (the
+// adjoint of E_i = T^T sum_m dw phi_m for a given R_i), so that the
+// convolution and an ordinary gather of the result give
+// sum_i q_i R_i . dE_i/dq_j at every site j.  The caller scales src to at
+// most about one.
+template <int P>
+__global__ void __launch_bounds__(256) k_p3m_spread_adj(const SysParams *__restrict__ sp,
+                                                        const int *__restrict__ fill, int bcap,
+                                                        const int4 *__restrict__ bgrid,
+                                                        const float4 *__restrict__ bfrac,
+                                                        float *__restrict__ mesh,
+                                                        const float4 *__restrict__ src) {
+  extern __shared__ unsigned long long acc[];
+  __shared__ ReachedSites reached;
+  const SysParams &Q = sp[0];
+  if (Q.kmode != 1 || Q.order != P) return;
+  const int blk = blockIdx.x;
+  if (blk >= Q.nbx * Q.nby) return;
+  const int nz = Q.nz, X0 = blk / Q.nby * Q.bx, Y0 = blk % Q.nby * Q.by;
+  for (int t = threadIdx.x; t < Q.bx * Q.by * nz; t += blockDim.x) acc[t] = 0ull;
+  reached.collect<P>(Q, X0, Y0, fill, bcap);
+  const int total = reached.total();
+  constexpr int istart = -((P + 1) / 2 - 1);
   for (int u = threadIdx.x; u < total; u += blockDim.x) {
-    int lo = 0, hi = nbin - 1;   // last bin with sb_off[bin] <= u
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (sb_off[mid] <= u) lo = mid; else hi = mid - 1;
-    }
-    const int t = sb_start[lo] + (u - sb_off[lo]);
+    const int t = reached.slot(u);
     const int4 g = bgrid[t];
     const float4 f = bfrac[t];
     float wx[P], wy[P], wz[P], dwx[P], dwy[P], dwz[P];
-    bspline_w<P>(f.x, wx, ADJ ? dwx : nullptr);
-    bspline_w<P>(f.y, wy, ADJ ? dwy : nullptr);
-    bspline_w<P>(f.z, wz, ADJ ? dwz : nullptr);
-    int lx[P], ly[P], iz[P];
+    bspline_w<P>(f.x, wx, dwx);
+    bspline_w<P>(f.y, wy, dwy);
+    bspline_w<P>(f.z, wz, dwz);
+    int iz[P];
 #pragma unroll
-    for (int a = 0; a < P; a++) {
-      lx[a] = wrap(g.x + istart + a, nx) - X0;
-      ly[a] = wrap(g.y + istart + a, ny) - Y0;
-      iz[a] = wrap(g.z + istart + a, nz);
-    }
-    float4 sv = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (ADJ) sv = src[g.w];
+    for (int c = 0; c < P; c++) iz[c] = wrap(g.z + istart + c, nz);
+    const float4 sv = src[g.w];
+    for (int ox = 0; ox < Q.bx; ox++) {
+      const int a = wrap(X0 + ox - g.x - istart, Q.nx);
+      if (a >= P) continue;
+      float wa = wx[0], da = dwx[0];
 #pragma unroll
-    for (int a = 0; a < P; a++) {
-      if (lx[a] < 0 || lx[a] >= bx) continue;
-      const float qa = f.w * wx[a];
+      for (int k = 1; k < P; k++) {
+        wa = a == k ? wx[k] : wa;
+        da = a == k ? dwx[k] : da;
+      }
+      for (int oy = 0; oy < Q.by; oy++) {
+        const int b = wrap(Y0 + oy - g.y - istart, Q.ny);
+        if (b >= P) continue;
+        float wb = wy[0], db = dwy[0];
 #pragma unroll
-      for (int bb = 0; bb < P; bb++) {
-        if (ly[bb] < 0 || ly[bb] >= by) continue;
-        unsigned long long *col = acc + (lx[a] * by + ly[bb]) * nz;
-        if (ADJ) {
-          const float al = sv.x * dwx[a] * wy[bb] + sv.y * wx[a] * dwy[bb];
-          const float be = sv.z * wx[a] * wy[bb];
-#pragma unroll
-          for (int c = 0; c < P; c++)
-            atomicAdd(col + iz[c],
-                      (unsigned long long)__float2ll_rn((al * wz[c] + be * dwz[c]) * FIX_SCALE));
-        } else {
-          const float qw = qa * wy[bb];
-#pragma unroll
-          for (int c = 0; c < P; c++)
-            atomicAdd(col + iz[c], (unsigned long long)__float2ll_rn(qw * wz[c] * FIX_SCALE));
+        for (int k = 1; k < P; k++) {
+          wb = b == k ? wy[k] : wb;
+          db = b == k ? dwy[k] : db;
         }
+        const float al = sv.x * da * wb + sv.y * wa * db;
+        const float be = sv.z * wa * wb;
+        unsigned long long *col = acc + (ox * Q.by + oy) * nz;
+#pragma unroll
+        for (int c = 0; c < P; c++) atomicAdd(col + iz[c], to_fix(al * wz[c] + be * dwz[c]));
       }
     }
   }
   __syncthreads();
-  for (int t = threadIdx.x; t < npts; t += blockDim.x) {
-    const int gz = t % nz, gy = (t / nz) % by, gx = t / (nz * by);
-    mesh[Q.mesh0 + ((long)(X0 + gx) * ny + (Y0 + gy)) * nz + gz] =
-        (float)((double)(long long)acc[t] * FIX_INV);
-  }
+  store_columns(Q, acc, X0, Y0, mesh);
 }
 
 // Spreading by owner: the block of column block k takes only the sites
@@ -275,7 +389,7 @@ __global__ void __launch_bounds__(256) k_p3m_spread(const SysParams *__restrict_
 // z offset c): the P lanes of a site write P consecutive points of a
 // column, in different LDS banks.
 template <int P>
-__global__ void __launch_bounds__(256) k_p3m_spread_halo(const SysParams *__restrict__ sp,
+__global__ void __launch_bounds__(512) k_p3m_spread_halo(const SysParams *__restrict__ sp,
                                                          const int *__restrict__ fill, int bcap,
                                                          const int4 *__restrict__ bgrid,
                                                          const float4 *__restrict__ bfrac,
@@ -307,15 +421,23 @@ __global__ void __launch_bounds__(256) k_p3m_spread_halo(const SysParams *__rest
     for (int k = 1; k < P; k++)
       if (c == k) wc = wz[k];
     const int iz = wrap(g.z + istart + c, nz);
-    unsigned long long *base = hacc + ((long)(g.x - X0) * HY + (g.y - Y0)) * nz + iz;
+    unsigned long long *base = hacc + ((g.x - X0) * HY + (g.y - Y0)) * nz + iz;
+    if (fabsf(f.w) < FIX_MAXQ) {
 #pragma unroll
-    for (int a = 0; a < P; a++) {
-      const float qa = f.w * wx[a];
+      for (int a = 0; a < P; a++) {
+        const float qa = f.w * wx[a];
 #pragma unroll
-      for (int bb = 0; bb < P; bb++) {
-        const float qw = qa * wy[bb];
-        atomicAdd(base + ((long)a * HY + bb) * nz,
-                  (unsigned long long)__float2ll_rn(qw * wc * FIX_SCALE));
+        for (int bb = 0; bb < P; bb++)
+          atomicAdd(base + (a * HY + bb) * nz, to_fix(qa * wy[bb] * wc));
+      }
+    } else {
+      for (int a = 0; a < P; a++) {
+        float wa = wx[0];
+#pragma unroll
+        for (int k = 1; k < P; k++) wa = a == k ? wx[k] : wa;
+#pragma unroll
+        for (int bb = 0; bb < P; bb++)
+          atomicAdd(base + (a * HY + bb) * nz, to_fix<true>(f.w * wa * wy[bb] * wc));
       }
     }
   }
@@ -346,61 +468,55 @@ __device__ __forceinline__ void load_freq(short *f, const float2 *tw, int n) {
     f[t] = (short)__float_as_int(tw[3 * FFT_MAXN + t].y);
 }
 
-constexpr int HALO_T = 16;   // threads per halo line
+// Mesh line `line` (column xi = line / ny, yi = line % ny) of a P3M system is
+// the sum of the spreading blocks' halo columns that cover it: halo column
+// (dx, dy) of block (bi, bj) is mesh column (bi bx + istart + dx,
+// bj by + istart + dy) mod n, so the covering blocks have
+// dx = xi - istart (mod bx), dy likewise.  The block's threads first list the
+// covering columns of its lines, one (line, column) each, and then sum them,
+// one point each with four loads in flight: integer sums, then the
+// conversion a single accumulator would make.  (Sixteen threads per line that
+// each worked out the line's columns took 35 us for 32 meshes of 30^3 and
+// 36^3 at order 6, and take 15 this way)
+constexpr int HALO_MAXCOV = (MAXORDER + 1) * (MAXORDER + 1);   // blocks of one column each
+struct HaloLists {
+  int off[2 * FZ_LINES][HALO_MAXCOV], n[2 * FZ_LINES];
+};
 
-// The z line `line` (mesh column xi = line / ny, yi = line % ny) of a P3M
-// system as the sum of the spreading blocks' halo columns that cover it:
-// halo column (dx, dy) of block (bi, bj) is mesh column
-// (bi bx + istart + dx, bj by + istart + dy) mod n, so the covering blocks
-// have dx = xi - istart (mod bx), dy likewise; up to 4 x 4 of them are
-// read at once (all loads in flight), more in further rounds.  Integer
-// sums, then the conversion a single accumulator would make, into every
-// other float of xl (one component of a packed line).
-__device__ __forceinline__ void halo_line(const SysParams &P,
-                                          const unsigned long long *__restrict__ halo, int line,
-                                          int tid, float *xl) {
-  const int nx = P.nx, ny = P.ny, nz = P.nz;
-  const int xi = line / ny, yi = line % ny;
-  const int istart = -((P.order + 1) / 2 - 1);
-  const int bxs = P.bx, bys = P.by, HX = bxs + P.order - 1, HY = bys + P.order - 1;
+__device__ __forceinline__ void halo_lines(const SysParams &P, const unsigned long long *__restrict__ halo,
+                                           int l0, int nl, int ls, float *fb, HaloLists &L) {
+  const int nz = P.nz, ny = P.ny, bxs = P.bx, bys = P.by;
+  const int istart = -((P.order + 1) / 2 - 1), HX = bxs + P.order - 1, HY = bys + P.order - 1;
   const int hpts = HX * HY * nz;
-  const unsigned long long *h = halo + P.halo0;
-  constexpr int NK = FFT_MAXN / HALO_T;
-  unsigned long long acc[NK];
-#pragma unroll
-  for (int k = 0; k < NK; k++) acc[k] = 0ull;
-  const int dx0 = mod_nonneg(xi - istart, bxs), dy0 = mod_nonneg(yi - istart, bys);
-  for (int dxb = dx0; dxb < HX; dxb += 4 * bxs)
-    for (int dyb = dy0; dyb < HY; dyb += 4 * bys) {
-      int off[16];
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int dx = dxb + i * bxs;
-        const int bi = mod_nonneg(xi - istart - dx, nx) / bxs;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          const int dy = dyb + j * bys;
-          const int bj = mod_nonneg(yi - istart - dy, ny) / bys;
-          off[4 * i + j] =
-              (dx < HX && dy < HY) ? (bi * P.nby + bj) * hpts + (dx * HY + dy) * nz : -1;
-        }
-      }
-#pragma unroll
-      for (int k = 0; k < NK; k++) {
-        const int t = tid + k * HALO_T;
-        if (t < nz) {
-          unsigned long long v = 0ull;
-#pragma unroll
-          for (int m = 0; m < 16; m++)
-            if (off[m] >= 0) v += h[off[m] + t];
-          acc[k] += v;
-        }
-      }
+  const int mx = (HX + bxs - 1) / bxs, my = (HY + bys - 1) / bys;   // most per axis
+  for (int t = threadIdx.x; t < 2 * FZ_LINES * mx * my; t += FZ_TB) {
+    const int l = t / (mx * my), e = t - l * mx * my, i = e / my, j = e - i * my;
+    if (l >= nl) {
+      if (e == 0) L.n[l] = 0;
+      continue;
     }
+    const int xi = (l0 + l) / ny, yi = (l0 + l) - xi * ny;
+    const int dx0 = mod_nonneg(xi - istart, bxs), dy0 = mod_nonneg(yi - istart, bys);
+    const int ni = (HX - dx0 + bxs - 1) / bxs, nj = (HY - dy0 + bys - 1) / bys;
+    if (e == 0) L.n[l] = ni * nj;
+    if (i >= ni || j >= nj) continue;
+    const int dx = dx0 + i * bxs, dy = dy0 + j * bys;
+    const int bi = mod_nonneg(xi - istart - dx, P.nx) / bxs, bj = mod_nonneg(yi - istart - dy, ny) / bys;
+    L.off[l][i * nj + j] = (bi * P.nby + bj) * hpts + (dx * HY + dy) * nz;
+  }
+  __syncthreads();
+  const unsigned long long *h = halo + P.halo0;
+  const float inv = 1.f / (float)nz;
+  for (int t = threadIdx.x; t < 2 * FZ_LINES * nz; t += FZ_TB) {
+    const int l = div_small(t, inv), z = t - l * nz, n = L.n[l];
+    unsigned long long sum = 0ull;
+    for (int e = 0; e < n; e += 4) {
+      unsigned long long v[4];
 #pragma unroll
-  for (int k = 0; k < NK; k++) {
-    const int t = tid + k * HALO_T;
-    if (t < nz) xl[2 * t] = (float)((double)(long long)acc[k] * FIX_INV);
+      for (int k = 0; k < 4; k++) v[k] = e + k < n ? h[L.off[l][e + k] + z] : 0ull;
+      sum += (v[0] + v[1]) + (v[2] + v[3]);
+    }
+    fb[2 * ((l >> 1) * ls + z) + (l & 1)] = (float)((double)(long long)sum * FIX_INV);
   }
 }
 
@@ -409,7 +525,7 @@ __device__ __forceinline__ void halo_line(const SysParams &P,
 // as a_k = (Z_k + conj Z_-k) / 2, b_k = (Z_k - conj Z_-k) / 2i, so a block of
 // two waves takes 32 lines with one butterfly per thread and stage.
 // HALO: a line is the sum of the spreading blocks' halo columns that cover it
-// (halo_line) instead of the real mesh.  What bounds it is the launch and one
+// (halo_lines) instead of the real mesh.  What bounds it is the launch and one
 // trip to memory: 5.7 us at 48^3, 6.7 at 64^3, and the inverse 5.9 and 7
 // (5.65 and 6 with one line per transform, 16 lines a block).
 template <bool HALO>
@@ -428,12 +544,8 @@ __global__ void __launch_bounds__(FZ_TB) k_fft_z(
   load_pos(pos, twid_all + P.twid0 + 2 * FFT_MAXN, nz);
   float *fb = reinterpret_cast<float *>(buf);
   if constexpr (HALO) {
-    for (int l = threadIdx.x / HALO_T; l < 2 * FZ_LINES; l += FZ_TB / HALO_T) {
-      float *xl = fb + 2 * (l >> 1) * ls + (l & 1);
-      if (l < nl) halo_line(P, halo, l0 + l, threadIdx.x % HALO_T, xl);
-      else
-        for (int z = threadIdx.x % HALO_T; z < nz; z += HALO_T) xl[2 * z] = 0.f;
-    }
+    __shared__ HaloLists lists;
+    halo_lines(P, halo, l0, nl, ls, fb, lists);
   } else {
     const float *src = mesh + P.mesh0 + (long)l0 * nz;
     const float inv = 1.f / (float)nz;
@@ -751,7 +863,7 @@ int p3m_energy_blocks(const SysParams &P) {
 // interpolated from their four meshes with the assignment weights
 // (pppm.c:618-626), E already Cartesian
 template <int P, bool IK = false>
-__global__ void __launch_bounds__(256) k_p3m_gather(const SysParams *__restrict__ sp,
+__global__ void __launch_bounds__(256, 4) k_p3m_gather(const SysParams *__restrict__ sp,
                                                     const int4 *__restrict__ sgrid,
                                                     const float4 *__restrict__ sfrac,
                                                     const float *__restrict__ mesh,
@@ -915,19 +1027,24 @@ int launch_p3m(Engine &e, int want_virial, hipStream_t st, int energies) {
       used[p.order] = true;
       (p.ik ? used_ik : used_ad)[p.order] = true;
     }
-  // LDS of the spreading: the largest halo of the systems of each order
+  // LDS of the spreading: the largest halo, or block, of the systems of each order
   size_t hbytes[MAXORDER + 1] = {0};
+  const int h = e.spread_halo ? 1 : 0;
+  int htb = 256;   // by owner: a second round of work items costs more than idle threads
   for (auto &p : e.hsp)
     if (p.kmode == 1)
-      hbytes[p.order] = std::max(hbytes[p.order], sizeof(unsigned long long) *
-                                                      (p.bx + p.order - 1) * (p.by + p.order - 1) * p.nz);
+      hbytes[p.order] = std::max(hbytes[p.order], sizeof(unsigned long long) * p.nz *
+                                                      (p.bx + h * (p.order - 1)) *
+                                                      (p.by + h * (p.order - 1)));
+  for (auto &p : e.hsp)
+    if (p.kmode == 1 && (long)p.nsite * p.order > 384L * p.nbx * p.nby) htb = 512;
 #define SPREAD(PO)                                                                           \
   if (used[PO] && e.spread_halo)                                                             \
-    hipLaunchKernelGGL(k_p3m_spread_halo<PO>, dim3(maxbins, e.nsys), dim3(256), hbytes[PO],   \
+    hipLaunchKernelGGL(k_p3m_spread_halo<PO>, dim3(maxbins, e.nsys), dim3(htb), hbytes[PO],   \
                        st, e.d_sp, e.d_bin_fill, e.bcap, e.d_bgrid, e.d_bfrac, e.d_halo);     \
   else if (used[PO])                                                                         \
-    hipLaunchKernelGGL(k_p3m_spread<PO>, dim3(maxbins, e.nsys), dim3(256), 0, st, e.d_sp,    \
-                       e.d_bin_fill, e.bcap, e.d_bgrid, e.d_bfrac, e.d_mesh);
+    hipLaunchKernelGGL(k_p3m_spread<PO>, dim3(maxbins, e.nsys), dim3(256), hbytes[PO], st,    \
+                       e.d_sp, e.d_bin_fill, e.bcap, e.d_bgrid, e.d_bfrac, e.d_mesh);
   SPREAD(1) SPREAD(2) SPREAD(3) SPREAD(4) SPREAD(5) SPREAD(6) SPREAD(7)
 #undef SPREAD
   launch_fft(e, want_virial, energies, st, e.d_sp, e.hsp.data(), e.nsys,
@@ -961,9 +1078,10 @@ int launch_p3m_adjoint(Engine &e, int sys, const float4 *src, hipStream_t st) {
                      e.d_sfrac, e.d_bin_fill, e.bcap, e.d_bgrid, e.d_bfrac, e.d_err,
                      e.d_bin_fill + e.nbin_total);
   const dim3 gb(P.nbx * P.nby, 1);
+  const size_t blds = sizeof(unsigned long long) * P.bx * P.by * P.nz;
 #define ADJ_ORDER(PO)                                                                        \
   case PO:                                                                                   \
-    hipLaunchKernelGGL((k_p3m_spread<PO, true>), gb, dim3(256), 0, st, sp, e.d_bin_fill,     \
+    hipLaunchKernelGGL(k_p3m_spread_adj<PO>, gb, dim3(256), blds, st, sp, e.d_bin_fill,      \
                        e.bcap, e.d_bgrid, e.d_bfrac, e.d_mesh, src);                         \
     break;
   switch (P.order) {
@@ -1003,10 +1121,11 @@ int launch_p3m_ik_pass(Engine &e, int sys, const double *q, hipStream_t st) {
                      e.d_sfrac, e.d_bin_fill, e.bcap, e.d_bgrid, e.d_bfrac, e.d_err,
                      e.d_bin_fill + e.nbin_total);
   const dim3 gb(P.nbx * P.nby, 1);
+  const size_t blds = sizeof(unsigned long long) * P.bx * P.by * P.nz;
 #define IK_SPREAD(PO)                                                                        \
   case PO:                                                                                   \
-    hipLaunchKernelGGL((k_p3m_spread<PO, false>), gb, dim3(256), 0, st, sp, e.d_bin_fill,    \
-                       e.bcap, e.d_bgrid, e.d_bfrac, e.d_mesh, nullptr);                     \
+    hipLaunchKernelGGL(k_p3m_spread<PO>, gb, dim3(256), blds, st, sp, e.d_bin_fill, e.bcap,  \
+                       e.d_bgrid, e.d_bfrac, e.d_mesh);                                      \
     break;
   switch (P.order) {
     IK_SPREAD(1) IK_SPREAD(2) IK_SPREAD(3) IK_SPREAD(4) IK_SPREAD(5) IK_SPREAD(6) IK_SPREAD(7)
