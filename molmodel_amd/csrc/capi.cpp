@@ -429,8 +429,14 @@ static int enqueue_forces(mm_engine *m, int field_mode, int want_virial,
     TRY(launch_nl_build(e, 1));
     e.first_eval = 0;
   } else {
-    if (m->pos_dirty) TRY(launch_skin(e));
-    TRY(launch_nl_build(e, 0, nl_from_partials));
+    // new positions are packed together with their skin test; a rebuild packs
+    // again in its new order
+    if (m->pos_dirty) {
+      TRY(launch_skin_pack(e));
+      e.need_pack = 0;
+    }
+    TRY(launch_nl_build(e, 0, nl_from_partials || m->pos_dirty));
+    m->pos_dirty = 0;
   }
   if (e.need_pack || m->pos_dirty) TRY(launch_pack(e));
   e.need_pack = 0;
@@ -654,8 +660,8 @@ int mm_nlist_update(mm_nlist *nl, const double *r) {
       e.first_eval = 0;
     } else {
       TRY(launch_set_rebuild(e, 0));   // the skin test alone decides
-      TRY(launch_skin(e));
-      TRY(launch_nl_build(e, 0));
+      TRY(launch_skin_pack(e));
+      TRY(launch_nl_build(e, 0, 1));
     }
     m->pos_dirty = 0;
     int f = 0;

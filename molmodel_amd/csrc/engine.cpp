@@ -712,7 +712,9 @@ int engine_create(Engine &e, const std::vector<SystemInput> &in) {
   MM_TRY(dalloc(&e.d_gcell, G));
   MM_TRY(dalloc(&e.d_cell_count, e.ncell_total + 1));
   MM_TRY(dalloc(&e.d_cell_start, e.ncell_total + 1));
-  MM_TRY(dalloc(&e.d_cell_fill, e.ncell_total + 1));
+  MM_TRY(dalloc(&e.d_cell_head, e.ncell_total));
+  MM_HIP(hipMemset(e.d_cell_head, 0xff, sizeof(int) * e.ncell_total));   // -1: empty
+  MM_TRY(dalloc(&e.d_gnext, G));
   {
     std::vector<int> rank_all, unrank_all, rk, ur;
     for (auto &P : e.hsp) {
@@ -733,6 +735,7 @@ int engine_create(Engine &e, const std::vector<SystemInput> &in) {
     for (int g = 0; g < G; g++) inv[g] = g;
     MM_TRY(dalloc(&e.d_gslot_inv, inv.size()));
     MM_TRY(dput(e.d_gslot_inv, inv));
+    MM_TRY(dput(e.d_order, inv));
   }
   MM_TRY(dalloc(&e.d_last, 3 * (size_t)G));
   MM_TRY(dalloc(&e.d_sten, sten.size())); MM_TRY(dput(e.d_sten, sten));
@@ -967,7 +970,7 @@ void engine_destroy(Engine &e) {
   void *ptrs[] = {e.d_sp, e.d_gfirst, e.d_gns, e.d_gsys, e.d_gexcl, e.d_ginfo, e.d_q, e.d_mass,
                   e.d_r, e.d_v, e.d_f, e.d_r0, e.d_gcell, e.d_cell_count, e.d_cell_start,
                   e.d_cell_rank, e.d_cell_unrank,
-                  e.d_cell_fill, e.d_order, e.d_gslot, e.d_gslot_inv, e.d_last, e.d_sten, e.d_nbr,
+                  e.d_cell_head, e.d_gnext, e.d_order, e.d_gslot, e.d_gslot_inv, e.d_last, e.d_sten, e.d_nbr,
                   e.d_nnb, e.d_rebuild,
                   e.d_err, e.d_gpos, e.d_spk, e.d_gmeta, e.d_pf, e.d_plj, e.d_gacc, e.d_tab,
                   e.d_ljt, e.d_kres, e.d_kvec, e.d_ksc, e.d_mesh, e.d_cmesh, e.d_green, e.d_twid,

@@ -72,7 +72,8 @@ struct Engine {
   double *d_r = nullptr, *d_v = nullptr, *d_f = nullptr, *d_r0 = nullptr;
   // neighbor list
   int ncell_total = 0;
-  int *d_gcell = nullptr, *d_cell_count = nullptr, *d_cell_start = nullptr, *d_cell_fill = nullptr;
+  int *d_gcell = nullptr, *d_cell_count = nullptr, *d_cell_start = nullptr;
+  int *d_cell_head = nullptr, *d_gnext = nullptr;   // a build's lists of each cell's groups
   // cells are stored in Hilbert-curve order: d_cell_rank maps a cell index
   // (ix*n + iy)*n + iz to its storage position, d_cell_unrank back (both per
   // system, relative to SysParams::cell0); groups sorted by stored cell are
@@ -127,7 +128,7 @@ struct Engine {
   double *d_fpart = nullptr;  // per-block partials of the finish kernel: the next
                               // step's neighbour-list check reads them while the
                               // reciprocal-space kernels write d_part
-  int *d_done = nullptr;      // per-system block counters
+  int *d_done = nullptr;      // block counters: per system of the finish, mesh energy, exchange, cells
   // pair-kernel work: tiles of 16 i-groups numbered over all systems
   int bcap = 0;               // slots per P3M column bin (bgrid/bfrac hold nbin_total * bcap)
   int any_water = 0;          // some system holds only three-site waters (SysParams::water)
@@ -275,7 +276,7 @@ int launch_adj_p3m_ik(Engine &e, int sys, const double *R, double scale, double 
                       double *psi);
 int launch_finish_ex(Engine &e, int mode, int want_virial, double *phi_out);
 int launch_field_out(Engine &e, double *out, double *ulj, int min_image = 1);
-int launch_skin(Engine &e);
+int launch_skin_pack(Engine &e);
 int launch_count_pairs(Engine &e, unsigned long long *d_out);
 int launch_remd_exchange(Engine &e, long long attempt);
 int launch_phi_points(Engine &e, const double4 *sites, int nsite, const double *pts, int npts,

@@ -16,6 +16,7 @@
 #include "engine.hpp"
 #include "scan.hpp"
 #include "reduce.hpp"
+#include "pack.hpp"
 
 #pragma clang fp contract(off)
 
@@ -31,131 +32,303 @@ __device__ __forceinline__ double min_image_sq(double ax, double ay, double az, 
   return x * x + y * y + z * z;
 }
 
-// from_part: the skin test (nbrlist.cpp:64-76) on the largest and second
-// largest first-site displacement since the last build, merged from the
-// per-block partials of the finish kernel that moved the positions (every
-// block forms the same values); a rebuild already requested stays
-// requested, and block 0 records the outcome for the rest of the chain.
+// The skin test (nbrlist.cpp:64-76) on the largest and second largest
+// first-site displacement since the last build, merged from per-block
+// partials in the finish kernel's layout (FIN_TB groups a block).  Every
+// thread of the block calls it and gets the outcome.
+__device__ __forceinline__ bool skin_fires(const SysParams &P, int s, const double *__restrict__ part,
+                                           int maxblk) {
+  __shared__ double w1[16], w2[16];
+  __shared__ int fire;
+  const int nb = (P.ngroup + FIN_TB - 1) / FIN_TB;
+  double t1 = 0, t2 = 0;
+  for (int b = threadIdx.x; b < nb; b += blockDim.x) {
+    const double *q = part + ((long)s * maxblk + b) * FIN_NPART + FIN_TOP;
+    top2_merge(t1, t2, load_coherent(q), load_coherent(q + 1));
+  }
+  for (int o = 32; o >= 1; o >>= 1) {
+    const double b1 = __shfl_xor(t1, o), b2 = __shfl_xor(t2, o);
+    top2_merge(t1, t2, b1, b2);
+  }
+  if ((threadIdx.x & 63) == 0) { w1[threadIdx.x >> 6] = t1; w2[threadIdx.x >> 6] = t2; }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double u1 = w1[0], u2 = w2[0];
+    for (int k = 1; k < (int)(blockDim.x >> 6); k++) top2_merge(u1, u2, w1[k], w2[k]);
+    fire = u1 + u2 > P.skin;   // nbrlist.cpp:75-76
+  }
+  __syncthreads();
+  return fire;
+}
+
+// the stored cell of a first site at (x, y, z), -1 for a position that is not
+// finite or so far out that a cell index would leave int range (an error)
+__device__ __forceinline__ int stored_cell(const SysParams &P, double x, double y, double z,
+                                           const int *__restrict__ cell_rank) {
+#pragma clang fp contract(off)
+  const double lim = 1e9 * P.lc;
+  if (!(fabs(x) <= lim && fabs(y) <= lim && fabs(z) <= lim)) return -1;
+  const int n = P.ncell;
+  const int ix = (int)floor(x / P.lc + 0.5);
+  const int iy = (int)floor(y / P.lc + 0.5);
+  const int iz = (int)floor(z / P.lc + 0.5);
+  // stored at the cell's position along the Hilbert curve
+  return cell_rank[P.cell0 + (mod_nonneg(ix, n) * n + mod_nonneg(iy, n)) * n + mod_nonneg(iz, n)];
+}
+
+// groups one cell may hold: far above any physical density (cells hold
+// about two groups on average), low enough that the serial sort stays short
+constexpr int NL_SORT_MAX = 512;
+constexpr int NL_CELL_REGS = 8;   // cells up to this size are sorted in registers
+
+// A cell's n groups (v: the first NL_CELL_REGS of them; all of them already in
+// order[b ..] if there are more) into ascending group order at order[b ..],
+// so that the sorted order is deterministic, and their first-site positions
+// into the pair kernel's gpos.
+__device__ __forceinline__ void place_cell(int b, int n, int *v, int *__restrict__ order,
+                                           const double *__restrict__ last,
+                                           double4 *__restrict__ gpos) {
+  if (n <= NL_CELL_REGS) {
+#pragma unroll
+    for (int k = 0; k < NL_CELL_REGS; k++) v[k] = k < n ? v[k] : 0x7fffffff;
+#pragma unroll
+    for (int p = 0; p < NL_CELL_REGS; p++)   // odd-even transpositions
+#pragma unroll
+      for (int k = p & 1; k + 1 < NL_CELL_REGS; k += 2) {
+        const int lo = min(v[k], v[k + 1]);
+        v[k + 1] = max(v[k], v[k + 1]);
+        v[k] = lo;
+      }
+    double4 p[NL_CELL_REGS];
+#pragma unroll
+    for (int k = 0; k < NL_CELL_REGS; k++)
+      if (k < n) p[k] = make_double4(last[3 * v[k]], last[3 * v[k] + 1], last[3 * v[k] + 2], 0.0);
+#pragma unroll
+    for (int k = 0; k < NL_CELL_REGS; k++)
+      if (k < n) {
+        order[b + k] = v[k];
+        gpos[b + k] = p[k];
+      }
+    return;
+  }
+  for (int i = b + 1; i < b + n; i++) {
+    const int x = order[i];
+    int j = i - 1;
+    while (j >= b && order[j] > x) { order[j + 1] = order[j]; j--; }
+    order[j + 1] = x;
+  }
+  for (int i = b; i < b + n; i++) {
+    const int g = order[i];
+    gpos[i] = make_double4(last[3 * g], last[3 * g + 1], last[3 * g + 2], 0.0);
+  }
+}
+
+// Skin test, cells, counts and the cells' lists of groups (head, next); the
+// last block to finish scans the counts into sorted group offsets.  Only a
+// step that rebuilds pays for the fence and the counter.
+// from_part: the skin test on the partials of the kernel that moved the
+// positions; every block forms the same outcome, a rebuild already requested
+// stays requested, and block 0 records it for the rest of the chain.
 __global__ void __launch_bounds__(256) k_nl_assign(
     const SysParams *__restrict__ sp, const int *__restrict__ gfirst,
     const double *__restrict__ r, int nsite_total, int *__restrict__ rebuild,
     int *__restrict__ gcell, double *__restrict__ last, int *__restrict__ cell_count,
-    unsigned long long *__restrict__ builds, int *__restrict__ err,
+    int *__restrict__ cell_start, int *__restrict__ head, int *__restrict__ next,
+    int *__restrict__ done, unsigned long long *__restrict__ builds, int *__restrict__ err,
     const double *__restrict__ part, int maxblk, int from_part, const int *__restrict__ cell_rank) {
-#pragma clang fp contract(off)
+  __shared__ int lastblk;
   const int s = blockIdx.y;
   const SysParams &P = sp[s];
+  const int nblk = (P.ngroup + 255) / 256;
+  if ((int)blockIdx.x >= nblk) return;
   int want = rebuild[s];
   if (from_part) {
-    __shared__ double w1[4], w2[4];
-    __shared__ int fire;
-    const int nb = (P.ngroup + FIN_TB - 1) / FIN_TB;
-    double t1 = 0, t2 = 0;
-    for (int b = threadIdx.x; b < nb; b += blockDim.x) {
-      const double *q = part + ((long)s * maxblk + b) * FIN_NPART + FIN_TOP;
-      top2_merge(t1, t2, load_coherent(q), load_coherent(q + 1));
-    }
-    for (int o = 32; o >= 1; o >>= 1) {
-      const double b1 = __shfl_xor(t1, o), b2 = __shfl_xor(t2, o);
-      top2_merge(t1, t2, b1, b2);
-    }
-    if ((threadIdx.x & 63) == 0) { w1[threadIdx.x >> 6] = t1; w2[threadIdx.x >> 6] = t2; }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      double u1 = w1[0], u2 = w2[0];
-      for (int k = 1; k < (int)(blockDim.x >> 6); k++) top2_merge(u1, u2, w1[k], w2[k]);
-      fire = u1 + u2 > P.skin;   // nbrlist.cpp:75-76
-    }
-    __syncthreads();
+    const bool fire = skin_fires(P, s, part, maxblk);
     want |= fire;
     if (blockIdx.x == 0 && threadIdx.x == 0 && fire) rebuild[s] = 1;
   }
   if (!want) return;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i == 0) builds[s] += 1;
-  if (i >= P.ngroup) return;
-  const int g = P.group0 + i;
-  const int site = gfirst[g];
-  const double x = r[site], y = r[nsite_total + site], z = r[2 * nsite_total + site];
-  const int n = P.ncell;
-  int c = P.cell0;
-  // cell indices stay far inside int range; a position beyond (or NaN) is
-  // an error
-  const double lim = 1e9 * P.lc;
-  if (fabs(x) <= lim && fabs(y) <= lim && fabs(z) <= lim) {
-    const int ix = (int)floor(x / P.lc + 0.5);
-    const int iy = (int)floor(y / P.lc + 0.5);
-    const int iz = (int)floor(z / P.lc + 0.5);
-    // stored at the cell's position along the Hilbert curve
-    c += cell_rank[P.cell0 + (mod_nonneg(ix, n) * n + mod_nonneg(iy, n)) * n + mod_nonneg(iz, n)];
-  } else {
-    atomicOr(err, ERR_NAN);   // reported; the group is parked in cell 0
+  if (i < P.ngroup) {
+    const int g = P.group0 + i;
+    const int site = gfirst[g];
+    const double x = r[site], y = r[nsite_total + site], z = r[2 * nsite_total + site];
+    int c = stored_cell(P, x, y, z, cell_rank);
+    if (c < 0) {
+      atomicOr(err, ERR_NAN);   // reported; the group is parked in cell 0
+      c = 0;
+    }
+    c += P.cell0;
+    gcell[g] = c;
+    last[3 * g] = x;
+    last[3 * g + 1] = y;
+    last[3 * g + 2] = z;
+    next[g] = atomicExch(&head[c], g);
+    atomicAdd(&cell_count[c], 1);
   }
-  gcell[g] = c;
-  last[3 * g] = x;
-  last[3 * g + 1] = y;
-  last[3 * g + 2] = z;
-  atomicAdd(&cell_count[c], 1);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    __threadfence();
+    lastblk = atomicAdd(&done[s], 1) == nblk - 1;
+  }
+  __syncthreads();
+  if (!lastblk) return;
+  __threadfence();
+  if (threadIdx.x == 0) done[s] = 0;
+  block_scan_clear(cell_count + P.cell0, cell_start + P.cell0, P.ncell * P.ncell * P.ncell, P.group0);
 }
 
-// one block per system: exclusive scan of that system's cells into sorted
-// group offsets; counts and fill cursors are cleared for the next build
-__global__ void k_nl_scan(const SysParams *__restrict__ sp, const int *__restrict__ rebuild,
-                          int *__restrict__ cell_count, int *__restrict__ cell_start,
-                          int *__restrict__ cell_fill) {
+// The groups of each cell from its list, in ascending order, one thread per
+// cell; the lists are cleared for the next build.  After a non-finite
+// position (its group parked in cell 0) or in a collapsed cell the list is
+// not walked: the rows of an error are discarded, and the slots keep the
+// order of the last build.
+__global__ void k_nl_order(const SysParams *__restrict__ sp, const int *__restrict__ rebuild,
+                           const int *__restrict__ cell_start, int *__restrict__ head,
+                           const int *__restrict__ next, int *__restrict__ order,
+                           const double *__restrict__ last, double4 *__restrict__ gpos,
+                           int *__restrict__ err) {
   const int s = blockIdx.y;
   if (!rebuild[s]) return;
-  const SysParams &P = sp[s];
-  block_scan_clear(cell_count + P.cell0, cell_start + P.cell0, cell_fill + P.cell0,
-                   P.ncell * P.ncell * P.ncell, P.group0);
-}
-
-__global__ void k_nl_scatter(const SysParams *__restrict__ sp, const int *__restrict__ rebuild,
-                             const int *__restrict__ gcell, const int *__restrict__ cell_start,
-                             int *__restrict__ cell_fill, int *__restrict__ order) {
-  const int s = blockIdx.y;
-  if (!rebuild[s]) return;
-  const SysParams &P = sp[s];
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= P.ngroup) return;
-  const int g = P.group0 + i;
-  const int c = gcell[g];
-  order[cell_start[c] + atomicAdd(&cell_fill[c], 1)] = g;
-}
-
-// groups one cell may hold: far above any physical density (cells hold
-// about two groups on average), low enough that the serial sort stays short
-constexpr int NL_SORT_MAX = 512;
-
-// ascending group id within each cell, so the sorted order is deterministic;
-// then the first-site positions in sorted order (the pair kernel's gpos)
-__global__ void k_nl_sortcell(const SysParams *__restrict__ sp, const int *__restrict__ rebuild,
-                              const int *__restrict__ cell_start, int *__restrict__ order,
-                              const double *__restrict__ last, double4 *__restrict__ gpos,
-                              int *__restrict__ err) {
-  const int s = blockIdx.y;
-  if (!rebuild[s]) return;
-  // after a non-finite position (its group parked in cell 0) skip the sort,
-  // whose serial cost grows with the square of a cell's population; the
-  // rows built from the unsorted order are discarded with the error
-  if (__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & ERR_NAN) return;
   const SysParams &P = sp[s];
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= P.ncell * P.ncell * P.ncell) return;
-  const int b = cell_start[P.cell0 + c], e = cell_start[P.cell0 + c + 1];
-  if (e - b > NL_SORT_MAX) {   // collapsed positions: reported, not sorted
+  int g = head[P.cell0 + c];
+  head[P.cell0 + c] = -1;
+  if (__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & ERR_NAN) return;
+  const int b = cell_start[P.cell0 + c], n = cell_start[P.cell0 + c + 1] - b;
+  if (n > NL_SORT_MAX) {   // collapsed positions: reported, not sorted
     atomicOr(err, ERR_CELL);
     return;
   }
-  for (int i = b + 1; i < e; i++) {
-    const int v = order[i];
-    int j = i - 1;
-    while (j >= b && order[j] > v) { order[j + 1] = order[j]; j--; }
-    order[j + 1] = v;
+  int v[NL_CELL_REGS];
+  if (n <= NL_CELL_REGS) {
+#pragma unroll
+    for (int k = 0; k < NL_CELL_REGS; k++) {
+      if (k >= n) break;
+      v[k] = g;
+      g = next[g];
+    }
+  } else {
+    for (int k = 0; k < n; k++, g = next[g]) order[b + k] = g;
   }
-  for (int i = b; i < e; i++) {
-    const int g = order[i];
-    gpos[i] = make_double4(last[3 * g], last[3 * g + 1], last[3 * g + 2], 0.0);
+  place_cell(b, n, v, order, last, gpos);
+}
+
+// The same for one system in one block, with the cells' counts in LDS: one
+// launch less, which a step that does not rebuild saves about 2.5 us by.  A
+// rebuild takes one block 27 us for 4 096 groups (20 in the two kernels
+// above) and 200 for 32 768 (45), so with a rebuild every 25 to 30 steps the
+// line lies near 8 000 groups.
+constexpr int NL_BIN_TB = 1024;
+constexpr int NL_BIN_CELLS = 12000;    // 47 KB of counts
+constexpr int NL_BIN_GROUPS = 8192;
+
+__global__ void __launch_bounds__(NL_BIN_TB) k_nl_bin(
+    const SysParams *__restrict__ sp, const int *__restrict__ gfirst,
+    const double *__restrict__ r, int N, int *__restrict__ rebuild, int *__restrict__ gcell,
+    double *__restrict__ last, int *__restrict__ cell_start, int *__restrict__ order,
+    double4 *__restrict__ gpos, unsigned long long *__restrict__ builds, int *__restrict__ err,
+    const double *__restrict__ part, int maxblk, int from_part, const int *__restrict__ cell_rank) {
+  extern __shared__ int cnt[];
+  __shared__ int wsum[NL_BIN_TB / 64], bad;
+  const int s = blockIdx.x, tid = threadIdx.x;
+  const SysParams &P = sp[s];
+  int want = rebuild[s];
+  if (from_part && skin_fires(P, s, part, maxblk)) {
+    if (tid == 0) rebuild[s] = 1;
+    want = 1;
+  }
+  if (!want) return;
+  const int nc = P.ncell * P.ncell * P.ncell, G = P.ngroup;
+  if (tid == 0) {
+    builds[s] += 1;
+    // another system's error leaves this one's rows empty too (k_nl_pairs)
+    bad = (__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & ERR_NAN) != 0;
+  }
+  for (int c = tid; c < nc; c += NL_BIN_TB) cnt[c] = 0;
+  __syncthreads();
+  constexpr int U = 4;   // groups in flight per thread
+  for (int i0 = tid; i0 < G; i0 += U * NL_BIN_TB) {
+    int site[U];
+    double x[U][3];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int i = i0 + u * NL_BIN_TB;
+      site[u] = gfirst[P.group0 + (i < G ? i : 0)];
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int d = 0; d < 3; d++) x[u][d] = r[(long)d * N + site[u]];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int i = i0 + u * NL_BIN_TB, g = P.group0 + i;
+      if (i >= G) break;
+      int c = stored_cell(P, x[u][0], x[u][1], x[u][2], cell_rank);
+      if (c < 0) {
+        atomicOr(err, ERR_NAN);   // reported; the group is parked in cell 0
+        bad = 1;
+        c = 0;
+      }
+      gcell[g] = P.cell0 + c;
+      last[3 * g] = x[u][0];
+      last[3 * g + 1] = x[u][1];
+      last[3 * g + 2] = x[u][2];
+      atomicAdd(&cnt[c], 1);
+    }
+  }
+  __syncthreads();
+  // exclusive scan: each thread its own run of cells, then over the block
+  const int per = (nc + NL_BIN_TB - 1) / NL_BIN_TB, c0 = min(tid * per, nc), c1 = min(c0 + per, nc);
+  int sum = 0;
+  for (int c = c0; c < c1; c++) sum += cnt[c];
+  int incl = sum;
+  const int lane = tid & 63, wid = tid >> 6;
+  for (int o = 1; o < 64; o <<= 1) {
+    const int v = __shfl_up(incl, o);
+    if (lane >= o) incl += v;
+  }
+  if (lane == 63) wsum[wid] = incl;
+  __syncthreads();
+  int at = P.group0 + incl - sum;
+  for (int w = 0; w < wid; w++) at += wsum[w];
+  for (int c = c0; c < c1; c++) {
+    const int n = cnt[c];
+    cell_start[P.cell0 + c] = at;
+    cnt[c] = at;   // the next free slot of the cell
+    at += n;
+  }
+  if (tid == 0) cell_start[P.cell0 + nc] = P.group0 + G;
+  __syncthreads();
+  for (int i0 = tid; i0 < G; i0 += U * NL_BIN_TB) {
+    int c[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int i = i0 + u * NL_BIN_TB;
+      c[u] = i < G ? gcell[P.group0 + i] - P.cell0 : 0;
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int i = i0 + u * NL_BIN_TB;
+      if (i < G) order[atomicAdd(&cnt[c[u]], 1)] = P.group0 + i;
+    }
+  }
+  __syncthreads();
+  if (bad) return;   // the rows of an error are discarded, so skip the sort
+  for (int c = tid; c < nc; c += NL_BIN_TB) {
+    // cnt[c] is now the end of cell c and the start of cell c + 1
+    const int b = c ? cnt[c - 1] : P.group0, n = cnt[c] - b;
+    if (n > NL_SORT_MAX) {   // collapsed positions: reported, not sorted
+      atomicOr(err, ERR_CELL);
+      continue;
+    }
+    int v[NL_CELL_REGS];
+#pragma unroll
+    for (int k = 0; k < NL_CELL_REGS; k++)
+      if (k < n) v[k] = order[b + k];
+    place_cell(b, n, v, order, last, gpos);
   }
 }
 
@@ -331,42 +504,44 @@ __global__ void k_set_flags(int *f, int n, int v) {
   if (i < n) f[i] = v;
 }
 
-// skin test for externally supplied positions (nbrlist.cpp:64-76): one
-// block per system; a rebuild already requested stays requested
-__global__ void k_skin(const SysParams *__restrict__ sp, const int *__restrict__ gfirst,
-                       const double *__restrict__ r, int N, const double *__restrict__ last,
-                       int *__restrict__ rebuild) {
+// Externally supplied positions: the pair kernel's packed inputs in the
+// present sorted order (as k_pack) and the displacements since the last build
+// (nbrlist.cpp:64-76) as per-block partials that the build check merges.  One
+// block per FIN_TB groups; a block per system alone took 35 us for 32 768
+// groups, and the packing was a kernel of its own (6.5 us): 6.3 us for both
+__global__ void __launch_bounds__(FIN_TB) k_skin_pack(
+    const SysParams *__restrict__ sp, const int *__restrict__ order, const int *__restrict__ gfirst,
+    const int *__restrict__ gns, const int *__restrict__ ginfo, const double *__restrict__ r,
+    const double *__restrict__ q, int N, const double *__restrict__ last,
+    double4 *__restrict__ gpos, float4 *__restrict__ spk, int2 *__restrict__ gmeta,
+    double *__restrict__ part, int maxblk) {
+  __shared__ double red[FIN_TB / 64][2];
   const int s = blockIdx.y;
   const SysParams &P = sp[s];
-  double t1 = 0, t2 = 0;
-  for (int i = threadIdx.x; i < P.ngroup; i += blockDim.x) {
-    const int g = P.group0 + i, st = gfirst[g];
-    const double dx = r[st] - last[3 * g], dy = r[N + st] - last[3 * g + 1],
-                 dz = r[2 * N + st] - last[3 * g + 2];
-    double d = sqrt(dx * dx + dy * dy + dz * dz);
-    if (!(d <= 1e300)) d = 1e300;   // a non-finite position (or a list built from one) rebuilds
-    if (d > t1) { t2 = t1; t1 = d; } else if (d > t2) t2 = d;
+  const int i = blockIdx.x * FIN_TB + threadIdx.x;
+  if ((int)(blockIdx.x * FIN_TB) >= P.ngroup) return;
+  double top[2] = {0, 0};
+  if (i < P.ngroup) {
+    const int gs = P.group0 + i;
+    const int g = order[gs];
+    const double4 p = pack_group(gs, gfirst[g], gns[g], ginfo[g], r, q, N, gpos, spk, gmeta);
+    const double dx = p.x - last[3 * g], dy = p.y - last[3 * g + 1], dz = p.z - last[3 * g + 2];
+    const double d = sqrt(dx * dx + dy * dy + dz * dz);
+    top[0] = d <= 1e300 ? d : 1e300;   // a non-finite position (or a list built from one) rebuilds
   }
-  __shared__ double a1[16], a2[16];
-  for (int o = 32; o >= 1; o >>= 1) {
-    const double b1 = __shfl_xor(t1, o), b2 = __shfl_xor(t2, o);
-    if (b1 > t1) { t2 = fmax(t1, b2); t1 = b1; } else if (b1 > t2) t2 = b1;
-  }
-  const int w = threadIdx.x >> 6;
-  if ((threadIdx.x & 63) == 0) { a1[w] = t1; a2[w] = t2; }
-  __syncthreads();
+  block_reduce<2, 0, FIN_TB>(top, red);
   if (threadIdx.x == 0) {
-    double u1 = 0, u2 = 0;
-    for (int k = 0; k < (int)(blockDim.x >> 6); k++) {
-      if (a1[k] > u1) { u2 = fmax(u1, a2[k]); u1 = a1[k]; } else if (a1[k] > u2) u2 = a1[k];
-    }
-    if (u1 + u2 > P.skin) rebuild[s] = 1;
+    double *o = part + ((long)s * maxblk + blockIdx.x) * FIN_NPART + FIN_TOP;
+    o[0] = top[0];
+    o[1] = top[1];
   }
 }
 
-int launch_skin(Engine &e) {
-  hipLaunchKernelGGL(k_skin, dim3(1, e.nsys), dim3(1024), 0, e.stream, e.d_sp, e.d_gfirst, e.d_r,
-                     e.nsite, e.d_last, e.d_rebuild);
+// after it, launch_nl_build takes the partials
+int launch_skin_pack(Engine &e) {
+  hipLaunchKernelGGL(k_skin_pack, dim3((e.maxg + FIN_TB - 1) / FIN_TB, e.nsys), dim3(FIN_TB), 0,
+                     e.stream, e.d_sp, e.d_order, e.d_gfirst, e.d_gns, e.d_ginfo, e.d_r, e.d_q,
+                     e.nsite, e.d_last, e.d_gpos, e.d_spk, e.d_gmeta, e.d_fpart, e.nblk_part);
   MM_HIP(hipGetLastError());
   return 0;
 }
@@ -386,18 +561,22 @@ int launch_nl_build(Engine &e, int force, int from_partials) {
   const int tb = 256;
   dim3 gg((e.maxg + tb - 1) / tb, e.nsys);
   const double *r = e.d_r;
-  hipLaunchKernelGGL(k_nl_assign, gg, dim3(tb), 0, e.stream, e.d_sp, e.d_gfirst, r, e.nsite,
-                     e.d_rebuild, e.d_gcell, e.d_last, e.d_cell_count, e.d_nlb, e.d_err,
-                     e.d_fpart, e.nblk_part, from_partials, e.d_cell_rank);
-  hipLaunchKernelGGL(k_nl_scan, dim3(1, e.nsys), dim3(1024), 0, e.stream, e.d_sp, e.d_rebuild,
-                     e.d_cell_count, e.d_cell_start, e.d_cell_fill);
-  hipLaunchKernelGGL(k_nl_scatter, gg, dim3(tb), 0, e.stream, e.d_sp, e.d_rebuild, e.d_gcell,
-                     e.d_cell_start, e.d_cell_fill, e.d_order);
   int maxc = 0;
   for (auto &p : e.hsp) maxc = std::max(maxc, p.ncell * p.ncell * p.ncell);
-  hipLaunchKernelGGL(k_nl_sortcell, dim3((maxc + tb - 1) / tb, e.nsys), dim3(tb), 0, e.stream,
-                     e.d_sp, e.d_rebuild, e.d_cell_start, e.d_order, e.d_last, e.d_gpos,
-                     e.d_err);
+  if (maxc <= NL_BIN_CELLS && e.maxg <= NL_BIN_GROUPS) {
+    hipLaunchKernelGGL(k_nl_bin, dim3(e.nsys), dim3(NL_BIN_TB), sizeof(int) * maxc, e.stream, e.d_sp,
+                       e.d_gfirst, r, e.nsite, e.d_rebuild, e.d_gcell, e.d_last, e.d_cell_start,
+                       e.d_order, e.d_gpos, e.d_nlb, e.d_err, e.d_fpart, e.nblk_part, from_partials,
+                       e.d_cell_rank);
+  } else {
+    hipLaunchKernelGGL(k_nl_assign, gg, dim3(tb), 0, e.stream, e.d_sp, e.d_gfirst, r, e.nsite,
+                       e.d_rebuild, e.d_gcell, e.d_last, e.d_cell_count, e.d_cell_start,
+                       e.d_cell_head, e.d_gnext, e.d_done + 3 * e.nsys, e.d_nlb, e.d_err, e.d_fpart,
+                       e.nblk_part, from_partials, e.d_cell_rank);
+    hipLaunchKernelGGL(k_nl_order, dim3((maxc + tb - 1) / tb, e.nsys), dim3(tb), 0, e.stream,
+                       e.d_sp, e.d_rebuild, e.d_cell_start, e.d_cell_head, e.d_gnext, e.d_order,
+                       e.d_last, e.d_gpos, e.d_err);
+  }
   hipLaunchKernelGGL(k_nl_pairs, dim3((e.maxg + 3) / 4, e.nsys), dim3(256), 0,
                      e.stream, e.d_sp, e.d_rebuild, e.d_order, e.d_gcell, e.d_cell_start,
                      e.d_sten, e.nbcap, e.d_nbr, e.d_nnb, e.d_err, e.d_r, e.nsite, e.d_q,

@@ -30,7 +30,6 @@
 // Assignment weights are the cardinal B-splines that the reference's
 // polynomial tables tabulate (pppm.c:69-275), evaluated by recursion in FP32.
 #include "engine.hpp"
-#include "scan.hpp"
 #include "reduce.hpp"
 #include "fft.hpp"
 #include <cmath>

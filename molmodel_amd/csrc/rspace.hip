@@ -19,6 +19,7 @@
 // partial sums are added into FP64 accumulators; the 16 lanes of an i-group
 // are reduced with cross-lane shuffles at the end.
 #include "engine.hpp"
+#include "pack.hpp"
 
 namespace mmamd {
 
@@ -34,20 +35,7 @@ __global__ void k_pack(const SysParams *__restrict__ sp, const int *__restrict__
   if (i >= P.ngroup) return;
   const int gs = P.group0 + i;
   const int g = order[gs];
-  const int s0 = gfirst[g], ns = gns[g];
-  const double x0 = r[s0], y0 = r[N + s0], z0 = r[2 * N + s0];
-  gpos[gs] = make_double4(x0, y0, z0, 0.0);
-#pragma unroll
-  for (int k = 0; k < MAXS; k++) {
-    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (k < ns) {
-      const int sk = s0 + k;
-      v = make_float4((float)(r[sk] - x0), (float)(r[N + sk] - y0), (float)(r[2 * N + sk] - z0),
-                      ((ginfo[g] >> (8 * k)) & SITE_HAS_Q) ? (float)q[sk] : 0.f);
-    }
-    spk[(long)gs * MAXS + k] = v;
-  }
-  gmeta[gs] = make_int2(ns, ginfo[g]);
+  pack_group(gs, gfirst[g], gns[g], ginfo[g], r, q, N, gpos, spk, gmeta);
 }
 
 __device__ __forceinline__ double shfl_xor_d(double v, int m) { return __shfl_xor(v, m, 16); }

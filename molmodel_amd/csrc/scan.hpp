@@ -1,46 +1,48 @@
-// scan.hpp -- one-block exclusive scan used by the counting sorts (cells,
-// mesh column bins): start[i] = base + sum_{j<i} count[j], start[n] = base +
-// total; count and fill are cleared for the next use.  Call with all threads
-// of a block (<= 1024 threads, multiple of 64).
+// scan.hpp -- one-block exclusive scan of the neighbour list's cell counts:
+// start[i] = base + sum_{j<i} count[j], start[n] = base + total; the counts
+// are cleared for the next use.  They may have been written by other blocks'
+// atomics, so they are read past the caches.  Call with all threads of a
+// block (<= 1024 threads, multiple of 64).
 #pragma once
 #include <hip/hip_runtime.h>
 
 namespace mmamd {
 
-__device__ inline void block_scan_clear(int *count, int *start, int *fill, int n, int base) {
+constexpr int SCAN_PER = 8;   // consecutive counts per thread and round
+
+__device__ inline void block_scan_clear(int *count, int *start, int n, int base) {
   __shared__ int wsum[16];
-  __shared__ int carry;
-  if (threadIdx.x == 0) carry = base;
-  __syncthreads();
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  for (int b = 0; b < n; b += blockDim.x) {
-    const int c = b + threadIdx.x;
-    const int v = c < n ? count[c] : 0;
-    int x = v;
+  int carry = base;
+  for (int b = 0; b < n; b += SCAN_PER * blockDim.x) {
+    const int c = b + SCAN_PER * threadIdx.x;
+    int v[SCAN_PER], sum = 0;
+#pragma unroll
+    for (int k = 0; k < SCAN_PER; k++)
+      v[k] = c + k < n ? __hip_atomic_load(count + c + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+#pragma unroll
+    for (int k = 0; k < SCAN_PER; k++) sum += v[k];
+    int x = sum;
     for (int o = 1; o < 64; o <<= 1) {
       const int y = __shfl_up(x, o, 64);
       if (lane >= o) x += y;
     }
     if (lane == 63) wsum[wid] = x;
     __syncthreads();
-    if (wid == 0) {
-      int w = lane < nw ? wsum[lane] : 0;
-      for (int o = 1; o < 16; o <<= 1) {
-        const int y = __shfl_up(w, o, 64);
-        if (lane >= o) w += y;
+    int at = carry + x - sum;
+    for (int w = 0; w < nw; w++) {
+      if (w < wid) at += wsum[w];
+      carry += wsum[w];
+    }
+#pragma unroll
+    for (int k = 0; k < SCAN_PER; k++) {
+      if (c + k < n) {
+        start[c + k] = at;
+        count[c + k] = 0;
       }
-      if (lane < nw) wsum[lane] = w;
+      at += v[k];
     }
-    __syncthreads();
-    const int excl = carry + (wid > 0 ? wsum[wid - 1] : 0) + x - v;
-    if (c < n) {
-      start[c] = excl;
-      count[c] = 0;
-      fill[c] = 0;
-    }
-    __syncthreads();
-    if (threadIdx.x == blockDim.x - 1) carry = excl + v;
-    __syncthreads();
+    __syncthreads();   // the next round writes wsum
   }
   if (threadIdx.x == 0) start[n] = carry;
 }
