@@ -778,7 +778,8 @@ int engine_create(Engine &e, const std::vector<SystemInput> &in) {
     // occupancy allows 4; the default 3 leaves one slot on every CU to the
     // reciprocal-space kernels of the other stream)
     std::vector<int> ts(e.nsys + 1, 0);
-    for (int s = 0; s < e.nsys; s++) ts[s + 1] = ts[s] + pair_tiles(e.hsp[s].ngroup);
+    e.pair_lanes = e.ngroup <= PAIR_WIDE_GROUPS ? 64 : 16;
+    for (int s = 0; s < e.nsys; s++) ts[s + 1] = ts[s] + pair_tiles(e.hsp[s].ngroup, e.pair_lanes);
     e.ntile = ts[e.nsys];
     int dev = 0, ncu = 256;
     MM_HIP(hipGetDevice(&dev));

@@ -129,10 +129,11 @@ struct Engine {
                               // step's neighbour-list check reads them while the
                               // reciprocal-space kernels write d_part
   int *d_done = nullptr;      // block counters: per system of the finish, mesh energy, exchange, cells
-  // pair-kernel work: tiles of 16 i-groups numbered over all systems
+  // pair-kernel work: tiles of 256 / pair_lanes i-groups numbered over all systems
   int bcap = 0;               // slots per P3M column bin (bgrid/bfrac hold nbin_total * bcap)
   int any_water = 0;          // some system holds only three-site waters (SysParams::water)
   int ntile = 0;
+  int pair_lanes = 16;        // pair-kernel lanes per i-group: 16 or 64
   int pair_blocks = 0;        // persistent grid (a multiple of 8)
   // shape (mm_shape): mean groups per neighbour-list cell (2: the
   // reference's cell count), pair workgroups per CU, spreading column-block
@@ -235,7 +236,10 @@ int engine_grow_bins(Engine &e);
 int launch_nl_build(Engine &e, int force, int from_partials = 0);
 int launch_pack(Engine &e);
 int launch_pair(Engine &e, int field_mode, int want_virial, int energy = 1);
-int pair_tiles(int ngroup);
+int pair_tiles(int ngroup, int lanes);
+// groups of all systems up to which a group gets a whole wavefront of the pair
+// kernel (rspace.hip)
+constexpr int PAIR_WIDE_GROUPS = 2048;
 // P3M mesh buffers of one system (pppm.hip)
 int p3m_mesh_layout(SysParams &P, long &mesh, long &cmesh);
 long p3m_green_at(const SysParams &P, int ix, int iy, int kz);

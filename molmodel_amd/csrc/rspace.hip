@@ -11,7 +11,7 @@
 //   * Lorentz-Berthelot LJ (rspace.c:258-297) via a per-type-pair table;
 //   * the switching derivative times the sum of unswitched pair energies acts
 //     on the first sites (rspace.c:479-489).
-// MI355X mapping: groups are cell-sorted; 16 lanes serve one i-group and
+// MI355X mapping: groups are cell-sorted; 16 or 64 lanes serve one i-group and
 // walk its full neighbour row (both directions, so every force lands on the
 // lane's own i-group and no atomics are needed); the i-group lives in
 // registers; neighbours inside the cutoff are compacted into an LDS queue
@@ -38,24 +38,21 @@ __global__ void k_pack(const SysParams *__restrict__ sp, const int *__restrict__
   pack_group(gs, gfirst[g], gns[g], ginfo[g], r, q, N, gpos, spk, gmeta);
 }
 
+// (the width keeps the compiler's address arithmetic, and with it the kernel's
+// registers, low: without it k_pair spills)
 __device__ __forceinline__ double shfl_xor_d(double v, int m) { return __shfl_xor(v, m, 16); }
 
-
 constexpr int NSI = 3;       // sites per group handled by the pair kernel
-constexpr int LANES = 16;    // lanes per i-group
 constexpr int PAIR_TB = 256;
-constexpr int GPB = PAIR_TB / LANES;   // i-groups per block
 constexpr int MAXTAB = 1536;
 constexpr int MAXLJ = 64;
 
-constexpr int QCAP = 32;      // queue entries per i-group (one batch of 16 + a fill of 16)
-
-// The pair kernel.  Each 16-lane segment owns one i-group and alternates
-// two phases over its neighbour row:
-//   filter:  16 candidates at a time; FP64 minimum image and the
+// The pair kernel.  Each segment of LANES lanes (16, or a whole wavefront)
+// owns one i-group and alternates two phases over its neighbour row:
+//   filter:  LANES candidates at a time; FP64 minimum image and the
 //            r^2 > rc^2 decision of rspace.c:423-445, the switching value
 //            and derivative (rspace.c:52-58) from the FP64 distance in FP32;
-//            accepted neighbours are compacted into a per-segment LDS queue
+//            accepted neighbours are compacted into a per-segment LDS ring
 //            with a ballot (FP32 shift, switching value and derivative);
 //   compute: once every segment of the wavefront holds a full batch (or has
 //            no candidates left), each lane takes one queued group pair and
@@ -63,6 +60,22 @@ constexpr int QCAP = 32;      // queue entries per i-group (one batch of 16 + a 
 //            into FP64 accumulators.
 // Lanes therefore spend the expensive phase almost only on pairs inside the
 // cutoff.
+//
+// Bound by VALU issue (76 % of the cycles at 32768 waters, 81 us).  Below
+// some thousand groups the chip is not full and the time is one segment's
+// chain instead: with 16 lanes a row of 370 candidates is 23 filter passes
+// and about 12 batches one after the other.  A wavefront per group cuts the
+// chain to a fourth.  One step of dynamics, 16 and 64 lanes: 49.9 and 40.9 us
+// (216 waters), 71.1 and 49.6 (960 waters with ions); from about 3000 groups
+// on the chip is full, and the partly empty last batches and the other
+// stream's kernels make up for it: 70.7 and 71.9 us (2900), 64.0 and 68.5
+// (4096), 140 and 171 (32768).  PAIR_WIDE_GROUPS lies between.
+//
+// Both widths add in one order, so that a system's forces do not depend on
+// what else is in its engine: the a-th accepted neighbour of a group belongs
+// to accumulator a mod 16, in order.  With 64 lanes the four rows of 16 lanes
+// of a batch are therefore added one after the other, through shuffles, by
+// every row.
 // erfc(eta r)/r of one charged site pair (b0) and its radial force factor
 // times the smoothed charge qs (e), from the LDS table inside its range and
 // from the functions outside it (rspace.c:120-125).  Both table segments
@@ -118,14 +131,23 @@ __device__ __forceinline__ void coul_table(const TabView &T, const float4 *stab,
   e = fmaf(fr, fmaf(c.w, fr, p2), p1) * (inA ? qsA : qsB);
 }
 
+// FP32 sums of one group pair, and what the virial takes from it
+struct PairSums {
+  float fx[NSI], fy[NSI], fz[NSI], ph[NSI], gx[NSI], gy[NSI], gz[NSI];
+  float uu, sx, sy, sz, Dx, Dy, Dz;
+  double Fx, Fy, Fz;
+};
+
 // One tile: the GPB i-groups blk * GPB ... of system P.  The block's LDS
 // holds that system's erfc and LJ tables.
-template <bool FIELD, bool VIRIAL, bool WATER, bool ENERGY>
+template <bool FIELD, bool VIRIAL, bool WATER, bool ENERGY, int LANES>
 __device__ __forceinline__ void pair_tile(
-    const SysParams &P, int blk, const float4 *stab, const float2 *slj, float4 (*qd)[QCAP],
-    float2 (*qs)[QCAP], const double4 *__restrict__ gpos, const float4 *__restrict__ spk,
+    const SysParams &P, int blk, const float4 *stab, const float2 *slj, float4 (*qd)[2 * LANES],
+    float2 (*qs)[2 * LANES], const double4 *__restrict__ gpos, const float4 *__restrict__ spk,
     const int2 *__restrict__ gmeta, const int *__restrict__ nbr, const int *__restrict__ nnb,
     int nbcap, double *__restrict__ pf, double *__restrict__ plj, double *__restrict__ gacc) {
+  constexpr int GPB = PAIR_TB / LANES;
+  constexpr unsigned long long SEG = LANES == 64 ? ~0ull : (1ull << (LANES & 63)) - 1ull;
   const int lane = threadIdx.x & (LANES - 1);
   const int segw = (threadIdx.x & 63) / LANES;     // segment within the wavefront
   const int seg = threadIdx.x / LANES;             // segment within the block
@@ -168,7 +190,7 @@ __device__ __forceinline__ void pair_tile(
   const int *row = nbr + (long)gs * nbcap;
   float4 *myqd = qd[seg];
   float2 *myqs = qs[seg];
-  int qn = 0, t0 = 0;
+  int qn = 0, qh = 0, t0 = 0;   // queued entries, the first one's place in the ring
   // the row entry of the lane's next candidate, loaded one filter pass ahead
   int hnext = lane < cnt ? row[lane] : 0;
 
@@ -201,14 +223,14 @@ __device__ __forceinline__ void pair_tile(
         dsmf = dsz;
       }
       const unsigned long long bal = __ballot(take);
-      const unsigned sb = (unsigned)(bal >> (segw * LANES)) & 0xffffu;
+      const unsigned long long sb = (bal >> (segw * LANES)) & SEG;
       if (take) {
-        const int pos = qn + __popc(sb & ((1u << lane) - 1u));
+        const int pos = (qh + qn + __popcll(sb & ((1ull << lane) - 1ull))) & (2 * LANES - 1);
         myqd[pos] = ent;
         myqs[pos] = make_float2(dsmf, __int_as_float(hs));
       }
       if (fill) {
-        qn += __popc(sb);
+        qn += __popcll(sb);
         t0 += LANES;
       }
       __builtin_amdgcn_wave_barrier();
@@ -216,17 +238,40 @@ __device__ __forceinline__ void pair_tile(
     if (!__any(qn > 0)) break;
     // ---- compute one batch per segment
     const int nb = qn < LANES ? qn : LANES;
-    if (lane < nb) {
-      const float4 ent = myqd[qn - nb + lane];
-      const float2 e2 = myqs[qn - nb + lane];
+    // a pair's sums into the accumulators: the lane's own (16 lanes), or those
+    // of lane (lane mod 16) + 16 q of the batch
+    auto accumulate = [&](const PairSums &S, int q) {
+      const int from = 16 * q + (lane & 15);
+      auto f = [&](float x) { return (double)(LANES == 64 ? __shfl(x, from) : x); };
+      auto d = [&](double x) { return LANES == 64 ? __shfl(x, from) : x; };
+#pragma unroll
+      for (int k = 0; k < NSI; k++) {
+        if (ENERGY) ap[k] += f(S.ph[k]);
+        ax[k] += f(S.fx[k]); ay[k] += f(S.fy[k]); az[k] += f(S.fz[k]);
+        if (FIELD) { lx[k] += f(S.gx[k]); ly[k] += f(S.gy[k]); lz[k] += f(S.gz[k]); }
+      }
+      if (FIELD) { lx[0] += f(S.sx); ly[0] += f(S.sy); lz[0] += f(S.sz); }
+      if (ENERGY) ulj += f(S.uu);
+      if (VIRIAL) {   // 1/2 D (x) F_gh per directed pair
+        const double dx = f(S.Dx), dy = f(S.Dy), dz = f(S.Dz), X = d(S.Fx), Y = d(S.Fy), Z = d(S.Fz);
+        w[0] += 0.5 * dx * X; w[1] += 0.5 * dx * Y; w[2] += 0.5 * dx * Z;
+        w[3] += 0.5 * dy * X; w[4] += 0.5 * dy * Y; w[5] += 0.5 * dy * Z;
+        w[6] += 0.5 * dz * X; w[7] += 0.5 * dz * Y; w[8] += 0.5 * dz * Z;
+      }
+    };
+    // the queued group pair of this lane
+    auto evaluate = [&](PairSums &S) {
+      float (&fx)[NSI] = S.fx, (&fy)[NSI] = S.fy, (&fz)[NSI] = S.fz, (&ph)[NSI] = S.ph;
+      float (&gx)[NSI] = S.gx, (&gy)[NSI] = S.gy, (&gz)[NSI] = S.gz;
+      float tmps, uu;
+      const int at = (qh + lane) & (2 * LANES - 1);
+      const float4 ent = myqd[at];
+      const float2 e2 = myqs[at];
       const int hs = __float_as_int(e2.y);
       const float smf = ent.w, dsmf = e2.x;
       const int2 mj = gmeta[hs];
       const int nsj = mj.x;
       const float Dx = ent.x, Dy = ent.y, Dz = ent.z;
-      // per group pair FP32 sums (set by the path that runs)
-      float fx[NSI], fy[NSI], fz[NSI], ph[NSI], gx[NSI], gy[NSI], gz[NSI];
-      float tmps, uu;
       bool general = true;
       if (WATER && P.water) {
         // every group of this system is a three-site water: nine charged
@@ -324,37 +369,44 @@ __device__ __forceinline__ void pair_tile(
       // smoothing force on the first site (rspace.c:479-489)
       const float fs = dsmf * tmps;
       const float sx = fs * Dx, sy = fs * Dy, sz = fs * Dz;
-      double Fx = 0, Fy = 0, Fz = 0;
+      S.uu = uu;
+      if (FIELD) {
+        S.sx = sx; S.sy = sy; S.sz = sz;
+      } else {
+        // forces: the smoothing force joins the first site's FP32 sum
+        if (VIRIAL) {
+          S.Dx = Dx; S.Dy = Dy; S.Dz = Dz;
+          S.Fx = S.Fy = S.Fz = 0;
+        }
 #pragma unroll
-      for (int k = 0; k < NSI; k++) {
-        if (ENERGY) ap[k] += (double)ph[k];
-        if (FIELD) {
-          ax[k] += (double)fx[k]; ay[k] += (double)fy[k]; az[k] += (double)fz[k];
-          lx[k] += (double)gx[k]; ly[k] += (double)gy[k]; lz[k] += (double)gz[k];
-        } else {
-          // the smoothing force joins the first site's FP32 sum
+        for (int k = 0; k < NSI; k++) {
           const float qk = oi[k].w;
-          float tx = qk * fx[k] + gx[k], ty = qk * fy[k] + gy[k], tz = qk * fz[k] + gz[k];
-          if (k == 0) { tx += sx; ty += sy; tz += sz; }
-          ax[k] += (double)tx; ay[k] += (double)ty; az[k] += (double)tz;
-          if (VIRIAL) { Fx += tx; Fy += ty; Fz += tz; }
+          fx[k] = qk * fx[k] + gx[k];
+          fy[k] = qk * fy[k] + gy[k];
+          fz[k] = qk * fz[k] + gz[k];
+          if (k == 0) { fx[k] += sx; fy[k] += sy; fz[k] += sz; }
+          if (VIRIAL) { S.Fx += fx[k]; S.Fy += fy[k]; S.Fz += fz[k]; }
         }
       }
-      if (FIELD) { lx[0] += (double)sx; ly[0] += (double)sy; lz[0] += (double)sz; }
-      if (ENERGY) ulj += (double)uu;
-      if (VIRIAL) {   // 1/2 D (x) F_gh per directed pair
-        const double dx = Dx, dy = Dy, dz = Dz;
-        w[0] += 0.5 * dx * Fx; w[1] += 0.5 * dx * Fy; w[2] += 0.5 * dx * Fz;
-        w[3] += 0.5 * dy * Fx; w[4] += 0.5 * dy * Fy; w[5] += 0.5 * dy * Fz;
-        w[6] += 0.5 * dz * Fx; w[7] += 0.5 * dz * Fy; w[8] += 0.5 * dz * Fz;
+    };
+    if constexpr (LANES == 16) {
+      if (lane < nb) {
+        PairSums S;
+        evaluate(S);
+        accumulate(S, 0);
       }
+    } else {
+      PairSums S = {};
+      if (lane < nb) evaluate(S);
+      for (int q = 0; 16 * q < nb; q++) accumulate(S, q);
     }
     qn -= nb;
+    qh = (qh + nb) & (2 * LANES - 1);
     __builtin_amdgcn_wave_barrier();
   }
-  // reduce the 16 lanes of each i-group
+  // reduce the 16 lanes of each i-group (64 lanes hold the sums four times over)
 #pragma unroll
-  for (int m = LANES / 2; m >= 1; m >>= 1) {
+  for (int m = 8; m >= 1; m >>= 1) {
 #pragma unroll
     for (int k = 0; k < NSI; k++) {
       ax[k] += shfl_xor_d(ax[k], m); ay[k] += shfl_xor_d(ay[k], m);
@@ -412,7 +464,7 @@ __device__ __forceinline__ void pair_tile(
 // another system's tables.  The host sizes the grid below the device's
 // resident capacity, which leaves room on every CU for the reciprocal-space
 // kernels running on the other stream.
-template <bool FIELD, bool VIRIAL, bool WATER, bool ENERGY>
+template <bool FIELD, bool VIRIAL, bool WATER, bool ENERGY, int LANES>
 __global__ void __launch_bounds__(PAIR_TB, (FIELD || VIRIAL) ? 1 : 4) k_pair(
     const SysParams *__restrict__ sp, const int *__restrict__ tile_start, int nsys, int ntile,
     const double4 *__restrict__ gpos, const float4 *__restrict__ spk,
@@ -421,8 +473,10 @@ __global__ void __launch_bounds__(PAIR_TB, (FIELD || VIRIAL) ? 1 : 4) k_pair(
     double *__restrict__ pf, double *__restrict__ plj, double *__restrict__ gacc) {
   __shared__ float4 stab[MAXTAB];
   __shared__ float2 slj[MAXLJ];
-  __shared__ float4 qd[GPB][QCAP];    // Dx, Dy, Dz, switching value
-  __shared__ float2 qs[GPB][QCAP];    // switching derivative, neighbour (int bits)
+  // per i-group one batch and a fill: Dx, Dy, Dz, switching value; switching
+  // derivative, neighbour (int bits)
+  __shared__ float4 qd[PAIR_TB / LANES][2 * LANES];
+  __shared__ float2 qs[PAIR_TB / LANES][2 * LANES];
   const int cls = blockIdx.x & 7;
   const int nper = (int)((gridDim.x + 7 - cls) >> 3);   // blocks in this class
   const int lo = (int)((long)ntile * cls / 8), hi = (int)((long)ntile * (cls + 1) / 8);
@@ -442,7 +496,7 @@ __global__ void __launch_bounds__(PAIR_TB, (FIELD || VIRIAL) ? 1 : 4) k_pair(
       __syncthreads();
       cur = a;
     }
-    pair_tile<FIELD, VIRIAL, WATER, ENERGY>(P, t - tile_start[a], stab, slj, qd, qs, gpos, spk, gmeta, nbr,
+    pair_tile<FIELD, VIRIAL, WATER, ENERGY, LANES>(P, t - tile_start[a], stab, slj, qd, qs, gpos, spk, gmeta, nbr,
                              nnb, nbcap, pf, plj, gacc);
   }
 }
@@ -679,7 +733,7 @@ __global__ void __launch_bounds__(NP_TB) k_nonperiodic(const double4 *__restrict
     }
   }
   if (MODE == 0) {   // the block's LJ energy, reduced in a fixed order
-    for (int o = 32; o >= 1; o >>= 1) u += __shfl_xor(u, o);
+    for (int o = 32; o >= 1; o >>= 1) u += shfl_xor_d(u, o);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = u;
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -746,7 +800,10 @@ int launch_nonperiodic_points(const double4 *site, const double *rscreen, int n,
   return 0;
 }
 
-int pair_tiles(int ngroup) { return (ngroup + GPB - 1) / GPB; }
+int pair_tiles(int ngroup, int lanes) {
+  const int g = PAIR_TB / lanes;
+  return (ngroup + g - 1) / g;
+}
 
 int launch_pair(Engine &e, int field_mode, int want_virial, int energy) {
   if (e.ntile == 0) return 0;
@@ -757,11 +814,13 @@ int launch_pair(Engine &e, int field_mode, int want_virial, int energy) {
   // WATER: the kernel carries the path for systems made only of three-site
   // waters
   // ENERGY false (forces only) for steps whose energies nobody reads
-#define PAIR_LAUNCH(F, V, EN)                                                                \
+#define PAIR_LANES(F, V, EN, L)                                                              \
   if (e.any_water)                                                                           \
-    hipLaunchKernelGGL((k_pair<F, V, true, EN>), grid, tb, 0, e.stream, PAIR_ARGS);          \
+    hipLaunchKernelGGL((k_pair<F, V, true, EN, L>), grid, tb, 0, e.stream, PAIR_ARGS);       \
   else                                                                                       \
-    hipLaunchKernelGGL((k_pair<F, V, false, EN>), grid, tb, 0, e.stream, PAIR_ARGS);
+    hipLaunchKernelGGL((k_pair<F, V, false, EN, L>), grid, tb, 0, e.stream, PAIR_ARGS);
+#define PAIR_LAUNCH(F, V, EN)                                                                \
+  if (e.pair_lanes == 64) { PAIR_LANES(F, V, EN, 64) } else { PAIR_LANES(F, V, EN, 16) }
   if (field_mode) {
     PAIR_LAUNCH(true, false, true)
   } else if (want_virial) {
@@ -772,6 +831,7 @@ int launch_pair(Engine &e, int field_mode, int want_virial, int energy) {
     PAIR_LAUNCH(false, false, false)
   }
 #undef PAIR_LAUNCH
+#undef PAIR_LANES
 #undef PAIR_ARGS
   MM_HIP(hipGetLastError());
   return 0;
