@@ -133,6 +133,7 @@ int mm_engine_create_shaped(int nsys, const mm_system_desc *sys, const mm_shape 
   m->e.graph_steps = shape->graph_steps;
   m->e.spread_halo = shape->spread_halo;
   int rc = engine_create(m->e, in);
+  if (!rc) rc = stage_create(m->e);
   if (rc) {
     engine_destroy(m->e);
     delete m;
@@ -250,58 +251,30 @@ int mm_engine_sizes(const mm_engine *m, int *nsite, int *ngroup) {
   return MM_OK;
 }
 
-static int put_aos(mm_engine *m, double *d, const double *h) {
-  Engine &e = m->e;
-  const int N = e.nsite;
-  std::vector<double> soa(3 * (size_t)N);
-  for (int i = 0; i < N; i++)
-    for (int c = 0; c < 3; c++) soa[(size_t)c * N + i] = h[3 * (size_t)i + c];
-  MM_HIP(hipMemcpyAsync(d, soa.data(), soa.size() * sizeof(double), hipMemcpyHostToDevice, e.stream));
-  MM_HIP(hipStreamSynchronize(e.stream));
-  return 0;
-}
-
-static int get_aos(mm_engine *m, const double *d, double *h) {
-  Engine &e = m->e;
-  const int N = e.nsite;
-  std::vector<double> soa(3 * (size_t)N);
-  MM_HIP(hipMemcpyAsync(soa.data(), d, soa.size() * sizeof(double), hipMemcpyDeviceToHost, e.stream));
-  MM_HIP(hipStreamSynchronize(e.stream));
-  for (int i = 0; i < N; i++)
-    for (int c = 0; c < 3; c++) h[3 * (size_t)i + c] = soa[(size_t)c * N + i];
-  return 0;
-}
-
 int mm_set_positions(mm_engine *m, const double *r) {
   CHECK_ENGINE(m);
   if (!r) { set_last_error("null positions"); return MM_ERR_ARG; }
-  TRY(put_aos(m, m->e.d_r, r));
+  TRY(stage_put_sites(m->e, m->e.d_r, r));
   m->pos_dirty = 1;
   m->e.md_phase = 0;
   return MM_OK;
 }
-int mm_get_positions(mm_engine *m, double *r) { CHECK_ENGINE(m); return get_aos(m, m->e.d_r, r); }
+int mm_get_positions(mm_engine *m, double *r) { CHECK_ENGINE(m); return stage_get_sites(m->e, m->e.d_r, r); }
 int mm_set_velocities(mm_engine *m, const double *v) {
   CHECK_ENGINE(m);
   if (!v) { set_last_error("null velocities"); return MM_ERR_ARG; }
-  return put_aos(m, m->e.d_v, v);
+  return stage_put_sites(m->e, m->e.d_v, v);
 }
-int mm_get_velocities(mm_engine *m, double *v) { CHECK_ENGINE(m); return get_aos(m, m->e.d_v, v); }
-int mm_get_forces(mm_engine *m, double *f) { CHECK_ENGINE(m); return get_aos(m, m->e.d_f, f); }
+int mm_get_velocities(mm_engine *m, double *v) { CHECK_ENGINE(m); return stage_get_sites(m->e, m->e.d_v, v); }
+int mm_get_forces(mm_engine *m, double *f) { CHECK_ENGINE(m); return stage_get_sites(m->e, m->e.d_f, f); }
 
 int mm_get_potential(mm_engine *m, double *phi) {
   CHECK_ENGINE(m);
-  MM_HIP(hipMemcpyAsync(phi, m->e.d_phi, sizeof(double) * m->e.nsite, hipMemcpyDeviceToHost, m->e.stream));
-  MM_HIP(hipStreamSynchronize(m->e.stream));
-  return MM_OK;
+  return stage_get(m->e, m->e.d_phi, phi, sizeof(double) * m->e.nsite);
 }
 
 static int read_err(Engine &e, int *flags) {
-  int h = 0;
-  MM_HIP(hipMemcpyAsync(&h, e.d_err, sizeof(int), hipMemcpyDeviceToHost, e.stream));
-  MM_HIP(hipStreamSynchronize(e.stream));
-  *flags = h;
-  return 0;
+  return stage_get(e, e.d_err, flags, sizeof(int));
 }
 
 static int clear_err(Engine &e) {
@@ -495,8 +468,7 @@ int mm_get_energies(mm_engine *m, double *en) {
   CHECK_ENGINE(m);
   Engine &e = m->e;
   std::vector<double> acc((size_t)e.nsys * NACC);
-  MM_HIP(hipMemcpyAsync(acc.data(), e.d_acc, acc.size() * sizeof(double), hipMemcpyDeviceToHost, e.stream));
-  MM_HIP(hipStreamSynchronize(e.stream));
+  TRY(stage_get(e, e.d_acc, acc.data(), acc.size() * sizeof(double)));
   for (int s = 0; s < e.nsys; s++) {
     const double *a = &acc[(size_t)s * NACC];
     double *o = en + (size_t)s * MM_NE;
@@ -516,10 +488,8 @@ int mm_get_virial(mm_engine *m, double *w) {
   CHECK_ENGINE(m);
   Engine &e = m->e;
   std::vector<double> acc((size_t)e.nsys * NACC), kv(9 * (size_t)e.nsys);
-  MM_HIP(hipMemcpyAsync(acc.data(), e.d_acc, acc.size() * sizeof(double), hipMemcpyDeviceToHost, e.stream));
-  MM_HIP(hipMemcpyAsync(kv.data(), e.d_kres + 4L * e.nsite, kv.size() * sizeof(double),
-                        hipMemcpyDeviceToHost, e.stream));
-  MM_HIP(hipStreamSynchronize(e.stream));
+  TRY(stage_get(e, e.d_acc, acc.data(), acc.size() * sizeof(double)));
+  TRY(stage_get(e, e.d_kres + 4L * e.nsite, kv.data(), kv.size() * sizeof(double)));
   for (int s = 0; s < e.nsys; s++)
     for (int c = 0; c < 9; c++)
       w[9 * s + c] = acc[(size_t)s * NACC + ACC_VIR + c] + kv[9 * s + c] +
@@ -653,7 +623,7 @@ int mm_nlist_update(mm_nlist *nl, const double *r) {
   if (!nl || !r) { set_last_error("mm_nlist_update: bad arguments"); return MM_ERR_ARG; }
   mm_engine *m = nl->m;
   Engine &e = m->e;
-  TRY(put_aos(m, e.d_r, r));
+  TRY(stage_put_sites(e, e.d_r, r));
   for (int attempt = 0; attempt < 4; attempt++) {
     if (e.first_eval) {
       TRY(launch_nl_build(e, 1));

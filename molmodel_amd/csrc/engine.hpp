@@ -3,8 +3,10 @@
 // evaluation / one MD step on a single HIP stream.
 #pragma once
 #include "mm_common.hpp"
-#include <vector>
+#include <memory>
+#include <mutex>
 #include <string>
+#include <vector>
 
 namespace mmamd {
 
@@ -48,6 +50,15 @@ struct SystemInput {       // mirrors mm_system_desc of include/molmodel_amd.h
   double latv[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
 };
 
+// pinned host memory of an engine with a handle, which stage.hip's kernels read
+// and write (3 doubles a site); one call at a time uses it
+struct Stage {
+  double *h = nullptr;
+  int sites = 0;
+  std::mutex lock;
+  ~Stage() { if (h) hipHostFree(h); }
+};
+
 struct Engine {
   int nsys = 0, nsite = 0, ngroup = 0;
   int maxg = 0;               // max groups of any system (grid x extent)
@@ -60,6 +71,7 @@ struct Engine {
   // (forked from and joined back into `stream` with the two events)
   hipStream_t stream2 = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+  std::shared_ptr<Stage> stage = std::make_shared<Stage>();
 
   SysParams *d_sp = nullptr;
   // topology, original order
@@ -235,6 +247,11 @@ int engine_grow_bins(Engine &e);
 // displacement partials of the last (FIN_LAZY) finish exceed the skin
 int launch_nl_build(Engine &e, int force, int from_partials = 0);
 int launch_pack(Engine &e);
+int stage_create(Engine &e);
+// between the caller's xyz triples and the device's planes; plain words (stage.hip)
+int stage_get_sites(Engine &e, const double *soa, double *aos);
+int stage_put_sites(Engine &e, double *soa, const double *aos);
+int stage_get(Engine &e, const void *d, void *h, size_t bytes);
 int launch_pair(Engine &e, int field_mode, int want_virial, int energy = 1);
 int pair_tiles(int ngroup, int lanes);
 // groups of all systems up to which a group gets a whole wavefront of the pair

@@ -384,7 +384,7 @@ class Engine:
         _check(lib().mm_set_positions(self.h, _ptr(r)))
 
     def positions(self):
-        r = np.zeros((self.nsite, 3))
+        r = np.empty((self.nsite, 3))
         _check(lib().mm_get_positions(self.h, _ptr(r)))
         return r
 
@@ -393,7 +393,7 @@ class Engine:
         _check(lib().mm_set_velocities(self.h, _ptr(v)))
 
     def velocities(self):
-        v = np.zeros((self.nsite, 3))
+        v = np.empty((self.nsite, 3))
         _check(lib().mm_get_velocities(self.h, _ptr(v)))
         return v
 
@@ -402,12 +402,12 @@ class Engine:
         _check(lib().mm_compute(self.h, VIRIAL if virial else 0))
 
     def forces(self):
-        f = np.zeros((self.nsite, 3))
+        f = np.empty((self.nsite, 3))
         _check(lib().mm_get_forces(self.h, _ptr(f)))
         return f
 
     def potential(self):
-        p = np.zeros(self.nsite)
+        p = np.empty(self.nsite)
         _check(lib().mm_get_potential(self.h, _ptr(p)))
         return p
 
