@@ -32,6 +32,44 @@ template <bool VIR> struct FinSlots {
 static_assert(FinSlots<false>::N == FIN_NPART && FinSlots<false>::TOP == FIN_TOP,
               "the neighbour-list check reads this layout");
 
+// erf(er)/r and the derivative factor of an excluded pair (rspace.c:506-512),
+// -erf(er)/r and (-erf(er)/r + 2 eta/sqrt(pi) exp(-er^2)) / r^2 with er = eta r,
+// as eta and eta^3 times power series in y = er^2: 2/sqrt(pi) times
+//   sum (-1)^(n+1) y^n / (n! (2n+1))  and  sum (-1)^(n+1) 2 y^n / (n! (2n+3)).
+// Fifteen terms leave less than 2^-54 of the sum for y <= 1/2, and nothing
+// cancels, as it does in the closed form of the second.
+constexpr double EXCL_Y = 0.5;
+constexpr int EXCL_TERMS = 15;
+struct ExclSeries { double b0[EXCL_TERMS], b1[EXCL_TERMS]; };
+constexpr ExclSeries excl_series() {
+  ExclSeries s{};
+  double f = -1.1283791670955126;   // 2/sqrt(pi) (-1)^(n+1) / n!
+  for (int n = 0; n < EXCL_TERMS; n++) {
+    s.b0[n] = f / (2 * n + 1);
+    s.b1[n] = 2 * f / (2 * n + 3);
+    f /= -(n + 1);
+  }
+  return s;
+}
+__device__ __forceinline__ void excl_pair(double y, double eta, double &b0, double &b1) {
+  constexpr ExclSeries c = excl_series();
+  double p = c.b0[EXCL_TERMS - 1], d = c.b1[EXCL_TERMS - 1];
+#pragma unroll
+  for (int n = EXCL_TERMS - 2; n >= 0; n--) {
+    p = p * y + c.b0[n];
+    d = d * y + c.b1[n];
+  }
+  b0 = eta * p;
+  b1 = eta * eta * eta * d;
+}
+
+// One thread a group: less than one wavefront per SIMD up to 65536 groups, so
+// the time is one thread's chain of FP64 instructions, not memory (of 16 us at
+// 32768 waters the traffic needs 5).  Hence the series of excl_pair for the
+// three pairs of a water at once (erf and exp one pair after the other were
+// 930 instructions, this is 200), water.hpp's economies, and a reduction of
+// only what an inner step's check reads.  An inner step's finish: 216 waters
+// 11.2 -> 7.8 us, 4096 waters 11.9 -> 8.0, 32768 waters 16.1 -> 11.7.
 template <int MODE, bool VIR, bool LAZY>
 __global__ void __launch_bounds__(FIN_TB) k_finish(
     const SysParams *__restrict__ sp, const int *__restrict__ order, const int *__restrict__ gfirst,
@@ -39,7 +77,7 @@ __global__ void __launch_bounds__(FIN_TB) k_finish(
     const double *__restrict__ mass, const double *__restrict__ pf, const double *__restrict__ gacc,
     const double *__restrict__ kres, double *__restrict__ r, double *__restrict__ v,
     double *__restrict__ f, double *__restrict__ phi_out, const double *__restrict__ last,
-    int N, int want_virial, double bond, double angle_rad, double tol,
+    int N, int want_virial, WaterGeom geom, double tol,
     double *__restrict__ part, int *__restrict__ done, int maxblk, double *__restrict__ acc,
     int *__restrict__ rebuild, int *__restrict__ err, double4 *__restrict__ gpos,
     float4 *__restrict__ spk, const int *__restrict__ ginfo, const int *__restrict__ gslot_inv) {
@@ -95,23 +133,46 @@ __global__ void __launch_bounds__(FIN_TB) k_finish(
     // excluded pairs inside the group (rspace.c:492-521)
     const int ex = gexcl[g];
     if (ex) {
-      const double L = P.L, invL = P.invL, eta = P.eta;
+      const double L = P.L, invL = P.invL, eta = P.eta, eta2 = eta * eta;
+      double D[K][3], y[K];   // pairs 01, 02, 12
+      bool on[K], far = false;
 #pragma unroll
       for (int k = 0; k < K; k++)
 #pragma unroll
         for (int l = k + 1; l < K; l++) {
-          if (!((ex >> (k * MAXS + l)) & 1)) continue;
-          double d0 = x[k][0] - x[l][0], d1 = x[k][1] - x[l][1], d2 = x[k][2] - x[l][2];
-          d0 -= L * floor(d0 * invL + 0.5);
-          d1 -= L * floor(d1 * invL + 0.5);
-          d2 -= L * floor(d2 * invL + 0.5);
-          const double r2 = d0 * d0 + d1 * d1 + d2 * d2;
-          const double rm = sqrt(r2), er = eta * rm;
-          const double b0 = -erf(er) / rm;
-          const double b1 = (b0 + eta * 1.1283791670955126 * exp(-er * er)) / r2;
-          ph[k] += qq[l] * b0;
-          ph[l] += qq[k] * b0;
-          const double fq = qq[k] * qq[l] * b1;
+          const int p = k + l - 1;
+#pragma unroll
+          for (int d = 0; d < 3; d++) {
+            D[p][d] = x[k][d] - x[l][d];
+            D[p][d] -= L * floor(D[p][d] * invL + 0.5);
+          }
+          on[p] = (ex >> (k * MAXS + l)) & 1;
+          y[p] = on[p] ? eta2 * (D[p][0] * D[p][0] + D[p][1] * D[p][1] + D[p][2] * D[p][2]) : 0.0;
+          if (y[p] > EXCL_Y) far = true;
+        }
+      double b0[K], b1[K];
+#pragma unroll
+      for (int p = 0; p < K; p++) excl_pair(y[p], eta, b0[p], b1[p]);
+      if (far)
+#pragma unroll 1
+        for (int p = 0; p < K; p++) {
+          const double yp = p == 0 ? y[0] : p == 1 ? y[1] : y[2];
+          if (!(yp > EXCL_Y)) continue;
+          const double er = sqrt(yp), e0 = -eta * erf(er) / er;
+          const double e1 = (e0 + eta * 1.1283791670955126 * exp(-yp)) * eta2 / yp;
+          if (p == 0) { b0[0] = e0; b1[0] = e1; }
+          else if (p == 1) { b0[1] = e0; b1[1] = e1; }
+          else { b0[2] = e0; b1[2] = e1; }
+        }
+#pragma unroll
+      for (int k = 0; k < K; k++)
+#pragma unroll
+        for (int l = k + 1; l < K; l++) {
+          const int p = k + l - 1;
+          const double d0 = D[p][0], d1 = D[p][1], d2 = D[p][2];
+          ph[k] += on[p] ? qq[l] * b0[p] : 0.0;
+          ph[l] += on[p] ? qq[k] * b0[p] : 0.0;
+          const double fq = on[p] ? qq[k] * qq[l] * b1[p] : 0.0;
           F[k][0] += fq * d0; F[k][1] += fq * d1; F[k][2] += fq * d2;
           F[l][0] -= fq * d0; F[l][1] -= fq * d1; F[l][2] -= fq * d2;
           if constexpr (VIR) {
@@ -146,27 +207,31 @@ __global__ void __launch_bounds__(FIN_TB) k_finish(
     if (MODE) {
       const double dt = P.dt;
       const bool water = (ns == 3);
+      WaterGrad c0;
+      double im[K], hm[K];
+#pragma unroll
+      for (int k = 0; k < K; k++) { im[k] = 1 / m[k]; hm[k] = dt / 2 * im[k]; }
+      if (water) water_constraints<false>(&x[0][0], geom, c0, nullptr);
       if (MODE & FIN_KICK) {
 #pragma unroll
         for (int k = 0; k < K; k++)
 #pragma unroll
-          for (int d = 0; d < 3; d++) vv[k][d] += F[k][d] * (dt / 2 / m[k]);
-        if (water) rattle_water(&x[0][0], &vv[0][0], m, bond, angle_rad);
+          for (int d = 0; d < 3; d++) vv[k][d] += F[k][d] * hm[k];
+        if (water) rattle_water(&vv[0][0], c0, im);
+        if (!LAZY)
 #pragma unroll
         for (int k = 0; k < K; k++)
           if (k < ns) vals[2] += 0.5 * m[k] * (vv[k][0] * vv[k][0] + vv[k][1] * vv[k][1] + vv[k][2] * vv[k][2]);
       }
       if (MODE & FIN_DRIFT) {
-        double x0[K][3];
 #pragma unroll
         for (int k = 0; k < K; k++)
 #pragma unroll
           for (int d = 0; d < 3; d++) {
-            x0[k][d] = x[k][d];
-            vv[k][d] += F[k][d] * (dt / 2 / m[k]);
+            vv[k][d] += F[k][d] * hm[k];
             x[k][d] += vv[k][d] * dt;
           }
-        if (water && !shake_water(&x[0][0], &vv[0][0], &x0[0][0], m, dt, bond, angle_rad, tol, 500))
+        if (water && !shake_water(&x[0][0], &vv[0][0], c0, im, dt, geom, tol, 500))
           atomicOr(err, ERR_CONSTRAINT);
 #pragma unroll
         for (int k = 0; k < K; k++)
@@ -199,10 +264,15 @@ __global__ void __launch_bounds__(FIN_TB) k_finish(
     vals[TOP] = sqrt(dx * dx + dy * dy + dz * dz);
   }
   if constexpr (LAZY) {
-    // partials only; a non-finite block sum is a non-finite total
-    store_partials<NPART, TOP, FIN_TB>(vals, part + (long)s * maxblk * NPART, blockIdx.x, red);
+    // the displacements' partials only, and the force sum for the error flag
+    // (a non-finite block sum is a non-finite total)
+    double t[3] = {vals[0], vals[TOP], 0.0};
+    block_reduce<3, 1, FIN_TB>(t, (double(*)[3])red);
     if (threadIdx.x == 0) {
-      if (!(vals[0] == vals[0]) || !(vals[1] == vals[1])) atomicOr(err, ERR_NAN);
+      double *o = part + ((long)s * maxblk + blockIdx.x) * NPART + TOP;
+      o[0] = t[1];
+      o[1] = t[2];
+      if (!(t[0] == t[0])) atomicOr(err, ERR_NAN);
       if (blockIdx.x == 0) rebuild[s] = 0;   // the next check decides
     }
     return;
@@ -224,8 +294,8 @@ __global__ void __launch_bounds__(FIN_TB) k_finish(
 // initial position constraints (mdyn.cpp:120-121: constrain_positions(0))
 __global__ void k_constrain0(const SysParams *__restrict__ sp, const int *__restrict__ gfirst,
                              const int *__restrict__ gns, const double *__restrict__ mass,
-                             double *__restrict__ r, int N, double bond, double angle_rad,
-                             double tol, int *__restrict__ err) {
+                             double *__restrict__ r, int N, WaterGeom geom, double tol,
+                             int *__restrict__ err) {
   const int s = blockIdx.y;
   const SysParams &P = sp[s];
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -233,13 +303,14 @@ __global__ void k_constrain0(const SysParams *__restrict__ sp, const int *__rest
   const int g = P.group0 + i;
   if (gns[g] != 3) return;
   const int s0 = gfirst[g];
-  double x[9], x0[9], vv[9], m[3];
+  double x[9], vv[9], im[3];
+  WaterGrad c0;
   for (int k = 0; k < 3; k++) {
     for (int d = 0; d < 3; d++) { x[3 * k + d] = r[d * N + s0 + k]; vv[3 * k + d] = 0; }
-    m[k] = mass[s0 + k];
+    im[k] = 1 / mass[s0 + k];
   }
-  for (int c = 0; c < 9; c++) x0[c] = x[c];
-  if (!shake_water(x, vv, x0, m, 0.0, bond, angle_rad, tol, 10000)) atomicOr(err, ERR_CONSTRAINT);
+  water_constraints<false>(x, geom, c0, nullptr);
+  if (!shake_water(x, vv, c0, im, 0.0, geom, tol, 10000)) atomicOr(err, ERR_CONSTRAINT);
   for (int k = 0; k < 3; k++)
     for (int d = 0; d < 3; d++) r[d * N + s0 + k] = x[3 * k + d];
 }
@@ -305,8 +376,8 @@ int launch_field_out(Engine &e, double *out, double *ulj, int min_image) {
 int launch_finish_ex(Engine &e, int mode, int want_virial, double *phi_out) {
   dim3 grid((e.maxg + FIN_TB - 1) / FIN_TB, e.nsys);
 #define FIN_ARGS e.d_sp, e.d_order, e.d_gfirst, e.d_gns, e.d_gexcl, e.d_q, e.d_mass, e.d_pf, \
-    e.d_gacc, e.d_kres, e.d_r, e.d_v, e.d_f, phi_out, e.d_last, e.nsite, want_virial, e.bond,  \
-    e.angle * (M_PI / 180.0), e.tol, e.d_fpart, e.d_done, e.nblk_part, e.d_acc, e.d_rebuild,  \
+    e.d_gacc, e.d_kres, e.d_r, e.d_v, e.d_f, phi_out, e.d_last, e.nsite, want_virial, \
+    water_geom(e.bond, e.angle), e.tol, e.d_fpart, e.d_done, e.nblk_part, e.d_acc, e.d_rebuild,  \
     e.d_err, e.d_gpos, e.d_spk, e.d_ginfo, e.d_gslot_inv
 #define FIN_CASE(M)                                                                            \
   if (want_virial)                                                                             \
@@ -339,8 +410,8 @@ int launch_finish(Engine &e, int mode) { return launch_finish_ex(e, mode, 0, nul
 int launch_constrain_initial(Engine &e) {
   const int tb = 256;
   hipLaunchKernelGGL(k_constrain0, dim3((e.maxg + tb - 1) / tb, e.nsys), dim3(tb), 0, e.stream,
-                     e.d_sp, e.d_gfirst, e.d_gns, e.d_mass, e.d_r, e.nsite, e.bond,
-                     e.angle * (M_PI / 180.0), e.tol, e.d_err);
+                     e.d_sp, e.d_gfirst, e.d_gns, e.d_mass, e.d_r, e.nsite,
+                     water_geom(e.bond, e.angle), e.tol, e.d_err);
   MM_HIP(hipGetLastError());
   return 0;
 }

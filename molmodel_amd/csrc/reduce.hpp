@@ -12,8 +12,8 @@ namespace mmamd {
 
 // merge two (largest, second largest) pairs
 __device__ __forceinline__ void top2_merge(double &a1, double &a2, double b1, double b2) {
-  if (b1 > a1) { a2 = fmax(a1, b2); a1 = b1; }
-  else a2 = fmax(a2, b1);
+  a2 = fmax(fmin(a1, b1), fmax(a2, b2));
+  a1 = fmax(a1, b1);
 }
 
 __device__ __forceinline__ double load_coherent(const double *p) {
@@ -43,14 +43,6 @@ __device__ __forceinline__ void block_reduce(double *v, double (*red)[NV]) {
     }
   }
   __syncthreads();
-}
-
-// Store this block's partials only (thread 0 keeps the block's values in v).
-template <int NV, int NSUM, int TB>
-__device__ void store_partials(double *v, double *part, int blk, double (*red)[NV]) {
-  block_reduce<NV, NSUM, TB>(v, red);
-  if (threadIdx.x == 0)
-    for (int c = 0; c < NV; c++) part[(long)blk * NV + c] = v[c];
 }
 
 // Store this block's partials and, in the last block, reduce all nblk

@@ -104,8 +104,8 @@ __global__ void k_copy(const double *__restrict__ a, double *__restrict__ b, lon
 __global__ void __launch_bounds__(256) k_remd_velocities(
     const SysParams *__restrict__ sp, const int *__restrict__ gfirst, const int *__restrict__ gns,
     const double *__restrict__ mass, const double *__restrict__ kT, const double *__restrict__ r,
-    double *__restrict__ v, int N, unsigned long long seed, long long attempt, double bond,
-    double angle_rad, double *__restrict__ part, int *__restrict__ done, int maxblk,
+    double *__restrict__ v, int N, unsigned long long seed, long long attempt, WaterGeom geom,
+    double *__restrict__ part, int *__restrict__ done, int maxblk,
     double *__restrict__ mom) {
   __shared__ double red[4][4];
   __shared__ int islast;
@@ -136,7 +136,12 @@ __global__ void __launch_bounds__(256) k_remd_velocities(
         }
       }
     }
-    if (ns == 3) rattle_water(x, vv, m, bond, angle_rad);
+    if (ns == 3) {
+      WaterGrad c;
+      const double im[3] = {1 / m[0], 1 / m[1], 1 / m[2]};
+      water_constraints<false>(x, geom, c, nullptr);
+      rattle_water(vv, c, im);
+    }
     for (int k = 0; k < 3; k++)
       if (k < ns) {
         const int sk = s0 + k;
@@ -168,7 +173,7 @@ int launch_remd_velocities(Engine &e, long long attempt) {
   const int tb = 256;
   hipLaunchKernelGGL(k_remd_velocities, dim3((e.maxg + 255) / 256, e.nsys), dim3(256), 0, e.stream,
                      e.d_sp, e.d_gfirst, e.d_gns, e.d_mass, e.d_kT, e.d_r, e.d_v, e.nsite,
-                     e.remd_seed, attempt, e.bond, e.angle * (M_PI / 180.0), e.d_part,
+                     e.remd_seed, attempt, water_geom(e.bond, e.angle), e.d_part,
                      e.d_done + 2 * e.nsys, e.nblk_part, e.d_mom);
   hipLaunchKernelGGL(k_remd_zero_momentum, dim3((e.maxs + tb - 1) / tb, e.nsys), dim3(tb), 0,
                      e.stream, e.d_sp, e.d_mom, e.d_v, e.nsite);

@@ -3,63 +3,80 @@
 // (value 0.5 (r^2 - l^2), constraint.cpp:30-66) and one H-O-H angle
 // constraint (constraint.cpp:68-112, geograd.cpp:59-103), solved with the
 // reference's Newton iteration (constraint.cpp:295-358) in FP64.
+//
+// The solver is one chain of FP64 instructions in a kernel that has less than
+// one wavefront per SIMD, so its time is their number.  Gradients are
+// therefore kept as the five vectors they consist of (the O-H1 length reaches
+// O and H1, the O-H2 length O and H2, the angle all three sites) instead of
+// three rows of nine; masses enter as reciprocals; the angle's deviation is
+// taken from the sine of the difference, not from an arc cosine; the 3x3
+// system is solved by cofactors with one division; and the velocity step
+// hands its gradients at the unmoved positions on to the position step.
+// Rattle and three Newton passes were some 3000 instructions and are 1200.
 #pragma once
 #include <hip/hip_runtime.h>
 
 namespace mmamd {
 
-struct WaterC {
-  double val[3];
-  double g[3][9];
+// target geometry: O-H length, H-O-H angle (radians)
+struct WaterGeom {
+  double bond, t0, cos0, sin0;
 };
-
-// gradient entries that can be nonzero: the O-H1 length reaches O and H1
-// (coordinates 0-5), the O-H2 length O and H2 (0-2, 6-8), the angle all
-// nine.  Products with the other entries are exact zeros, and adding a zero
-// leaves a sum unchanged, so the loops below skip them with results equal
-// to the full sums (for finite inputs).
-__host__ __device__ constexpr bool water_reach(int a, int d) {
-  return a == 2 || (a == 0 ? d < 6 : (d < 3 || d >= 6));
+inline WaterGeom water_geom(double bond, double angle_deg) {
+  const double t0 = angle_deg * (M_PI / 180.0);
+  return {bond, t0, cos(t0), sin(t0)};
 }
 
-// constraint values and gradients (constraint.cpp:30-112, geograd.cpp:59-103)
-__device__ inline void water_constraints(const double *x, double bond, double t0, WaterC &c) {
-  for (int a = 0; a < 3; a++)
-    for (int d = 0; d < 9; d++) c.g[a][d] = 0;
-  double r01[3], r02[3];
-  for (int d = 0; d < 3; d++) { r01[d] = x[d] - x[3 + d]; r02[d] = x[d] - x[6 + d]; }
-  c.val[0] = 0.5 * ((r01[0] * r01[0] + r01[1] * r01[1] + r01[2] * r01[2]) - bond * bond);
-  c.val[1] = 0.5 * ((r02[0] * r02[0] + r02[1] * r02[1] + r02[2] * r02[2]) - bond * bond);
-  for (int d = 0; d < 3; d++) {
-    c.g[0][d] = r01[d]; c.g[0][3 + d] = -r01[d];
-    c.g[1][d] = r02[d]; c.g[1][6 + d] = -r02[d];
-  }
-  // angle H1-O-H2: a = H1 - O, b = H2 - O
-  double a[3], b[3];
-  for (int d = 0; d < 3; d++) { a[d] = x[3 + d] - x[d]; b[d] = x[6 + d] - x[d]; }
-  const double a2 = a[0] * a[0] + a[1] * a[1] + a[2] * a[2];
-  const double b2 = b[0] * b[0] + b[1] * b[1] + b[2] * b[2];
-  const double ma2 = 1.0 / a2, mb2 = 1.0 / b2, ab = a[0] * b[0] + a[1] * b[1] + a[2] * b[2];
-  const double ma = sqrt(ma2), mb = sqrt(mb2);
-  const double t0a = ma * mb, t3 = -ma * ma2 * mb * ab, t4 = -ab * ma * mb * mb2;
+// gradients of one configuration: length 1 is r1 on O and -r1 on H1, length 2
+// r2 on O and -r2 on H2, the angle o on O, p on H1 and q on H2
+struct WaterGrad {
+  double r1[3], r2[3], o[3], p[3], q[3];
+};
+
+__device__ __forceinline__ double dot3(const double *a, const double *b) {
+  return a[0] * b[0] + a[1] * b[1] + a[2] * b[2];
+}
+
+// gradients and, if val is given, constraint values
+// (constraint.cpp:30-112, geograd.cpp:59-103)
+template <bool VALUES>
+__device__ __forceinline__ void water_constraints(const double *x, const WaterGeom &w, WaterGrad &c,
+                                                  double *val) {
+  // angle H1-O-H2: a = H1 - O = -r1, b = H2 - O = -r2
+#pragma unroll
+  for (int d = 0; d < 3; d++) { c.r1[d] = x[d] - x[3 + d]; c.r2[d] = x[d] - x[6 + d]; }
+  const double a2 = dot3(c.r1, c.r1), b2 = dot3(c.r2, c.r2), ab = dot3(c.r1, c.r2);
+  const double ma = rsqrt(a2), mb = rsqrt(b2), t0a = ma * mb;
+  const double t3 = -t0a * ab * ma * ma, t4 = -t0a * ab * mb * mb;
   double ct = ab * t0a;
   ct = ct > 1 ? 1 : (ct < -1 ? -1 : ct);
   const double s2t = 1 - ct * ct;
-  double dt, t;
-  if (s2t < 64.0 * 2.220446049250313e-16) { dt = 0; t = ct > 0 ? 0 : M_PI; }
-  else { dt = -1 / sqrt(s2t); t = acos(ct); }
-  for (int d = 0; d < 3; d++) {
-    const double g1 = (b[d] * t0a + a[d] * t3) * dt;
-    const double g3 = (a[d] * t0a + b[d] * t4) * dt;
-    c.g[2][3 + d] = g1;
-    c.g[2][6 + d] = g3;
-    c.g[2][d] = -g1 - g3;
+  const bool flat = s2t < 64.0 * 2.220446049250313e-16;
+  const double is = flat ? 0 : rsqrt(s2t);
+#pragma unroll
+  for (int d = 0; d < 3; d++) {   // -1/sin times the derivative of cos
+    c.p[d] = (c.r2[d] * t0a + c.r1[d] * t3) * is;
+    c.q[d] = (c.r1[d] * t0a + c.r2[d] * t4) * is;
+    c.o[d] = -c.p[d] - c.q[d];
   }
-  c.val[2] = t - t0;
+  if constexpr (VALUES) {
+    val[0] = 0.5 * (a2 - w.bond * w.bond);
+    val[1] = 0.5 * (b2 - w.bond * w.bond);
+    // t - t0 from z = sin(t - t0): near the target the arc sine's series
+    // (through z^9; the next term is below 2^-65 of z at |z| = 1/64),
+    // elsewhere, and where t - t0 is not within a quarter turn, the angle
+    const double st = s2t * is, z = st * w.cos0 - ct * w.sin0;
+    if (!flat && fabs(z) < 0.015625 && ct * w.cos0 + st * w.sin0 > 0) {
+      const double z2 = z * z;
+      val[2] = z + z * z2 * (1.0 / 6 + z2 * (3.0 / 40 + z2 * (15.0 / 336 + z2 * (105.0 / 3456))));
+    } else {
+      val[2] = (flat ? (ct > 0 ? 0 : M_PI) : acos(ct)) - w.t0;
+    }
+  }
 }
 
 // 3x3 Gaussian elimination with partial pivoting
-__device__ inline bool solve3(double s[3][3], double *x) {
+__device__ inline bool solve3_pivot(double s[3][3], double *x) {
   for (int c = 0; c < 3; c++) {
     int piv = c;
     for (int r = c + 1; r < 3; r++)
@@ -83,81 +100,87 @@ __device__ inline bool solve3(double s[3][3], double *x) {
   return true;
 }
 
-// constraint.cpp:295-335; returns false if not converged
-__device__ inline bool shake_water(double *x, double *v, const double *x0, const double *m, double dt,
-                            double bond, double t0, double tol, int maxit) {
-  WaterC c0;
-  water_constraints(x0, bond, t0, c0);
-  double sci0[3][9];
+// By cofactors where the determinant is of the size of the diagonal's product
+// (a water's is 0.997 of it), by elimination where it is not: a bent molecule
+// stretched flat, masses of very different size.
+__device__ __forceinline__ bool solve3(double s[3][3], double *x) {
+  const double c0 = s[1][1] * s[2][2] - s[1][2] * s[2][1];
+  const double c1 = s[1][2] * s[2][0] - s[1][0] * s[2][2];
+  const double c2 = s[1][0] * s[2][1] - s[1][1] * s[2][0];
+  const double det = s[0][0] * c0 + s[0][1] * c1 + s[0][2] * c2;
+  if (!(fabs(det) > 0.01 * fabs(s[0][0] * s[1][1] * s[2][2]))) return solve3_pivot(s, x);
+  const double id = 1.0 / det, b0 = x[0], b1 = x[1], b2 = x[2];
+  x[0] = (b0 * c0 + b1 * (s[0][2] * s[2][1] - s[0][1] * s[2][2]) +
+          b2 * (s[0][1] * s[1][2] - s[0][2] * s[1][1])) * id;
+  x[1] = (b0 * c1 + b1 * (s[0][0] * s[2][2] - s[0][2] * s[2][0]) +
+          b2 * (s[0][2] * s[1][0] - s[0][0] * s[1][2])) * id;
+  x[2] = (b0 * c2 + b1 * (s[0][1] * s[2][0] - s[0][0] * s[2][1]) +
+          b2 * (s[0][0] * s[1][1] - s[0][1] * s[1][0])) * id;
+  return true;
+}
+
+// s[a][b] = (gradient a of c) . (gradient b of c0) / masses
+__device__ __forceinline__ void water_matrix(const WaterGrad &c, const WaterGrad &c0, const double *im,
+                                             double s[3][3]) {
+  s[0][0] = dot3(c.r1, c0.r1) * (im[0] + im[1]);
+  s[0][1] = dot3(c.r1, c0.r2) * im[0];
+  s[0][2] = dot3(c.r1, c0.o) * im[0] - dot3(c.r1, c0.p) * im[1];
+  s[1][0] = dot3(c.r2, c0.r1) * im[0];
+  s[1][1] = dot3(c.r2, c0.r2) * (im[0] + im[2]);
+  s[1][2] = dot3(c.r2, c0.o) * im[0] - dot3(c.r2, c0.q) * im[2];
+  s[2][0] = dot3(c.o, c0.r1) * im[0] - dot3(c.p, c0.r1) * im[1];
+  s[2][1] = dot3(c.o, c0.r2) * im[0] - dot3(c.q, c0.r2) * im[2];
+  s[2][2] = dot3(c.o, c0.o) * im[0] + dot3(c.p, c0.p) * im[1] + dot3(c.q, c0.q) * im[2];
+}
+
+// sum over the constraints of x[a] (gradient a) / masses
+__device__ __forceinline__ void water_shift(const WaterGrad &c, const double *im, const double *x,
+                                            double *dx) {
 #pragma unroll
-  for (int a = 0; a < 3; a++)
-#pragma unroll
-    for (int d = 0; d < 9; d++) sci0[a][d] = water_reach(a, d) ? c0.g[a][d] / m[d / 3] : 0.0;
+  for (int d = 0; d < 3; d++) {
+    dx[d] = (x[0] * c.r1[d] + x[1] * c.r2[d] + x[2] * c.o[d]) * im[0];
+    dx[3 + d] = (x[2] * c.p[d] - x[0] * c.r1[d]) * im[1];
+    dx[6 + d] = (x[2] * c.q[d] - x[1] * c.r2[d]) * im[2];
+  }
+}
+
+// constraint.cpp:295-335 from the gradients c0 at the old positions (im:
+// reciprocal masses); returns false if not converged
+__device__ inline bool shake_water(double *x, double *v, const WaterGrad &c0, const double *im, double dt,
+                                   const WaterGeom &w, double tol, int maxit) {
   const double invdt = dt > 0 ? 1 / dt : 0;
   for (int it = 0; it < maxit; it++) {
-    WaterC c;
-    water_constraints(x, bond, t0, c);
-    double xs[3];
+    WaterGrad c;
+    double xs[3], s[3][3], dx[9];
+    water_constraints<true>(x, w, c, xs);
     bool sat = true;
-    for (int a = 0; a < 3; a++) { xs[a] = -c.val[a]; if (fabs(xs[a]) > tol) sat = false; }
+#pragma unroll
+    for (int a = 0; a < 3; a++) { xs[a] = -xs[a]; if (fabs(xs[a]) > tol) sat = false; }
     if (sat) return true;
-    double s[3][3];
-#pragma unroll
-    for (int a = 0; a < 3; a++)
-#pragma unroll
-      for (int b = 0; b < 3; b++) {
-        double t = 0;
-#pragma unroll
-        for (int d = 0; d < 9; d++)
-          if (water_reach(a, d) && water_reach(b, d)) t += c.g[a][d] * sci0[b][d];
-        s[a][b] = t;
-      }
+    water_matrix(c, c0, im, s);
     if (!solve3(s, xs)) return false;
+    water_shift(c0, im, xs, dx);
 #pragma unroll
-    for (int a = 0; a < 3; a++)
-#pragma unroll
-      for (int d = 0; d < 9; d++) {
-        if (!water_reach(a, d)) continue;
-        const double dx = xs[a] * sci0[a][d];
-        x[d] += dx;
-        v[d] += dx * invdt;
-      }
+    for (int d = 0; d < 9; d++) { x[d] += dx[d]; v[d] += dx[d] * invdt; }
   }
   return false;
 }
 
-// constraint.cpp:336-358
-__device__ inline void rattle_water(const double *x, double *v, const double *m, double bond, double t0) {
-  WaterC c;
-  water_constraints(x, bond, t0, c);
-  double sci0[3][9], xs[3], s[3][3];
+// constraint.cpp:336-358 from the gradients at the positions
+__device__ __forceinline__ void rattle_water(double *v, const WaterGrad &c, const double *im) {
+  double xs[3], s[3][3], dx[9];
+  xs[0] = xs[1] = xs[2] = 0;
 #pragma unroll
-  for (int a = 0; a < 3; a++) {
-    xs[a] = 0;
-#pragma unroll
-    for (int d = 0; d < 9; d++) {
-      sci0[a][d] = 0.0;
-      if (!water_reach(a, d)) continue;
-      sci0[a][d] = c.g[a][d] / m[d / 3];
-      xs[a] -= c.g[a][d] * v[d];
-    }
+  for (int d = 0; d < 3; d++) {
+    xs[0] -= c.r1[d] * (v[d] - v[3 + d]);
+    xs[1] -= c.r2[d] * (v[d] - v[6 + d]);
+    xs[2] -= c.o[d] * v[d] + c.p[d] * v[3 + d] + c.q[d] * v[6 + d];
   }
-#pragma unroll
-  for (int a = 0; a < 3; a++)
-#pragma unroll
-    for (int b = a; b < 3; b++) {
-      double t = 0;
-#pragma unroll
-      for (int d = 0; d < 9; d++)
-        if (water_reach(a, d) && water_reach(b, d)) t += c.g[a][d] * sci0[b][d];
-      s[a][b] = s[b][a] = t;
-    }
+  water_matrix(c, c, im, s);
   if (!solve3(s, xs)) return;
+  water_shift(c, im, xs, dx);
 #pragma unroll
-  for (int a = 0; a < 3; a++)
-#pragma unroll
-    for (int d = 0; d < 9; d++)
-      if (water_reach(a, d)) v[d] += xs[a] * sci0[a][d];
+  for (int d = 0; d < 9; d++) v[d] += dx[d];
 }
 
 }  // namespace mmamd
