@@ -733,7 +733,7 @@ __global__ void __launch_bounds__(NP_TB) k_nonperiodic(const double4 *__restrict
     }
   }
   if (MODE == 0) {   // the block's LJ energy, reduced in a fixed order
-    for (int o = 32; o >= 1; o >>= 1) u += shfl_xor_d(u, o);
+    for (int o = 32; o >= 1; o >>= 1) u += __shfl_xor(u, o);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = u;
     __syncthreads();
     if (threadIdx.x == 0) {
