@@ -387,19 +387,28 @@ static int enqueue_forces(mm_engine *m, int field_mode, int want_virial,
   // its own buffers, so it runs on the second stream beside the
   // neighbour-list and pair kernels; the join comes before anything that
   // consumes it.
-  const bool fork = e.stream2 != nullptr;
+  const bool together = !e.external_nl && kspace_takes_list(e);
+  bool ksum = false;
+  for (auto &p : e.hsp) ksum |= p.kmode != 2;
+  const bool fork = e.stream2 != nullptr && ksum && !together;
   hipStream_t kst = e.stream;
   if (fork) {
     MM_HIP(hipEventRecord(e.ev_fork, e.stream));
     MM_HIP(hipStreamWaitEvent(e.stream2, e.ev_fork, 0));
     kst = e.stream2;
   }
-  TRY(launch_kspace(e, want_virial, kst, energy || want_virial));
-  TRY(launch_p3m(e, want_virial, kst, energy || want_virial));
+  if (!together) {
+    TRY(launch_kspace(e, want_virial, kst, energy || want_virial));
+    TRY(launch_p3m(e, want_virial, kst, energy || want_virial));
+  }
+  auto build = [&](int force, int from_partials) {
+    return together ? launch_kspace_list(e, want_virial, energy || want_virial, force, from_partials)
+                    : launch_nl_build(e, force, from_partials);
+  };
   if (e.external_nl) {
     e.first_eval = 0;
   } else if (e.first_eval) {
-    TRY(launch_nl_build(e, 1));
+    TRY(build(1, 0));
     e.first_eval = 0;
   } else {
     // new positions are packed together with their skin test; a rebuild packs
@@ -408,7 +417,7 @@ static int enqueue_forces(mm_engine *m, int field_mode, int want_virial,
       TRY(launch_skin_pack(e));
       e.need_pack = 0;
     }
-    TRY(launch_nl_build(e, 0, nl_from_partials || m->pos_dirty));
+    TRY(build(0, nl_from_partials || m->pos_dirty));
     m->pos_dirty = 0;
   }
   if (e.need_pack || m->pos_dirty) TRY(launch_pack(e));

@@ -266,6 +266,9 @@ void p3m_twiddles(const SysParams &P, std::vector<float2> &tw);
 
 // energies 0: the reciprocal-space energy (a diagnostic total) is not formed
 int launch_kspace(Engine &e, int want_virial, hipStream_t st, int energies = 1);
+// the Ewald sums with launch_nl_build's work in the same launches
+bool kspace_takes_list(const Engine &e);
+int launch_kspace_list(Engine &e, int want_virial, int energies, int force, int from_partials);
 int kspace_rows(double kc, std::vector<int4> &rows);
 int launch_p3m(Engine &e, int want_virial, hipStream_t st, int energies = 1);
 inline int launch_kspace(Engine &e, int want_virial) { return launch_kspace(e, want_virial, e.stream); }

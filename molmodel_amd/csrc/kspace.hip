@@ -23,6 +23,7 @@
 // (W_ab = sum a_k |rho_k|^2 (delta_ab - 2 k_a k_b (1/k^2 + 1/(4 eta^2))))
 // are formed by a block of its own beside the field kernel's.
 #include "engine.hpp"
+#include "nlist.hpp"
 
 namespace mmamd {
 
@@ -42,11 +43,17 @@ constexpr int SF_TB = 512;
 __global__ void __launch_bounds__(SF_TB) k_ks_sf(const SysParams *__restrict__ sp,
                                                const int4 *__restrict__ krow,
                                                const double *__restrict__ r, const double *__restrict__ q,
-                                               int N, double *__restrict__ ksc) {
+                                               int N, double *__restrict__ ksc, NlArgs nl, int nlb) {
   const int s = blockIdx.y;
   const SysParams &P = sp[s];
-  if (P.kmode != 0 || (int)blockIdx.x >= P.nkrow) return;
-  const KRow row(krow[P.krow0 + blockIdx.x]);
+  if ((int)blockIdx.x < nlb) {
+    extern __shared__ int cnt[];
+    if (blockIdx.z == 0) nl.bin<SF_TB>(P, s, cnt);
+    return;
+  }
+  const int rw = blockIdx.x - nlb;
+  if (P.kmode != 0 || rw >= P.nkrow) return;
+  const KRow row(krow[P.krow0 + rw]);
   const int z0 = blockIdx.z * KS_NZ;
   if (z0 > row.m) return;
   const double *B = P.RL;
@@ -121,22 +128,31 @@ constexpr int KS_MAXTAB = 31;   // largest |n| whose table fits beside the parti
 // Each team of 16 lanes (one per site) takes rows team, team + KS_SPLIT, ...;
 // the teams' sums are added in team order (deterministic).  TABLE false: wave
 // vectors beyond KS_MAXTAB, whose factors are formed where they are used.
-template <bool TABLE>
+// LIST: the first nlb blocks of a system carry a neighbour-list build's pair
+// search (16 wavefronts each); without it the kernel needs 69 registers
+// instead of 124, which leaves room on a CU for the pair kernel beside it.
+template <bool TABLE, bool LIST>
 __global__ void __launch_bounds__(KS_TB) k_ks_field(const SysParams *__restrict__ sp,
                                                     const double4 *__restrict__ kvec,
                                                     const int4 *__restrict__ krow,
                                                     const double *__restrict__ ksc,
                                                     const double *__restrict__ r, int N,
                                                     double *__restrict__ kres,
-                                                    double *__restrict__ acc, int want_virial) {
+                                                    double *__restrict__ acc, int want_virial,
+                                                    NlArgs nl, int nlb) {
   extern __shared__ double2 tab[];   // [axis][n][site]: (cos, sin)
   __shared__ double part[KS_SPLIT][4 * KS_SITES];
   const int s = blockIdx.y;
   const SysParams &P = sp[s];
+  if (LIST && (int)blockIdx.x < nlb) {
+    nl.pairs<KS_TB / 64>(P, s, blockIdx.x, nlb, (int *)tab);
+    return;
+  }
+  const int blk = blockIdx.x - nlb;
   if (P.kmode != 0) return;
   const int nblk = (P.nsite + KS_SITES - 1) / KS_SITES;
-  if ((int)blockIdx.x > nblk) return;
-  if ((int)blockIdx.x == nblk) {
+  if (blk > nblk) return;
+  if (blk == nblk) {
     if (!acc) return;
     // k-sum energy and virial of this system
     double e = 0, w[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
@@ -176,7 +192,7 @@ __global__ void __launch_bounds__(KS_TB) k_ks_field(const SysParams *__restrict_
     return;
   }
   const int site = threadIdx.x & (KS_SITES - 1), team = threadIdx.x / KS_SITES;
-  const int i = blockIdx.x * KS_SITES + site;
+  const int i = blk * KS_SITES + site;
   const int si = P.site0 + (i < P.nsite ? i : 0);
   const double *B = P.RL;
   double th[3];
@@ -249,7 +265,7 @@ __global__ void __launch_bounds__(KS_TB) k_ks_field(const SysParams *__restrict_
     double u = 0;
 #pragma unroll
     for (int k = 0; k < KS_TB / 64; k++) u += part[k][at];
-    const int c = at / KS_SITES, j = blockIdx.x * KS_SITES + (at & (KS_SITES - 1));
+    const int c = at / KS_SITES, j = blk * KS_SITES + (at & (KS_SITES - 1));
     if (j < P.nsite) kres[4L * (P.site0 + j) + c] = u;
   }
 }
@@ -272,27 +288,44 @@ int kspace_rows(double kc, std::vector<int4> &rows) {
   return nk;
 }
 
+// a neighbour-list build that goes along: nl null without one
+struct WithList {
+  const NlArgs *nl = nullptr;
+  int maxg = 0, maxc = 0;
+};
+
 static void launch_sf(dim3 rows_sys, int nm, hipStream_t st, const SysParams *sp,
-                      const int4 *krow, const double *r, const double *q, int N, double *ksc) {
+                      const int4 *krow, const double *r, const double *q, int N, double *ksc,
+                      const WithList &l = {}) {
+  const int nlb = l.nl ? 1 : 0;
+  rows_sys.x += nlb;
   rows_sys.z = nm / KS_NZ + 1;
-  hipLaunchKernelGGL(k_ks_sf, rows_sys, dim3(SF_TB), 0, st, sp, krow, r, q, N, ksc);
+  hipLaunchKernelGGL(k_ks_sf, rows_sys, dim3(SF_TB), sizeof(int) * l.maxc, st, sp, krow, r, q, N,
+                     ksc, l.nl ? *l.nl : NlArgs{}, nlb);
 }
 
 // acc null: energy and virial are not formed
 static void launch_field(int nsite, int nsys, int nm, hipStream_t st, const SysParams *sp,
                          const double4 *kvec, const int4 *krow, const double *ksc,
-                         const double *r, int N, double *kres, double *acc, int want_virial) {
-  const dim3 grid((nsite + KS_SITES - 1) / KS_SITES + (acc ? 1 : 0), nsys);
-  if (nm <= KS_MAXTAB)
-    hipLaunchKernelGGL(k_ks_field<true>, grid, dim3(KS_TB),
-                       sizeof(double2) * 3 * (nm + 1) * KS_SITES, st, sp, kvec, krow, ksc, r, N,
-                       kres, acc, want_virial);
-  else
-    hipLaunchKernelGGL(k_ks_field<false>, grid, dim3(KS_TB), 0, st, sp, kvec, krow, ksc, r, N,
-                       kres, acc, want_virial);
+                         const double *r, int N, double *kres, double *acc, int want_virial,
+                         const WithList &l = {}) {
+  constexpr int NW = KS_TB / 64;
+  const int nlb = (l.maxg + NW - 1) / NW;
+  const dim3 grid((nsite + KS_SITES - 1) / KS_SITES + (acc ? 1 : 0) + nlb, nsys);
+  const NlArgs a = l.nl ? *l.nl : NlArgs{};
+  const size_t list = nlb ? sizeof(int) * NL_LDS * NW : 0;
+  const size_t tab = nm <= KS_MAXTAB ? sizeof(double2) * 3 * (nm + 1) * KS_SITES : 0;
+#define FIELD(T, L)                                                                             \
+  hipLaunchKernelGGL((k_ks_field<T, L>), grid, dim3(KS_TB), std::max(tab, list), st, sp, kvec,  \
+                     krow, ksc, r, N, kres, acc, want_virial, a, nlb)
+  if (tab && nlb) FIELD(true, true);
+  else if (tab) FIELD(true, false);
+  else if (nlb) FIELD(false, true);
+  else FIELD(false, false);
+#undef FIELD
 }
 
-int launch_kspace(Engine &e, int want_virial, hipStream_t st, int energies) {
+static int launch_ewald(Engine &e, int want_virial, hipStream_t st, int energies, const WithList &l) {
   int maxrow = 0, maxn = 0, nm = 0;
   for (auto &p : e.hsp)
     if (p.kmode == 0) {
@@ -301,11 +334,40 @@ int launch_kspace(Engine &e, int want_virial, hipStream_t st, int energies) {
       nm = std::max(nm, p.nkmax);
     }
   if (maxrow == 0) return 0;
-  launch_sf(dim3(maxrow, e.nsys), nm, st, e.d_sp, e.d_krow, e.d_r, e.d_q, e.nsite, e.d_ksc);
+  launch_sf(dim3(maxrow, e.nsys), nm, st, e.d_sp, e.d_krow, e.d_r, e.d_q, e.nsite, e.d_ksc, l);
   launch_field(maxn, e.nsys, nm, st, e.d_sp, (const double4 *)e.d_kvec, e.d_krow, e.d_ksc, e.d_r,
-               e.nsite, e.d_kres, energies ? e.d_acc : nullptr, want_virial);
+               e.nsite, e.d_kres, energies ? e.d_acc : nullptr, want_virial, l);
   MM_HIP(hipGetLastError());
   return 0;
+}
+
+int launch_kspace(Engine &e, int want_virial, hipStream_t st, int energies) {
+  return launch_ewald(e, want_virial, st, energies, {});
+}
+
+// Small plain-Ewald engines: the two launches of a neighbour-list build, which
+// in most steps find nothing to do, ride in those of the reciprocal sum, and
+// everything stays on one stream.  A launch of its own costs 3 us whatever it
+// does, a fork to the second stream and back 10.  A step of 216 waters
+// 36.3 us forked, 36.3 in a line, 30.5 like this; 960 waters with ions 44.9,
+// 46.9 and 42.4.  Beyond PAIR_WIDE_GROUPS the pair kernel fills the chip and
+// the sums beside it are the longer part, so the fork pays.
+bool kspace_takes_list(const Engine &e) {
+  bool ewald = false;
+  for (auto &p : e.hsp) {
+    if (p.kmode == 1 || p.ncell * p.ncell * p.ncell > NL_BIN_CELLS) return false;
+    ewald |= p.kmode == 0 && p.nkrow > 0;
+  }
+  return ewald && e.pair_lanes == 64;
+}
+
+int launch_kspace_list(Engine &e, int want_virial, int energies, int force, int from_partials) {
+  NlArgs a;
+  WithList l;
+  if (int rc = nl_prepare(e, force, from_partials, a, l.maxc)) return rc;
+  l.nl = &a;
+  l.maxg = e.maxg;
+  return launch_ewald(e, want_virial, e.stream, energies, l);
 }
 
 // Structure factors and field of one system whose parameters, wave vectors,
