@@ -44,6 +44,7 @@ __global__ void __launch_bounds__(SF_TB) k_ks_sf(const SysParams *__restrict__ s
                                                const int4 *__restrict__ krow,
                                                const double *__restrict__ r, const double *__restrict__ q,
                                                int N, double *__restrict__ ksc, NlArgs nl, int nlb) {
+  before_pairs();
   const int s = blockIdx.y;
   const SysParams &P = sp[s];
   if ((int)blockIdx.x < nlb) {
@@ -140,6 +141,7 @@ __global__ void __launch_bounds__(KS_TB) k_ks_field(const SysParams *__restrict_
                                                     double *__restrict__ kres,
                                                     double *__restrict__ acc, int want_virial,
                                                     NlArgs nl, int nlb) {
+  before_pairs();
   extern __shared__ double2 tab[];   // [axis][n][site]: (cos, sin)
   __shared__ double part[KS_SPLIT][4 * KS_SITES];
   const int s = blockIdx.y;

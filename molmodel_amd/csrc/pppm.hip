@@ -108,6 +108,7 @@ __global__ void __launch_bounds__(256) k_p3m_bin(const SysParams *__restrict__ s
                                                  int4 *__restrict__ bgrid,
                                                  float4 *__restrict__ bfrac,
                                                  int *__restrict__ err, int *__restrict__ need) {
+  before_pairs();
   __shared__ int cnt[MAXBINS];
   const int s = blockIdx.y;
   const SysParams &P = sp[s];
@@ -209,6 +210,62 @@ struct ReachedSites {
   }
 };
 
+constexpr int FFT_MAXN = 128;
+// an axis' factors exp(-2 pi i t / n), and (pos) each frequency's place and
+// each place's signed frequency, from the system's tables (p3m_twiddles)
+__device__ __forceinline__ void load_tw(float2 *stw, const float2 *tw, int n) {
+  for (int t = threadIdx.x; t < n; t += blockDim.x) stw[t] = tw[t];
+}
+__device__ __forceinline__ void load_pos(int *pos, const float2 *tw, int n) {
+  for (int t = threadIdx.x; t < n; t += blockDim.x) pos[t] = __float_as_int(tw[3 * FFT_MAXN + t].x);
+}
+__device__ __forceinline__ void load_freq(short *f, const float2 *tw, int n) {
+  for (int t = threadIdx.x; t < n; t += blockDim.x)
+    f[t] = (short)__float_as_int(tw[3 * FFT_MAXN + t].y);
+}
+
+// half spectrum of two real lines a + i b from their transform at k and -k
+__device__ __forceinline__ float2 half_a(float2 zp, float2 zm) {
+  return make_float2(0.5f * (zp.x + zm.x), 0.5f * (zp.y - zm.y));
+}
+__device__ __forceinline__ float2 half_b(float2 zp, float2 zm) {
+  return make_float2(0.5f * (zp.y + zm.y), 0.5f * (zm.x - zp.x));
+}
+
+// A pulling block holds whole z lines, so it transforms them itself, where its
+// columns come in the pairs that k_fft_z makes one complex line of: an even
+// number of y columns a block and on the mesh.  (The bound keeps the LDS of a
+// block at 24 KB.)  One launch and a trip of the mesh through memory less, the
+// writes in runs of two columns: spreading and z pass of 12 288 sites on 48^3
+// took 7.0 and 5.7 us and take 9.5 together, of 98 304 on 64^3 17.2 and 7.0, now 20.3.
+constexpr int FUSE_POINTS = 2048;
+__host__ __device__ __forceinline__ bool spread_transforms(const SysParams &Q) {
+  return !(Q.by & 1) && !(Q.ny & 1) && Q.bx * Q.by * Q.nz <= FUSE_POINTS;
+}
+__device__ __forceinline__ void transform_columns(const SysParams &Q, const unsigned long long *acc,
+                                                  float2 *buf, const float2 *stw, const int *pos,
+                                                  int X0, int Y0, float2 *__restrict__ cmesh) {
+  const int nz = Q.nz, nzh = nz / 2 + 1, ls = nz | 1, nl = Q.bx * Q.by / 2, half = Q.by / 2;
+  float *fb = reinterpret_cast<float *>(buf);
+  const float inv = 1.f / (float)nz, inv_nl = 1.f / (float)nl, inv_half = 1.f / (float)half;
+  for (int t = threadIdx.x; t < 2 * nl * nz; t += blockDim.x) {
+    const int c = div_small(t, inv), z = t - c * nz;
+    fb[2 * ((c >> 1) * ls + z) + (c & 1)] = (float)((double)(long long)acc[t] * FIX_INV);
+  }
+  __syncthreads();
+  fft_forward(buf, nl, ls, 1, nz, Q.rad[2], stw);
+  float2 *dst = cmesh + Q.cmesh0 + (long)X0 * Q.ny + Y0;
+  const long plane = (long)Q.nx * Q.ny;
+  for (int t = threadIdx.x; t < nzh * nl; t += blockDim.x) {
+    const int k = div_small(t, inv_nl), l = t - k * nl;
+    const int ox = div_small(l, inv_half), oy = 2 * (l - ox * half);
+    const float2 zp = buf[l * ls + pos[k]], zm = buf[l * ls + pos[k ? nz - k : 0]];
+    float2 *o = dst + k * plane + ox * Q.ny + oy;
+    o[0] = half_a(zp, zm);
+    o[1] = half_b(zp, zm);
+  }
+}
+
 // the block's points out to the mesh
 __device__ __forceinline__ void store_columns(const SysParams &Q, const unsigned long long *acc,
                                               int X0, int Y0, float *__restrict__ mesh) {
@@ -274,17 +331,28 @@ __global__ void __launch_bounds__(256) k_p3m_spread(const SysParams *__restrict_
                                                     const int *__restrict__ fill, int bcap,
                                                     const int4 *__restrict__ bgrid,
                                                     const float4 *__restrict__ bfrac,
-                                                    float *__restrict__ mesh) {
+                                                    float *__restrict__ mesh,
+                                                    const float2 *__restrict__ twid_all,
+                                                    float2 *__restrict__ cmesh) {
+  before_pairs();
   extern __shared__ unsigned long long acc[];
   __shared__ ReachedSites reached;
   __shared__ float swx[P * 256], swy[P * 256];   // staged so that an offset can index them
+  __shared__ float2 stw[FFT_MAXN];
+  __shared__ int pos[FFT_MAXN];
   const int s = blockIdx.y;
   const SysParams &Q = sp[s];
   if (Q.kmode != 1 || Q.order != P) return;
   const int blk = blockIdx.x;
   if (blk >= Q.nbx * Q.nby) return;
   const int X0 = blk / Q.nby * Q.bx, Y0 = blk % Q.nby * Q.by;
-  for (int t = threadIdx.x; t < Q.bx * Q.by * Q.nz; t += blockDim.x) acc[t] = 0ull;
+  const int npts = Q.bx * Q.by * Q.nz;
+  for (int t = threadIdx.x; t < npts; t += blockDim.x) acc[t] = 0ull;
+  const bool z = spread_transforms(Q);
+  if (z) {
+    load_tw(stw, twid_all + Q.twid0 + 2 * FFT_MAXN, Q.nz);
+    load_pos(pos, twid_all + Q.twid0 + 2 * FFT_MAXN, Q.nz);
+  }
   reached.collect<P>(Q, X0, Y0, fill, bcap);
   const int total = reached.total();
   // a site is loaded while the one before it is spread
@@ -306,7 +374,8 @@ __global__ void __launch_bounds__(256) k_p3m_spread(const SysParams *__restrict_
     else spread_site<P, true>(Q, X0, Y0, g, f, wx, wy, acc);
   }
   __syncthreads();
-  store_columns(Q, acc, X0, Y0, mesh);
+  if (z) transform_columns(Q, acc, reinterpret_cast<float2 *>(acc + npts), stw, pos, X0, Y0, cmesh);
+  else store_columns(Q, acc, X0, Y0, mesh);
 }
 
 // The transpose of the gather's field instead of the charge: site i
@@ -393,6 +462,7 @@ __global__ void __launch_bounds__(512) k_p3m_spread_halo(const SysParams *__rest
                                                          const int4 *__restrict__ bgrid,
                                                          const float4 *__restrict__ bfrac,
                                                          unsigned long long *__restrict__ halo) {
+  before_pairs();
   extern __shared__ unsigned long long hacc[];
   const int s = blockIdx.y;
   const SysParams &Q = sp[s];
@@ -449,23 +519,9 @@ __global__ void __launch_bounds__(512) k_p3m_spread_halo(const SysParams *__rest
 // Half spectra are stored plane by plane, [kz][x][y], the influence function
 // likewise but with x and y in the digit-reversed order the forward
 // transforms leave (fft.hpp), so that its factors line up with the spectrum.
-constexpr int FFT_MAXN = 128;
 constexpr int FZ_LINES = 16;                 // complex lines per z block: 32 mesh lines
 constexpr int FZ_TB = 256;
 constexpr int FP_TB = 512;                   // plane block
-
-// an axis' factors exp(-2 pi i t / n), and (pos) each frequency's place and
-// each place's signed frequency, from the system's tables (p3m_twiddles)
-__device__ __forceinline__ void load_tw(float2 *stw, const float2 *tw, int n) {
-  for (int t = threadIdx.x; t < n; t += blockDim.x) stw[t] = tw[t];
-}
-__device__ __forceinline__ void load_pos(int *pos, const float2 *tw, int n) {
-  for (int t = threadIdx.x; t < n; t += blockDim.x) pos[t] = __float_as_int(tw[3 * FFT_MAXN + t].x);
-}
-__device__ __forceinline__ void load_freq(short *f, const float2 *tw, int n) {
-  for (int t = threadIdx.x; t < n; t += blockDim.x)
-    f[t] = (short)__float_as_int(tw[3 * FFT_MAXN + t].y);
-}
 
 // Mesh line `line` (column xi = line / ny, yi = line % ny) of a P3M system is
 // the sum of the spreading blocks' halo columns that cover it: halo column
@@ -531,11 +587,12 @@ template <bool HALO>
 __global__ void __launch_bounds__(FZ_TB) k_fft_z(
     const SysParams *__restrict__ sp, const float2 *__restrict__ twid_all,
     const float *__restrict__ mesh, float2 *__restrict__ cmesh,
-    const unsigned long long *__restrict__ halo) {
+    const unsigned long long *__restrict__ halo, int spread_does) {
+  before_pairs();
   __shared__ float2 buf[FZ_LINES * (FFT_MAXN + 1)], stw[FFT_MAXN];
   __shared__ int pos[FFT_MAXN];
   const SysParams &P = sp[blockIdx.y];
-  if (P.kmode != 1) return;
+  if (P.kmode != 1 || (spread_does && spread_transforms(P))) return;
   const int nz = P.nz, nzh = nz / 2 + 1, ls = nz | 1;
   const int nlines = P.nx * P.ny, l0 = blockIdx.x * 2 * FZ_LINES, nl = min(2 * FZ_LINES, nlines - l0);
   if (nl <= 0) return;
@@ -561,8 +618,8 @@ __global__ void __launch_bounds__(FZ_TB) k_fft_z(
     const int k = t / FZ_LINES, l = t % FZ_LINES;
     const float2 zp = buf[l * ls + pos[k]], zm = buf[l * ls + pos[k ? nz - k : 0]];
     float2 *o = dst + (long)k * nlines + 2 * l;
-    if (2 * l < nl) o[0] = make_float2(0.5f * (zp.x + zm.x), 0.5f * (zp.y - zm.y));
-    if (2 * l + 1 < nl) o[1] = make_float2(0.5f * (zp.y + zm.y), 0.5f * (zm.x - zp.x));
+    if (2 * l < nl) o[0] = half_a(zp, zm);
+    if (2 * l + 1 < nl) o[1] = half_b(zp, zm);
   }
 }
 
@@ -575,6 +632,7 @@ __global__ void __launch_bounds__(FZ_TB) k_fft_zinv(const SysParams *__restrict_
                                                     const float2 *__restrict__ twid_all,
                                                     const float2 *__restrict__ cmesh,
                                                     float *__restrict__ mesh) {
+  before_pairs();
   __shared__ float2 buf[FZ_LINES * (FFT_MAXN + 1)], stw[FFT_MAXN];
   __shared__ int pos[FFT_MAXN];
   const SysParams &P = sp[blockIdx.y];
@@ -702,6 +760,7 @@ __global__ void __launch_bounds__(FP_TB, (VIR || ENER) ? 4 : 8) k_fft_plane(cons
                                                         int *__restrict__ done,
                                                         double *__restrict__ acc,
                                                         double *__restrict__ kvir, int maxblk) {
+  before_pairs();
   extern __shared__ float2 plane[];
   __shared__ float2 twx[FFT_MAXN], twy[FFT_MAXN];
   __shared__ short fx[FFT_MAXN], fy[FFT_MAXN];
@@ -744,6 +803,7 @@ template <bool INV>
 __global__ void __launch_bounds__(FL_TB, 4) k_fft_y(const SysParams *__restrict__ sp,
                                                     const float2 *__restrict__ twid_all,
                                                     float2 *__restrict__ cmesh) {
+  before_pairs();
   __shared__ float2 buf[FL_LINES * (FFT_MAXN + 1)], twy[FFT_MAXN];
   const SysParams &P = sp[blockIdx.y];
   if (P.kmode != 1 || P.plane) return;
@@ -772,6 +832,7 @@ __global__ void __launch_bounds__(FL_TB, 4) k_fft_x(const SysParams *__restrict_
                                                     int *__restrict__ done,
                                                     double *__restrict__ acc,
                                                     double *__restrict__ kvir, int maxblk) {
+  before_pairs();
   constexpr int LS = FL_LINES + 1;
   __shared__ float2 buf[LS * FFT_MAXN], twx[FFT_MAXN];
   __shared__ short fx[FFT_MAXN], fy[FFT_MAXN];
@@ -868,6 +929,7 @@ __global__ void __launch_bounds__(256, 4) k_p3m_gather(const SysParams *__restri
                                                     const float *__restrict__ mesh,
                                                     double *__restrict__ kres,
                                                     int *__restrict__ fill) {
+  before_pairs();
   const int s = blockIdx.y;
   const SysParams &Q = sp[s];
   if (Q.kmode != 1 || Q.order != P || Q.ik != (int)IK) return;
@@ -981,20 +1043,22 @@ static void launch_planes(Engine &e, hipStream_t st, const SysParams *sp, const 
 }
 
 static void launch_fft(Engine &e, int want_virial, int energies, hipStream_t st, const SysParams *sp,
-                       const SysParams *hp, int nsg, const unsigned long long *halo) {
+                       const SysParams *hp, int nsg, const unsigned long long *halo,
+                       bool spread_does) {
   int nz = 0;
-  bool ik = false;
+  bool ik = false, left = false;   // left: z lines that the spreading did not transform
   for (int s = 0; s < nsg; s++)
     if (hp[s].kmode == 1) {
+      left |= !(spread_does && spread_transforms(hp[s]));
       nz = std::max(nz, (hp[s].nx * hp[s].ny + 2 * FZ_LINES - 1) / (2 * FZ_LINES));
       ik |= hp[s].ik != 0;
     }
   if (halo)
     hipLaunchKernelGGL(k_fft_z<true>, dim3(nz, nsg), dim3(FZ_TB), 0, st, sp, e.d_twid, e.d_mesh,
-                       e.d_cmesh, halo);
-  else
+                       e.d_cmesh, halo, 0);
+  else if (left)
     hipLaunchKernelGGL(k_fft_z<false>, dim3(nz, nsg), dim3(FZ_TB), 0, st, sp, e.d_twid, e.d_mesh,
-                       e.d_cmesh, halo);
+                       e.d_cmesh, halo, spread_does ? 1 : 0);
 #define PLANES(V, E)                                             \
   if (ik) launch_planes<V, E, true>(e, st, sp, hp, nsg);         \
   else launch_planes<V, E, false>(e, st, sp, hp, nsg);
@@ -1004,6 +1068,11 @@ static void launch_fft(Engine &e, int want_virial, int energies, hipStream_t st,
 #undef PLANES
   hipLaunchKernelGGL(k_fft_zinv, dim3(nz, nsg, ik ? 4 : 1), dim3(FZ_TB), 0, st, sp, e.d_twid,
                      e.d_cmesh, e.d_mesh);
+}
+
+// LDS of a pulling block's complex lines
+static size_t pull_lines(const SysParams &p) {
+  return spread_transforms(p) ? sizeof(float2) * p.bx * p.by / 2 * (p.nz | 1) : 0;
 }
 
 int launch_p3m(Engine &e, int want_virial, hipStream_t st, int energies) {
@@ -1034,7 +1103,8 @@ int launch_p3m(Engine &e, int want_virial, hipStream_t st, int energies) {
     if (p.kmode == 1)
       hbytes[p.order] = std::max(hbytes[p.order], sizeof(unsigned long long) * p.nz *
                                                       (p.bx + h * (p.order - 1)) *
-                                                      (p.by + h * (p.order - 1)));
+                                                      (p.by + h * (p.order - 1)) +
+                                                      (h ? 0 : pull_lines(p)));
   for (auto &p : e.hsp)
     if (p.kmode == 1 && (long)p.nsite * p.order > 384L * p.nbx * p.nby) htb = 512;
 #define SPREAD(PO)                                                                           \
@@ -1043,11 +1113,12 @@ int launch_p3m(Engine &e, int want_virial, hipStream_t st, int energies) {
                        st, e.d_sp, e.d_bin_fill, e.bcap, e.d_bgrid, e.d_bfrac, e.d_halo);     \
   else if (used[PO])                                                                         \
     hipLaunchKernelGGL(k_p3m_spread<PO>, dim3(maxbins, e.nsys), dim3(256), hbytes[PO], st,    \
-                       e.d_sp, e.d_bin_fill, e.bcap, e.d_bgrid, e.d_bfrac, e.d_mesh);
+                       e.d_sp, e.d_bin_fill, e.bcap, e.d_bgrid, e.d_bfrac, e.d_mesh, e.d_twid,  \
+                       e.d_cmesh);
   SPREAD(1) SPREAD(2) SPREAD(3) SPREAD(4) SPREAD(5) SPREAD(6) SPREAD(7)
 #undef SPREAD
   launch_fft(e, want_virial, energies, st, e.d_sp, e.hsp.data(), e.nsys,
-             e.spread_halo ? e.d_halo : nullptr);
+             e.spread_halo ? e.d_halo : nullptr, !e.spread_halo);
 #define GATHER(PO)                                                                        \
   if (used_ad[PO])                                                                        \
     hipLaunchKernelGGL(k_p3m_gather<PO>, gs, dim3(tb), 0, st, e.d_sp, e.d_sgrid,     \
@@ -1088,7 +1159,7 @@ int launch_p3m_adjoint(Engine &e, int sys, const float4 *src, hipStream_t st) {
     default: set_last_error("assignment order out of range"); return -1;
   }
 #undef ADJ_ORDER
-  launch_fft(e, 0, 0, st, sp, &P, 1, nullptr);
+  launch_fft(e, 0, 0, st, sp, &P, 1, nullptr, false);
 #define ADJ_GATHER(PO)                                                                      \
   case PO:                                                                                  \
     hipLaunchKernelGGL(k_p3m_gather<PO>, gs, dim3(tb), 0, st, sp, e.d_sgrid, e.d_sfrac,     \
@@ -1120,18 +1191,18 @@ int launch_p3m_ik_pass(Engine &e, int sys, const double *q, hipStream_t st) {
                      e.d_sfrac, e.d_bin_fill, e.bcap, e.d_bgrid, e.d_bfrac, e.d_err,
                      e.d_bin_fill + e.nbin_total);
   const dim3 gb(P.nbx * P.nby, 1);
-  const size_t blds = sizeof(unsigned long long) * P.bx * P.by * P.nz;
+  const size_t blds = sizeof(unsigned long long) * P.bx * P.by * P.nz + pull_lines(P);
 #define IK_SPREAD(PO)                                                                        \
   case PO:                                                                                   \
     hipLaunchKernelGGL(k_p3m_spread<PO>, gb, dim3(256), blds, st, sp, e.d_bin_fill, e.bcap,  \
-                       e.d_bgrid, e.d_bfrac, e.d_mesh);                                      \
+                       e.d_bgrid, e.d_bfrac, e.d_mesh, e.d_twid, e.d_cmesh);                  \
     break;
   switch (P.order) {
     IK_SPREAD(1) IK_SPREAD(2) IK_SPREAD(3) IK_SPREAD(4) IK_SPREAD(5) IK_SPREAD(6) IK_SPREAD(7)
     default: set_last_error("assignment order out of range"); return -1;
   }
 #undef IK_SPREAD
-  launch_fft(e, 0, 0, st, sp, &P, 1, nullptr);
+  launch_fft(e, 0, 0, st, sp, &P, 1, nullptr, true);
 #define IK_GATHER(PO)                                                                       \
   case PO:                                                                                  \
     hipLaunchKernelGGL((k_p3m_gather<PO, true>), gs, dim3(tb), 0, st, sp, e.d_sgrid,        \

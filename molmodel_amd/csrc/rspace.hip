@@ -471,7 +471,9 @@ __global__ void __launch_bounds__(PAIR_TB, (FIELD || VIRIAL) ? 1 : 4) k_pair(
     const int2 *__restrict__ gmeta, const int *__restrict__ nbr, const int *__restrict__ nnb,
     int nbcap, const float4 *__restrict__ tab, const float2 *__restrict__ ljt,
     double *__restrict__ pf, double *__restrict__ plj, double *__restrict__ gacc) {
-  __shared__ float4 stab[MAXTAB];
+  // the largest table of the engine's systems (10 KB less than room for any:
+  // three of these blocks then leave a CU room for a 64 x 64 plane transform)
+  extern __shared__ float4 stab[];
   __shared__ float2 slj[MAXLJ];
   // per i-group one batch and a fill: Dx, Dy, Dz, switching value; switching
   // derivative, neighbour (int bits)
@@ -808,6 +810,9 @@ int pair_tiles(int ngroup, int lanes) {
 int launch_pair(Engine &e, int field_mode, int want_virial, int energy) {
   if (e.ntile == 0) return 0;
   dim3 grid(e.pair_blocks), tb(PAIR_TB);
+  int ntab = 0;
+  for (auto &p : e.hsp) ntab = std::max(ntab, p.ntabA + p.ntabB);
+  const size_t lds = sizeof(float4) * ntab;
 #define PAIR_ARGS                                                                             \
   e.d_sp, e.d_tile_start, e.nsys, e.ntile, e.d_gpos, e.d_spk, e.d_gmeta, e.d_nbr, e.d_nnb,  \
       e.nbcap, e.d_tab, e.d_ljt, e.d_pf, e.d_plj, e.d_gacc
@@ -816,9 +821,9 @@ int launch_pair(Engine &e, int field_mode, int want_virial, int energy) {
   // ENERGY false (forces only) for steps whose energies nobody reads
 #define PAIR_LANES(F, V, EN, L)                                                              \
   if (e.any_water)                                                                           \
-    hipLaunchKernelGGL((k_pair<F, V, true, EN, L>), grid, tb, 0, e.stream, PAIR_ARGS);       \
+    hipLaunchKernelGGL((k_pair<F, V, true, EN, L>), grid, tb, lds, e.stream, PAIR_ARGS);     \
   else                                                                                       \
-    hipLaunchKernelGGL((k_pair<F, V, false, EN, L>), grid, tb, 0, e.stream, PAIR_ARGS);
+    hipLaunchKernelGGL((k_pair<F, V, false, EN, L>), grid, tb, lds, e.stream, PAIR_ARGS);
 #define PAIR_LAUNCH(F, V, EN)                                                                \
   if (e.pair_lanes == 64) { PAIR_LANES(F, V, EN, 64) } else { PAIR_LANES(F, V, EN, 16) }
   if (field_mode) {
