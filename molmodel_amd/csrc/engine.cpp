@@ -694,6 +694,15 @@ int engine_create(Engine &e, const std::vector<SystemInput> &in) {
   const char *serial = getenv("MOLMODEL_AMD_SERIAL_KSPACE");
   if (!(serial && serial[0] == '1'))
     MM_HIP(hipStreamCreateWithFlags(&e.stream2, hipStreamNonBlocking));
+  bool ewald = false, mesh = false;
+  for (auto &p : e.hsp) {
+    ewald |= p.kmode == 0;
+    mesh |= p.kmode == 1;
+  }
+  if (e.stream2 && ewald && mesh) {
+    MM_HIP(hipStreamCreateWithFlags(&e.stream3, hipStreamNonBlocking));
+    MM_HIP(hipEventCreateWithFlags(&e.ev_join3, hipEventDisableTiming));
+  }
   MM_HIP(hipEventCreateWithFlags(&e.ev_fork, hipEventDisableTiming));
   MM_HIP(hipEventCreateWithFlags(&e.ev_join, hipEventDisableTiming));
   MM_TRY(dalloc(&e.d_sp, e.nsys));
@@ -985,8 +994,10 @@ void engine_destroy(Engine &e) {
     if (p) hipFree(p);
   if (e.stream) hipStreamDestroy(e.stream);
   if (e.stream2) hipStreamDestroy(e.stream2);
+  if (e.stream3) hipStreamDestroy(e.stream3);
   if (e.ev_fork) hipEventDestroy(e.ev_fork);
   if (e.ev_join) hipEventDestroy(e.ev_join);
+  if (e.ev_join3) hipEventDestroy(e.ev_join3);
   e = Engine();
 }
 

@@ -68,9 +68,10 @@ struct Engine {
   std::vector<double> lj_tail;   // per system (host FP64)
   hipStream_t stream = nullptr;
   // second stream for the reciprocal-space branch of a force evaluation
-  // (forked from and joined back into `stream` with the two events)
-  hipStream_t stream2 = nullptr;
-  hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+  // (forked from and joined back into `stream` with the two events); a third
+  // for the plain-Ewald sums of engines that have P3M systems too
+  hipStream_t stream2 = nullptr, stream3 = nullptr;
+  hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_join3 = nullptr;
   std::shared_ptr<Stage> stage = std::make_shared<Stage>();
 
   SysParams *d_sp = nullptr;
