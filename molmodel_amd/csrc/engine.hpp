@@ -289,7 +289,7 @@ int launch_nonperiodic_points(const double4 *site, const double *rscreen, int n,
 // k-space structure factors and field of one system in buffers the caller
 // provides (kspace.hip)
 int launch_kspace_raw(const SysParams *sp, const double4 *kvec, const int4 *krow, int nkrow,
-                      int nm, int nsite, const double *r, const double *q, double *ksc,
+                      int nm, int nk, int nsite, const double *r, const double *q, double *ksc,
                       double *kres, hipStream_t st);
 // adjoint passes of one system (adjoint.hip, kspace.hip, pppm.hip)
 int launch_kspace_field_only(Engine &e, int sys, const double *ksc, double *kres_out);

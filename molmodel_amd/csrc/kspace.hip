@@ -17,8 +17,10 @@
 //               and wave vector), 3 120 sites: 10.2 (12.2)
 //   k_ks_field  a block serves 16 sites and its 64 16-lane teams take a row
 //               each; the sites' e^{i n b.r} for every n are formed once, in
-//               LDS; 7.9 us for 648 and for 3 120 sites (38 with 16 waves
-//               that walk the wave vectors with a sincos each, 64 sites a block)
+//               LDS, and so are the wave vectors' coefficients; 6.5 us for 648
+//               and for 2 920 sites (8.7 and 8.2 with the coefficients read from
+//               memory in the loop, 38 with 16 waves that walk the wave vectors
+//               with a sincos each, 64 sites a block)
 // The k-sum energy and virial
 // (W_ab = sum a_k |rho_k|^2 (delta_ab - 2 k_a k_b (1/k^2 + 1/(4 eta^2))))
 // are formed by a block of its own beside the field kernel's.
@@ -125,6 +127,9 @@ __global__ void __launch_bounds__(SF_TB) k_ks_sf(const SysParams *__restrict__ s
 
 constexpr int KS_SITES = 16, KS_SPLIT = 64, KS_TB = KS_SITES * KS_SPLIT;
 constexpr int KS_MAXTAB = 31;   // largest |n| whose table fits beside the partial sums
+// wave vectors whose coefficients 2 a_k (S, C) a block keeps in LDS: read from
+// memory inside the loop over nz, each cost its trip there one after the other
+constexpr int KS_STAGE = 1536;
 
 // Each team of 16 lanes (one per site) takes rows team, team + KS_SPLIT, ...;
 // the teams' sums are added in team order (deterministic).  TABLE false: wave
@@ -204,6 +209,14 @@ __global__ void __launch_bounds__(KS_TB) k_ks_field(const SysParams *__restrict_
     for (int a = 0; a < 3; a++) th[a] = B[3 * a] * x + B[3 * a + 1] * y + B[3 * a + 2] * z;
   }
   const int nm = P.nkmax;
+  double2 *coef = tab + (TABLE ? 3 * (nm + 1) * KS_SITES : 0);
+  const bool staged = P.nk <= KS_STAGE;
+  auto form = [&](int k) {
+    const double a = 2 * kvec[P.k0 + k].w;
+    return make_double2(a * ksc[2 * (P.k0 + k)], a * ksc[2 * (P.k0 + k) + 1]);
+  };
+  if (staged)
+    for (int k = threadIdx.x; k < P.nk; k += KS_TB) coef[k] = form(k);
   if (TABLE) {
     for (int t = team; t < 3 * (nm + 1); t += KS_SPLIT) {
       const int a = t / (nm + 1), n = t - a * (nm + 1);
@@ -211,8 +224,8 @@ __global__ void __launch_bounds__(KS_TB) k_ks_field(const SysParams *__restrict_
       sincos(n * (a == 0 ? th[0] : a == 1 ? th[1] : th[2]), &sn, &cs);
       tab[t * KS_SITES + site] = make_double2(cs, sn);
     }
-    __syncthreads();
   }
+  if (TABLE || staged) __syncthreads();
   auto factor = [&](int a, int n) {
     if (TABLE) return tab[(a * (nm + 1) + n) * KS_SITES + site];
     double2 f;
@@ -231,19 +244,19 @@ __global__ void __launch_bounds__(KS_TB) k_ks_field(const SysParams *__restrict_
     for (int nz = first; nz <= row.m; nz++) {
       const double2 ez = factor(2, nz);
       const double cc = xc * ez.x, ss = xs * ez.y, sc = xs * ez.x, cs = xc * ez.y;
-      const int kp = P.k0 + row.at(nz);
-      const double ap = 2 * kvec[kp].w, Sp = ksc[2 * kp], Cp = ksc[2 * kp + 1];
+      const int kp = row.at(nz);
+      const double2 ap = staged ? coef[kp] : form(kp);
       const double snp = sc + cs, csp = cc - ss;
-      double t = ap * (Cp * snp - Sp * csp);
-      p += ap * (Sp * snp + Cp * csp);
+      double t = ap.y * snp - ap.x * csp;
+      p += ap.x * snp + ap.y * csp;
       t0 += t;
       g3 += nz * t;
       if (!row.half && nz > 0) {
-        const int km = P.k0 + row.at(-nz);
-        const double am = 2 * kvec[km].w, Sm = ksc[2 * km], Cm = ksc[2 * km + 1];
+        const int km = row.at(-nz);
+        const double2 am = staged ? coef[km] : form(km);
         const double snm = sc - cs, csm = cc + ss;
-        t = am * (Cm * snm - Sm * csm);
-        p += am * (Sm * snm + Cm * csm);
+        t = am.y * snm - am.x * csm;
+        p += am.x * snm + am.y * csm;
         t0 += t;
         g3 -= nz * t;
       }
@@ -306,8 +319,10 @@ static void launch_sf(dim3 rows_sys, int nm, hipStream_t st, const SysParams *sp
                      ksc, l.nl ? *l.nl : NlArgs{}, nlb);
 }
 
-// acc null: energy and virial are not formed
-static void launch_field(int nsite, int nsys, int nm, hipStream_t st, const SysParams *sp,
+static int staged_nk(int nk) { return nk <= KS_STAGE ? nk : 0; }
+
+// acc null: energy and virial are not formed; nk: wave vectors to stage
+static void launch_field(int nsite, int nsys, int nm, int nk, hipStream_t st, const SysParams *sp,
                          const double4 *kvec, const int4 *krow, const double *ksc,
                          const double *r, int N, double *kres, double *acc, int want_virial,
                          const WithList &l = {}) {
@@ -316,9 +331,10 @@ static void launch_field(int nsite, int nsys, int nm, hipStream_t st, const SysP
   const dim3 grid((nsite + KS_SITES - 1) / KS_SITES + (acc ? 1 : 0) + nlb, nsys);
   const NlArgs a = l.nl ? *l.nl : NlArgs{};
   const size_t list = nlb ? sizeof(int) * NL_LDS * NW : 0;
-  const size_t tab = nm <= KS_MAXTAB ? sizeof(double2) * 3 * (nm + 1) * KS_SITES : 0;
+  const bool tab = nm <= KS_MAXTAB;
+  const size_t lds = std::max(list, sizeof(double2) * ((tab ? 3 * (nm + 1) * KS_SITES : 0) + nk));
 #define FIELD(T, L)                                                                             \
-  hipLaunchKernelGGL((k_ks_field<T, L>), grid, dim3(KS_TB), std::max(tab, list), st, sp, kvec,  \
+  hipLaunchKernelGGL((k_ks_field<T, L>), grid, dim3(KS_TB), lds, st, sp, kvec,                  \
                      krow, ksc, r, N, kres, acc, want_virial, a, nlb)
   if (tab && nlb) FIELD(true, true);
   else if (tab) FIELD(true, false);
@@ -328,16 +344,17 @@ static void launch_field(int nsite, int nsys, int nm, hipStream_t st, const SysP
 }
 
 static int launch_ewald(Engine &e, int want_virial, hipStream_t st, int energies, const WithList &l) {
-  int maxrow = 0, maxn = 0, nm = 0;
+  int maxrow = 0, maxn = 0, nm = 0, nk = 0;   // nk: the most that a block stages
   for (auto &p : e.hsp)
     if (p.kmode == 0) {
       maxrow = std::max(maxrow, p.nkrow);
       maxn = std::max(maxn, p.nsite);
       nm = std::max(nm, p.nkmax);
+      nk = std::max(nk, staged_nk(p.nk));
     }
   if (maxrow == 0) return 0;
   launch_sf(dim3(maxrow, e.nsys), nm, st, e.d_sp, e.d_krow, e.d_r, e.d_q, e.nsite, e.d_ksc, l);
-  launch_field(maxn, e.nsys, nm, st, e.d_sp, (const double4 *)e.d_kvec, e.d_krow, e.d_ksc, e.d_r,
+  launch_field(maxn, e.nsys, nm, nk, st, e.d_sp, (const double4 *)e.d_kvec, e.d_krow, e.d_ksc, e.d_r,
                e.nsite, e.d_kres, energies ? e.d_acc : nullptr, want_virial, l);
   MM_HIP(hipGetLastError());
   return 0;
@@ -350,10 +367,11 @@ int launch_kspace(Engine &e, int want_virial, hipStream_t st, int energies) {
 // Small plain-Ewald engines: the two launches of a neighbour-list build, which
 // in most steps find nothing to do, ride in those of the reciprocal sum, and
 // everything stays on one stream.  A launch of its own costs 3 us whatever it
-// does, a fork to the second stream and back 10.  A step of 216 waters
-// 36.3 us forked, 36.3 in a line, 30.5 like this; 960 waters with ions 44.9,
-// 46.9 and 42.4.  Beyond PAIR_WIDE_GROUPS the pair kernel fills the chip and
-// the sums beside it are the longer part, so the fork pays.
+// does, a fork to the second stream and back 10.  A step of 216 waters took
+// 36.3 us forked, 36.3 in a line and 30.5 like this, 960 waters with ions
+// 44.9, 46.9 and 42.4 (28.4 and 40.0 with the field's coefficients in LDS).
+// Beyond PAIR_WIDE_GROUPS the pair kernel fills the chip and the sums beside
+// it are the longer part, so the fork pays.
 bool kspace_takes_list(const Engine &e) {
   bool ewald = false;
   for (auto &p : e.hsp) {
@@ -377,10 +395,10 @@ int launch_kspace_list(Engine &e, int want_virial, int energies, int force, int 
 // caller provides (kspace_field_noalloc keeps them in its own device array):
 // ksc 2 nk, kres 4 nsite.
 int launch_kspace_raw(const SysParams *sp, const double4 *kvec, const int4 *krow, int nkrow,
-                      int nm, int nsite, const double *r, const double *q, double *ksc,
+                      int nm, int nk, int nsite, const double *r, const double *q, double *ksc,
                       double *kres, hipStream_t st) {
   launch_sf(dim3(nkrow, 1), nm, st, sp, krow, r, q, nsite, ksc);
-  launch_field(nsite, 1, nm, st, sp, kvec, krow, ksc, r, nsite, kres, nullptr, 0);
+  launch_field(nsite, 1, nm, staged_nk(nk), st, sp, kvec, krow, ksc, r, nsite, kres, nullptr, 0);
   MM_HIP(hipGetLastError());
   return 0;
 }
@@ -390,7 +408,7 @@ int launch_kspace_raw(const SysParams *sp, const double4 *kvec, const int4 *krow
 int launch_kspace_field_only(Engine &e, int sys, const double *ksc, double *kres_out) {
   const SysParams &P = e.hsp[sys];
   if (P.kmode != 0) return 0;
-  launch_field(P.nsite, 1, P.nkmax, e.stream, e.d_sp + sys, (const double4 *)e.d_kvec, e.d_krow,
+  launch_field(P.nsite, 1, P.nkmax, staged_nk(P.nk), e.stream, e.d_sp + sys, (const double4 *)e.d_kvec, e.d_krow,
                ksc, e.d_r, e.nsite, kres_out, nullptr, 0);
   MM_HIP(hipGetLastError());
   return 0;

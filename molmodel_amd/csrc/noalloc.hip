@@ -208,7 +208,7 @@ extern "C" int kspace_field_noalloc(double cutoff, int nsite, const cart_t *r, c
   const SysParams *dsp = reinterpret_cast<const SysParams *>(sc + NA_SP);
   const double4 *kv = reinterpret_cast<const double4 *>(sc + NA_KVEC);
   const int4 *krow = reinterpret_cast<const int4 *>(sc + NA_ROW);
-  if (int rc = launch_kspace_raw(dsp, kv, krow, P.nkrow, P.nkmax, nsite, sc + NA_R, q,
+  if (int rc = launch_kspace_raw(dsp, kv, krow, P.nkrow, P.nkmax, P.nk, nsite, sc + NA_R, q,
                                  sc + NA_KSC, sc + NA_KRES, st))
     return rc;
   hipLaunchKernelGGL(k_na_out, dim3((nsite + 255) / 256), dim3(256), 0, st, sc, nsite, phi,
