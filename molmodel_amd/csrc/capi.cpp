@@ -374,7 +374,7 @@ static int restore_state(Engine &e, int remd) {
 
 // nl_from_partials: the last finish left per-block partial sums (FIN_LAZY);
 // energy 0: an inner MD step, whose energies nobody reads: the pair kernel
-// and the P3M x pass form forces only
+// and the P3M planes form forces only
 static int enqueue_forces(mm_engine *m, int field_mode, int want_virial,
                           int nl_from_partials = 0, int energy = 1) {
   Engine &e = m->e;

@@ -19,13 +19,14 @@
 //            reaches, the halos cost their traffic, so columns holding many
 //            sites favour pulling and few sites the halos;
 //   fft      in-place mixed-radix line FFTs in LDS (fft.hpp): z (real to half
-//            spectrum), then per kz plane y and x forward, the influence
+//            spectrum; by the pulling blocks themselves where their columns
+//            come in pairs), then per kz plane y and x forward, the influence
 //            function (and the mesh energy/virial), x and y inverse, then z
 //            (half spectrum to real), unnormalised like FFTW;
 //   gather   phi_i = sum w phi_m and, with real-space differentiation (the
 //            reference default), E_i = (diag(n) L^-1)^T (sum -dw phi_m)
 //            (pppm.c:603-640); with the field formed on the mesh (ik), the
-//            x pass also forms E_a = -i k_a phi_k, the inverse passes run
+//            planes also form E_a = -i k_a phi_k, the inverse z pass runs
 //            over four components and E_i = sum w E_m (pppm.c:577-626).
 // Assignment weights are the cardinal B-splines that the reference's
 // polynomial tables tabulate (pppm.c:69-275), evaluated by recursion in FP32.
