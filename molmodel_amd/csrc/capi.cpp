@@ -657,6 +657,7 @@ int mm_nlist_update(mm_nlist *nl, const double *r) {
     TRY(read_err(e, &f));
     if (f & (ERR_NAN | ERR_CELL)) {
       TRY(clear_err(e));
+      after_position_error(e, f);
       set_last_error(f & ERR_NAN ? "mm_nlist_update: non-finite (or out-of-range) position"
                                  : "mm_nlist_update: positions collapsed, a cell is overfull");
       return MM_ERR_DEVICE;

@@ -76,19 +76,22 @@ __global__ void __launch_bounds__(256) k_nl_assign(
   if (!lastblk) return;
   __threadfence();
   if (threadIdx.x == 0) done[s] = 0;
-  block_scan_clear(cell_count + P.cell0, cell_start + P.cell0, P.ncell * P.ncell * P.ncell, P.group0);
+  if (block_scan_clear(cell_count + P.cell0, cell_start + P.cell0, P.ncell * P.ncell * P.ncell,
+                       P.group0, NL_SORT_MAX))
+    atomicOr(err, ERR_CELL);   // collapsed positions: reported, not sorted
 }
 
 // The groups of each cell from its list, in ascending order, one thread per
 // cell; the lists are cleared for the next build.  After a non-finite
-// position (its group parked in cell 0) or in a collapsed cell the list is
-// not walked: the rows of an error are discarded, and the slots keep the
-// order of the last build.
+// position (its group parked in cell 0) or a collapsed cell no list is
+// walked: the rows of an error are discarded, and the slots keep the order of
+// the last build, so that every group has one whatever was reported (the next
+// skin test walks them).
 __global__ void k_nl_order(const SysParams *__restrict__ sp, const int *__restrict__ rebuild,
                            const int *__restrict__ cell_start, int *__restrict__ head,
                            const int *__restrict__ next, int *__restrict__ order,
                            const double *__restrict__ last, double4 *__restrict__ gpos,
-                           int *__restrict__ err) {
+                           const int *__restrict__ err) {
   const int s = blockIdx.y;
   if (!rebuild[s]) return;
   const SysParams &P = sp[s];
@@ -96,12 +99,8 @@ __global__ void k_nl_order(const SysParams *__restrict__ sp, const int *__restri
   if (c >= P.ncell * P.ncell * P.ncell) return;
   int g = head[P.cell0 + c];
   head[P.cell0 + c] = -1;
-  if (__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & ERR_NAN) return;
+  if (__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & (ERR_NAN | ERR_CELL)) return;
   const int b = cell_start[P.cell0 + c], n = cell_start[P.cell0 + c + 1] - b;
-  if (n > NL_SORT_MAX) {   // collapsed positions: reported, not sorted
-    atomicOr(err, ERR_CELL);
-    return;
-  }
   int v[NL_CELL_REGS];
   if (n <= NL_CELL_REGS) {
 #pragma unroll
