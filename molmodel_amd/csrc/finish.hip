@@ -146,8 +146,11 @@ __global__ void __launch_bounds__(FIN_TB) k_finish(
             D[p][d] = x[k][d] - x[l][d];
             D[p][d] -= L * floor(D[p][d] * invL + 0.5);
           }
+          // two sites at one point are 0/0 (rspace.c:506-512) and refused as
+          // such (ERR_NAN), though the series has a limit there
+          const double r2 = D[p][0] * D[p][0] + D[p][1] * D[p][1] + D[p][2] * D[p][2];
           on[p] = (ex >> (k * MAXS + l)) & 1;
-          y[p] = on[p] ? eta2 * (D[p][0] * D[p][0] + D[p][1] * D[p][1] + D[p][2] * D[p][2]) : 0.0;
+          y[p] = !on[p] ? 0.0 : r2 > 0 ? eta2 * r2 : __builtin_nan("");
           if (y[p] > EXCL_Y) far = true;
         }
       double b0[K], b1[K];
