@@ -270,7 +270,10 @@ int launch_kspace(Engine &e, int want_virial, hipStream_t st, int energies = 1);
 // the Ewald sums with launch_nl_build's work in the same launches
 bool kspace_takes_list(const Engine &e);
 int launch_kspace_list(Engine &e, int want_virial, int energies, int force, int from_partials);
+// the rows of wave vectors up to kc, and their number alone; both return the
+// number of wave vectors
 int kspace_rows(double kc, std::vector<int4> &rows);
+int kspace_count(double kc, int &nrow);
 int launch_p3m(Engine &e, int want_virial, hipStream_t st, int energies = 1);
 // The reciprocal-space kernels are a chain that runs beside the pair kernel,
 // which fills every SIMD's issue slots: theirs come first.  (A step of 2900

@@ -285,9 +285,10 @@ __global__ void __launch_bounds__(KS_TB) k_ks_field(const SysParams *__restrict_
   }
 }
 
-// the rows of |n| <= kc (kspace.c:35-58), in the lexicographic order of the
-// wave vectors; returns the number of wave vectors
-int kspace_rows(double kc, std::vector<int4> &rows) {
+// f(first wave vector, nx, ny, largest |nz|) for the rows of |n| <= kc
+// (kspace.c:35-58), in the lexicographic order of the wave vectors; returns
+// the number of wave vectors
+template <class F> static int each_row(double kc, F f) {
   const double nsqmax = kc * kc + 1e-8;
   const int nm = (int)floor(kc);
   int nk = 0;
@@ -297,10 +298,19 @@ int kspace_rows(double kc, std::vector<int4> &rows) {
       while (m < nm && nx * nx + ny * ny + (m + 1) * (m + 1) <= nsqmax) m++;
       const bool half = nx == 0 && ny == 0;
       if (m < (half ? 1 : 0)) continue;
-      rows.push_back(make_int4(nk, nx, ny, m));
+      f(nk, nx, ny, m);
       nk += half ? m : 2 * m + 1;
     }
   return nk;
+}
+
+int kspace_rows(double kc, std::vector<int4> &rows) {
+  return each_row(kc, [&](int k0, int nx, int ny, int m) { rows.push_back(make_int4(k0, nx, ny, m)); });
+}
+
+int kspace_count(double kc, int &nrow) {
+  nrow = 0;
+  return each_row(kc, [&](int, int, int, int) { nrow++; });
 }
 
 // a neighbour-list build that goes along: nl null without one

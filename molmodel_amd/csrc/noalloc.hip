@@ -17,9 +17,8 @@ namespace mmamd {
 
 // kspace_field without allocation.  Everything the k_ks_* kernels need
 // beyond the caller's inputs and outputs (system parameters, wave vectors
-// and their coefficients, structure factors, SoA positions, per-site
-// results, the energy slot) lives in one file-scope device array; the
-// caller passes device pointers and a stream.  Each device holds its own
+// and their coefficients and rows, structure factors, SoA positions, per-site
+// results) lives in one file-scope device array; the caller passes device pointers and a stream.  Each device holds its own
 // copy of the array until the process ends; every call on a device uses
 // that device's copy, so calls that overlap on one device race.
 constexpr int NA_MAX_SITES = 65536;      // sites per call
@@ -29,7 +28,7 @@ constexpr long NA_KVEC = NA_SP + 128;                     // double4 per wave ve
 constexpr long NA_KSC = NA_KVEC + 4L * NA_MAX_K;          // S_k, C_k
 constexpr int NA_MAX_ROW = 512;                           // rows of wave vectors (326 at kc = 12)
 constexpr long NA_ROW = NA_KSC + 2L * NA_MAX_K;           // int4 per row
-constexpr long NA_R = NA_ROW + 2L * NA_MAX_ROW;             // x[N] y[N] z[N]
+constexpr long NA_R = NA_ROW + 2L * NA_MAX_ROW;           // x[N] y[N] z[N]
 constexpr long NA_KRES = NA_R + 3L * NA_MAX_SITES;        // phi, E per site
 constexpr long NA_TOTAL = NA_KRES + 4L * NA_MAX_SITES + 32;   // 3.9 MB
 static_assert(sizeof(SysParams) <= 128 * sizeof(double), "SysParams slot too small");
@@ -173,8 +172,8 @@ extern "C" int kspace_field_noalloc(double cutoff, int nsite, const cart_t *r, c
     set_last_error("kspace_field_noalloc: bad cutoff, eta, volume or lattice");
     return -1;
   }
-  std::vector<int4> rows;
-  const int nk = kspace_rows(cutoff, rows);
+  int nrow = 0;
+  const int nk = kspace_count(cutoff, nrow);
   if (nk > NA_MAX_K) {
     set_last_error("kspace_field_noalloc: more than " + std::to_string(NA_MAX_K) +
                    " wave vectors (cutoff above 12)");
@@ -193,7 +192,7 @@ extern "C" int kspace_field_noalloc(double cutoff, int nsite, const cart_t *r, c
   P.kmode = 0;
   P.nk = nk;
   P.k0 = 0;
-  P.nkrow = (int)rows.size();
+  P.nkrow = nrow;
   P.nkmax = (int)floor(cutoff);
   memcpy(P.RL, latv, sizeof P.RL);
   P.nsite = nsite;
