@@ -14,13 +14,15 @@
 //   k_ks_sf     one block per row (and per eight |nz| of it), one thread per
 //               site: two sincos per site and row, then a rotation per |nz|;
 //               648 sites, 709 wave vectors: 6.4 us (5.3 with a sincos per site
-//               and wave vector), 3 120 sites: 10.2 (12.2)
+//               and wave vector), 3 120 sites: 10.2 (12.2), 12 288: 27 (34),
+//               41 472: 79 (115), 65 856: 123 (177); its 80 or so blocks leave
+//               most CUs idle there, and are still faster than 709 that each walk the sites
 //   k_ks_field  a block serves 16 sites and its 64 16-lane teams take a row
 //               each; the sites' e^{i n b.r} for every n are formed once, in
 //               LDS, and so are the wave vectors' coefficients; 6.5 us for 648
 //               and for 2 920 sites (8.7 and 8.2 with the coefficients read from
 //               memory in the loop, 38 with 16 waves that walk the wave vectors
-//               with a sincos each, 64 sites a block)
+//               with a sincos each, 64 sites a block), 48 for 41 472 (107)
 // The k-sum energy and virial
 // (W_ab = sum a_k |rho_k|^2 (delta_ab - 2 k_a k_b (1/k^2 + 1/(4 eta^2))))
 // are formed by a block of its own beside the field kernel's.

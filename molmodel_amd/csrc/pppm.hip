@@ -578,8 +578,10 @@ __device__ __forceinline__ void halo_lines(const SysParams &P, const unsigned lo
 
 // z lines, real to half spectrum.  Two neighbouring mesh lines are one complex
 // line (a in the real, b in the imaginary part) whose transform Z separates
-// as a_k = (Z_k + conj Z_-k) / 2, b_k = (Z_k - conj Z_-k) / 2i, so a block of
-// two waves takes 32 lines with one butterfly per thread and stage.
+// as a_k = (Z_k + conj Z_-k) / 2, b_k = (Z_k - conj Z_-k) / 2i, so a block
+// takes 32 lines.  Its four waves share the loads and stores; a stage has
+// 16 nz / R butterflies (96 or 128 at 48 and 64 points), at most one a thread
+// where nz <= 16 R.
 // HALO: a line is the sum of the spreading blocks' halo columns that cover it
 // (halo_lines) instead of the real mesh.  What bounds it is the launch and one
 // trip to memory: 5.7 us at 48^3, 6.7 at 64^3, and the inverse 5.9 and 7
