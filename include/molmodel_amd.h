@@ -320,7 +320,9 @@ int mm_scale_system(mm_engine *e, int sys, double s);
  * the skin test kept it.  rows: the pair set in PairBinary layout (each pair
  * in the row of its pbin.c:6 owner), row_start[n+1] offsets into cols, at
  * most cap columns written; returns the pair count.  The same set as the
- * reference's for the same input; order within a row is the device's. */
+ * reference's for the same input; order within a row is the device's.  After
+ * an update that reported an error the next one rebuilds, and rows reports
+ * the error until then. */
 typedef struct mm_nlist mm_nlist;
 int mm_nlist_create(int n, double cutoff, double width, double boxl, mm_nlist **out);
 int mm_nlist_update(mm_nlist *nl, const double *r);
